@@ -24,7 +24,69 @@
 namespace pega {
 namespace {
 
-// One thread per output word: gathers its 8 nibbles from 4 checkpoint words.
+// One output word: columns n0 (words a0, a1 of its checkpoint row) and n0 + 8
+// (b0, b1), k pair at bit sh of each word (k 0..7 in a0 / b0, 8..15 in a1 / b1).
+__device__ __forceinline__ uint32_t marlin_word(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1,
+                                                int sh) {
+  // byte i: the even-k nibble below the odd-k one, of (n0, k), (n0, k+8), (n0+8, k), (n0+8, k+8)
+  const uint32_t t = ((a0 >> sh) & 0xffu) | (((a1 >> sh) & 0xffu) << 8) |
+                     (((b0 >> sh) & 0xffu) << 16) | (((b1 >> sh) & 0xffu) << 24);
+  uint32_t lo = t & 0x0f0f0f0fu, hi = (t >> 4) & 0x0f0f0f0fu;
+  lo = (lo | (lo >> 4)) & 0x00ff00ffu;
+  hi = (hi | (hi >> 4)) & 0x00ff00ffu;
+  return ((lo | (lo >> 8)) & 0xffffu) | ((hi | (hi >> 8)) << 16);
+}
+
+// The weight repack, a transpose bound by HBM: a workgroup takes 64 checkpoint
+// rows (one column tile) by up to 512 k.  It reads 256 contiguous bytes of each
+// row with 16-byte loads, and from LDS each thread builds whole 16-byte output
+// pieces (the four words of one th), so a k-tile's 512 bytes go out contiguous.
+// The row pitch of 66 words puts the eight rows a half-wave reads on distinct
+// bank pairs.  48 x 2048 x 7168: 426 us with one gathering thread per output
+// word (1.65 TB/s), 135 us (5.2 TB/s) here.
+constexpr int kRepackK = 512;                      // k per workgroup
+constexpr int kRepackPitch = kRepackK / 8 + 2;     // words per LDS row
+__global__ __launch_bounds__(256) void reorder_weight_tile_kernel(
+    const uint32_t* __restrict__ ckpt, uint32_t* __restrict__ marlin, int size_k, int size_n) {
+  __shared__ uint32_t rows[64 * kRepackPitch];
+  const int nt = blockIdx.y, n_tiles = size_n >> 6;
+  const int k0 = blockIdx.x * kRepackK;
+  const int kn = min(kRepackK, size_k - k0);  // a multiple of 32
+  const int k_words = size_k >> 3;
+  const long long per_expert = static_cast<long long>(size_n) * k_words;
+  const uint32_t* src = ckpt + blockIdx.z * per_expert +
+                        static_cast<long long>(nt) * 64 * k_words + (k0 >> 3);
+  const int quads = kn >> 5;  // 16-byte pieces of a row
+  for (int i = threadIdx.x; i < 64 * (kRepackK / 32); i += 256) {
+    const int r = i / (kRepackK / 32), q = i % (kRepackK / 32);
+    if (q >= quads) continue;
+    const uint4 v =
+        *reinterpret_cast<const uint4*>(src + static_cast<long long>(r) * k_words + 4 * q);
+    uint32_t* d = rows + r * kRepackPitch + 4 * q;
+    d[0] = v.x;
+    d[1] = v.y;
+    d[2] = v.z;
+    d[3] = v.w;
+  }
+  __syncthreads();
+  uint4* out = reinterpret_cast<uint4*>(marlin + blockIdx.z * per_expert) +
+               (static_cast<long long>(k0 >> 4) * n_tiles + nt) * 32;
+  for (int i = threadIdx.x; i < kn * 2; i += 256) {  // 32 pieces per k-tile
+    const int kt = i >> 5, th = i & 31;
+    const int sh = 8 * (th & 3);
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t* a = rows + (16 * j + (th >> 2)) * kRepackPitch + 2 * kt;
+      const uint32_t* b = a + 8 * kRepackPitch;
+      w[j] = marlin_word(a[0], a[1], b[0], b[1], sh);
+    }
+    out[static_cast<long long>(kt) * n_tiles * 32 + th] = make_uint4(w[0], w[1], w[2], w[3]);
+  }
+}
+
+// One thread per output word, for buffers that are not 16-byte aligned: gathers
+// its 8 nibbles from 4 checkpoint words.
 __global__ void reorder_weight_kernel(const uint32_t* __restrict__ ckpt,
                                       uint32_t* __restrict__ marlin, int size_k, int size_n,
                                       long long total_words) {
@@ -40,22 +102,38 @@ __global__ void reorder_weight_kernel(const uint32_t* __restrict__ ckpt,
   const int kt = static_cast<int>(tile / n_tiles);
   const int th = word >> 2, w = word & 3;
   const int n0 = nt * 64 + w * 16 + (th >> 2);
-  const int kb = kt * 16 + 2 * (th & 3);  // even, so kb and kb+1 share a word
   const int k_words = size_k / 8;
-  const uint32_t* src = ckpt + e * per_expert;
-  const uint32_t a0 = src[static_cast<long long>(n0) * k_words + (kb >> 3)];
-  const uint32_t a1 = src[static_cast<long long>(n0) * k_words + ((kb + 8) >> 3)];
-  const uint32_t b0 = src[static_cast<long long>(n0 + 8) * k_words + (kb >> 3)];
-  const uint32_t b1 = src[static_cast<long long>(n0 + 8) * k_words + ((kb + 8) >> 3)];
-  const int sh = (kb & 7) * 4;
-  const uint32_t nk0 = (a0 >> sh) & 0xf, nk1 = (a0 >> (sh + 4)) & 0xf;
-  const uint32_t nk8 = (a1 >> sh) & 0xf, nk9 = (a1 >> (sh + 4)) & 0xf;
-  const uint32_t mk0 = (b0 >> sh) & 0xf, mk1 = (b0 >> (sh + 4)) & 0xf;
-  const uint32_t mk8 = (b1 >> sh) & 0xf, mk9 = (b1 >> (sh + 4)) & 0xf;
-  marlin[idx] = nk0 | (nk8 << 4) | (mk0 << 8) | (mk8 << 12) | (nk1 << 16) | (nk9 << 20) |
-                (mk1 << 24) | (mk9 << 28);
+  const uint32_t* a = ckpt + e * per_expert + static_cast<long long>(n0) * k_words + 2 * kt;
+  const uint32_t* b = a + 8LL * k_words;
+  marlin[idx] = marlin_word(a[0], a[1], b[0], b[1], 8 * (th & 3));
 }
 
+// The scale repack of whole 64-column tiles, a transpose of 2-byte elements
+// through LDS: 64 checkpoint rows by up to 64 groups, read along the groups and
+// written along the permuted columns, 128 contiguous bytes a wave either way
+// (one element per thread from global memory to global memory: 81 us for
+// 48 x 2048 x 224, 1.1 TB/s; 22 us here).
+__global__ __launch_bounds__(256) void reorder_scale_tile_kernel(
+    const uint16_t* __restrict__ ckpt, uint16_t* __restrict__ marlin, int size_n, int scale_k) {
+  __shared__ uint16_t rows[64][66];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int n0 = blockIdx.y * 64, g0 = blockIdx.x * 64;
+  const long long base = static_cast<long long>(blockIdx.z) * size_n * scale_k;
+  const int gn = min(64, scale_k - g0);
+  if (lane < gn) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int r = wave * 16 + i;
+      rows[r][lane] = ckpt[base + static_cast<long long>(n0 + r) * scale_k + g0 + lane];
+    }
+  }
+  __syncthreads();
+  const int p = (lane >> 3) + 8 * (lane & 7);  // the column stored at position `lane`
+  for (int g = wave; g < gn; g += 4)
+    marlin[base + static_cast<long long>(g0 + g) * size_n + n0 + lane] = rows[p][g];
+}
+
+// One thread per element, for widths that are not whole 64-column tiles.
 __global__ void reorder_scale_kernel(const uint16_t* __restrict__ ckpt,
                                      uint16_t* __restrict__ marlin, int size_n, int scale_k,
                                      long long total) {
@@ -102,6 +180,8 @@ bool common_shape_ok(int in_dim, int out_dim, int local_experts, int group_size)
          in_dim % 16 == 0 && out_dim % 64 == 0 && in_dim % group_size == 0;
 }
 
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
 unsigned grid_for(long long n, int threads) {
   long long g = (n + threads - 1) / threads;
   return static_cast<unsigned>(g < 1 ? 1 : (g > 0x7fffffffLL ? 0x7fffffffLL : g));
@@ -115,6 +195,14 @@ int reorder_weight(const uint8_t* ckpt, uint8_t* marlin, int in_dim, int out_dim
   if (!common_shape_ok(in_dim, out_dim, local_experts, group_size))
     return fail(kInvalidValue, "reorder_weight: bad shape in=%d out=%d E=%d group=%d", in_dim,
                 out_dim, local_experts, group_size);
+  // the tile kernel's grid: k chunks, column tiles (at most 65535), experts (the same)
+  if (aligned16(ckpt) && aligned16(marlin) && out_dim / 64 <= 65535 && local_experts <= 65535) {
+    const dim3 grid(ceil_div(in_dim, kRepackK), out_dim / 64, local_experts);
+    hipLaunchKernelGGL(reorder_weight_tile_kernel, grid, dim3(256), 0, stream,
+                       reinterpret_cast<const uint32_t*>(ckpt),
+                       reinterpret_cast<uint32_t*>(marlin), in_dim, out_dim);
+    return launch_status("reorder_weight");
+  }
   const long long total = static_cast<long long>(local_experts) * out_dim * (in_dim / 8);
   hipLaunchKernelGGL(reorder_weight_kernel, dim3(grid_for(total, 256)), dim3(256), 0, stream,
                      reinterpret_cast<const uint32_t*>(ckpt), reinterpret_cast<uint32_t*>(marlin),
@@ -133,6 +221,12 @@ int reorder_scale(const uint16_t* ckpt, uint16_t* marlin, int in_dim, int out_di
   if (per_expert % 64 != 0)
     return fail(kInvalidValue, "reorder_scale: out*groups (%lld) not a multiple of 64",
                 per_expert);
+  if (out_dim % 64 == 0 && out_dim / 64 <= 65535 && local_experts <= 65535) {
+    const dim3 grid(ceil_div(scale_k, 64), out_dim / 64, local_experts);
+    hipLaunchKernelGGL(reorder_scale_tile_kernel, grid, dim3(256), 0, stream, ckpt, marlin,
+                       out_dim, scale_k);
+    return launch_status("reorder_scale");
+  }
   const long long total = per_expert * local_experts;
   hipLaunchKernelGGL(reorder_scale_kernel, dim3(grid_for(total, 256)), dim3(256), 0, stream,
                      ckpt, marlin, out_dim, scale_k, total);
@@ -157,6 +251,15 @@ int fuse_w13(const uint8_t* gate_w, const uint8_t* up_w, uint8_t* w13_w, const u
   int st = launch_status("fuse_w13 weights");
   if (st != kSuccess) return st;
   const long long srows = static_cast<long long>(local_experts) * (in_dim / group_size);
+  // 16 bytes a thread where the buffers allow it (inter is a multiple of 64): 48 x 224 rows of
+  // 2 x 2048 scales 67 -> 35 us
+  if (aligned16(gate_s) && aligned16(up_s) && aligned16(w13_s)) {
+    hipLaunchKernelGGL(concat_rows_kernel, dim3(grid_for(srows * (inter / 8), 256)), dim3(256), 0,
+                       stream, reinterpret_cast<const uint4*>(gate_s),
+                       reinterpret_cast<const uint4*>(up_s), reinterpret_cast<uint4*>(w13_s),
+                       srows, inter / 8);
+    return launch_status("fuse_w13 scales");
+  }
   hipLaunchKernelGGL(concat_rows_u16_kernel, dim3(grid_for(srows * inter, 256)), dim3(256), 0,
                      stream, gate_s, up_s, w13_s, srows, inter);
   return launch_status("fuse_w13 scales");

@@ -90,3 +90,65 @@ def test_checkpoint_loader_gives_the_packed_layout(tmp_path):
         assert torch.equal(got.weight_packed_uint4b8, ref.weight_packed_uint4b8)
         assert torch.equal(got.weight_scale_permuted.view(torch.int16),
                            ref.weight_scale_permuted.view(torch.int16))
+
+
+@pytest.mark.parametrize("E,K,N,shift", [(1, 32, 64, 0), (2, 480, 128, 0), (3, 544, 192, 0),
+                                         (2, 1024, 64, 0), (2, 2080, 128, 0), (2, 544, 128, 4)])
+def test_repack_tile_edges_and_unaligned(oracle, E, K, N, shift):
+    """Ragged last k chunks of the tile kernels (512 k of weights, 64 groups of scales), one
+    group, and buffers 4 bytes off a 16-byte boundary (the gathering kernel)."""
+    from pegainfer_amd import _lib
+    g = np.random.default_rng(K + N)
+    packed = g.integers(0, 256, size=E * N * K // 2, dtype=np.uint8)
+    scales = g.integers(0, 2 ** 16, size=E * N * (K // 32)).astype(np.uint16)
+    src = torch.zeros(packed.size + 16, dtype=torch.uint8, device="cuda")
+    out = torch.full_like(src, 0xAB)
+    src[shift:shift + packed.size].copy_(dev(packed))
+    s_src = torch.zeros(scales.size + 8, dtype=torch.int16, device="cuda")
+    s_out = torch.full_like(s_src, 0x2BAB)
+    s_src[shift // 2:shift // 2 + scales.size].copy_(dev(scales.view(np.int16)))
+    stream = torch.cuda.current_stream().cuda_stream
+    _lib.call("pega_marlin_int4_reorder_weight", src.data_ptr() + shift, out.data_ptr() + shift, K,
+              N, E, 32, stream)
+    _lib.call("pega_marlin_int4_reorder_scale", s_src.data_ptr() + shift, s_out.data_ptr() + shift,
+              K, N, E, 32, stream)
+    got, s_got = host(out), host(s_out).view(np.uint16)
+    assert np.array_equal(got[shift:shift + packed.size].view(np.uint32),
+                          oracle.marlin_reorder_weight(packed.view(np.uint32), K, N, E))
+    assert (got[:shift] == 0xAB).all() and (got[shift + packed.size:] == 0xAB).all()
+    lo = shift // 2
+    assert np.array_equal(s_got[lo:lo + scales.size], oracle.marlin_reorder_scale(scales, K, N, E))
+    assert (s_got[:lo] == 0x2BAB).all() and (s_got[lo + scales.size:] == 0x2BAB).all()
+
+
+def test_scale_repack_width_not_a_column_tile(oracle):
+    """out_dim 32 (two groups share a 64-element chunk): the element kernel."""
+    from pegainfer_amd import _lib
+    g = np.random.default_rng(3)
+    E, K, N = 2, 128, 32
+    scales = g.integers(0, 2 ** 16, size=E * N * (K // 32)).astype(np.uint16)
+    out = torch.zeros(scales.size, dtype=torch.int16, device="cuda")
+    src = dev(scales.view(np.int16))
+    _lib.call("pega_marlin_int4_reorder_scale", src.data_ptr(), out.data_ptr(), K, N, E, 32,
+              torch.cuda.current_stream().cuda_stream)
+    assert np.array_equal(host(out).view(np.uint16), oracle.marlin_reorder_scale(scales, K, N, E))
+
+
+@pytest.mark.parametrize("shift", [0, 2])
+def test_fuse_scales_aligned_and_not(shift):
+    """The W13 scale concatenation with 16-byte aligned buffers and 2 bytes off."""
+    from pegainfer_amd import _lib
+    g = np.random.default_rng(5)
+    E, K, I = 2, 96, 64
+    rows = E * (K // 32)
+    w = torch.zeros(E * I * K // 2, dtype=torch.uint8, device="cuda")
+    w13 = torch.zeros(2 * w.numel(), dtype=torch.uint8, device="cuda")
+    a, b = (g.integers(0, 2 ** 15, size=(rows, I)).astype(np.int16) for _ in range(2))
+    bufs = [torch.zeros(rows * I * k + 8, dtype=torch.int16, device="cuda") for k in (1, 1, 2)]
+    for buf, v in zip(bufs, (a, b)):
+        buf[shift // 2:shift // 2 + rows * I].copy_(dev(v.reshape(-1)))
+    _lib.call("pega_marlin_int4_fuse_w13", w.data_ptr(), w.data_ptr(), w13.data_ptr(),
+              *(t.data_ptr() + shift for t in bufs), K, I, E, 32,
+              torch.cuda.current_stream().cuda_stream)
+    got = host(bufs[2])[shift // 2:shift // 2 + 2 * rows * I].reshape(rows, 2 * I)
+    assert np.array_equal(got, np.concatenate([a, b], axis=1))
