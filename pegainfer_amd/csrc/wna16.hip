@@ -11,11 +11,14 @@
 //     c = bf16(acc);  if mul_topk_weights: c = bf16(f(c) * f(bf16(topk_w[sid])))
 //     C[sid][n] = c                                                (:1772-1900)
 //
-// Dequantisation is exact: the nibble v is placed in an fp16 whose value is
-// 1024 + v (or 64 + v), v_fma_mix_f32 forms (1024 + v)*s - 1032*s = (v-8)*s
-// with no rounding (every term fits fp32), and v_cvt_pk_bf16_f32 rounds that
-// product to bf16 with round-to-nearest-even -- the same value as the
-// reference's bf16 multiply q*s.
+// Dequantisation is exact: the nibble v, masked out of its word, is the fp16
+// denormal v 2^-24 (or v 2^-20, four bits further up), v_fma_mix_f32 forms
+// v 2^-24 * 2^24 s - 8 s = (v - 8) s with no rounding (both terms and the result fit
+// fp32 for scales below 2^104), and v_cvt_pk_bf16_f32 rounds that product to bf16
+// with round-to-nearest-even -- the same value as the reference's bf16 multiply
+// q*s.  The mask is a two-operand v_and_b32; biasing the nibble to 1024 + v takes a
+// three-operand v_and_or_b32, which issues at half the rate once two waves share a
+// SIMD (1.0 against 1.8 ns an instruction).
 //
 // Fragment map (per 64-column Marlin tile nt, per quant group g = k-tiles
 // 2g, 2g+1): lane l -> column c = l%32, k-half h = l/32.  The lane owns
@@ -28,6 +31,7 @@
 // row: index 8*(c%8) + 2*(c/8) (+1).
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "common.h"
 #include "pega_moe.h"
@@ -38,34 +42,18 @@ namespace {
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16_t;
 
-// (x & mask) | bits in plain C, never as a vector inline-asm statement: the
-// compiler's hazard tracking cannot see VGPRs written inside asm, and a VALU
-// write landing in the destination (or a source) of an MFMA still in flight
-// is exactly the hazard it must see to insert wait states.  With `mask` in an
-// SGPR this is one v_and_or_b32 (a VOP3 on gfx9 takes no literal operand, so
-// with literal masks the compiler would emit v_and + v_or instead).
-__device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t mask, uint32_t bits) {
-  return (x & mask) | bits;
-}
-
-// The dequant constants in registers the compiler treats as opaque: the
-// masks in SGPRs (s_mov_b32 in an asm statement that writes only SGPRs, which
-// no MFMA reads) and the fp16 bias patterns in VGPRs (a DPP move of a
-// wave-uniform value, which the compiler does not fold).  v_and_or_b32 then
-// takes one SGPR and one VGPR operand, within gfx9's one-scalar-operand limit.
+// The nibble masks in SGPRs the compiler treats as opaque (s_mov_b32 in an asm
+// statement that writes only SGPRs, which no MFMA reads; vector instructions are
+// never written as asm here, since the compiler's hazard tracking cannot see VGPRs
+// written inside one): v_and_b32 then is a 4-byte VOP2 with one scalar operand.
 struct DqConst {
   uint32_t m_lo, m_hi;  // 0x000F000F, 0x00F000F0
-  uint32_t k1024, k64;  // fp16 1024 | 1024 and 64 | 64
 };
 __device__ __forceinline__ DqConst dq_consts() {
   uint32_t lo, hi;
   asm("s_mov_b32 %0, 0x000f000f" : "=s"(lo));
   asm("s_mov_b32 %0, 0x00f000f0" : "=s"(hi));
-  const uint32_t k1024 = static_cast<uint32_t>(
-      __builtin_amdgcn_mov_dpp(static_cast<int>(0x64006400u), 0xB1, 0xF, 0xF, true));
-  const uint32_t k64 = static_cast<uint32_t>(
-      __builtin_amdgcn_mov_dpp(static_cast<int>(0x54005400u), 0xB1, 0xF, 0xF, true));
-  return DqConst{lo, hi, k1024, k64};
+  return DqConst{lo, hi};
 }
 
 __device__ __forceinline__ float h_lo(uint32_t p) {
@@ -76,11 +64,11 @@ __device__ __forceinline__ float h_hi(uint32_t p) {
 }
 
 struct ColScale {
-  float s, c1024, c72;  // s, -1032*s, -72*s
+  float s24, s20, c8;  // 2^24 s, 2^20 s, -8 s
 };
 
 __device__ __forceinline__ ColScale col_scale(float s) {
-  return ColScale{s, -1032.0f * s, -72.0f * s};
+  return ColScale{16777216.0f * s, 1048576.0f * s, -8.0f * s};
 }
 
 // One Marlin word -> bf16 pairs: (n0: k0k1, k8k9), (n1: k0k1, k8k9).
@@ -90,16 +78,16 @@ struct WordPairs {
 
 __device__ __forceinline__ WordPairs dequant_word(uint32_t x, const ColScale& a,
                                                   const ColScale& b, const DqConst& k) {
-  const uint32_t p0 = and_or(x, k.m_lo, k.k1024);
-  const uint32_t p1 = and_or(x, k.m_hi, k.k64);
+  const uint32_t p0 = x & k.m_lo;
+  const uint32_t p1 = x & k.m_hi;
   const uint32_t y = x >> 8;
-  const uint32_t p2 = and_or(y, k.m_lo, k.k1024);
-  const uint32_t p3 = and_or(y, k.m_hi, k.k64);
+  const uint32_t p2 = y & k.m_lo;
+  const uint32_t p3 = y & k.m_hi;
   WordPairs r;
-  r.n0_lo = pack_bf16x2(__builtin_fmaf(h_lo(p0), a.s, a.c1024), __builtin_fmaf(h_hi(p0), a.s, a.c1024));
-  r.n0_hi = pack_bf16x2(__builtin_fmaf(h_lo(p1), a.s, a.c72), __builtin_fmaf(h_hi(p1), a.s, a.c72));
-  r.n1_lo = pack_bf16x2(__builtin_fmaf(h_lo(p2), b.s, b.c1024), __builtin_fmaf(h_hi(p2), b.s, b.c1024));
-  r.n1_hi = pack_bf16x2(__builtin_fmaf(h_lo(p3), b.s, b.c72), __builtin_fmaf(h_hi(p3), b.s, b.c72));
+  r.n0_lo = pack_bf16x2(__builtin_fmaf(h_lo(p0), a.s24, a.c8), __builtin_fmaf(h_hi(p0), a.s24, a.c8));
+  r.n0_hi = pack_bf16x2(__builtin_fmaf(h_lo(p1), a.s20, a.c8), __builtin_fmaf(h_hi(p1), a.s20, a.c8));
+  r.n1_lo = pack_bf16x2(__builtin_fmaf(h_lo(p2), b.s24, b.c8), __builtin_fmaf(h_hi(p2), b.s24, b.c8));
+  r.n1_hi = pack_bf16x2(__builtin_fmaf(h_lo(p3), b.s20, b.c8), __builtin_fmaf(h_hi(p3), b.s20, b.c8));
   return r;
 }
 
@@ -681,115 +669,158 @@ void launch_decode_pair(const GemmArgs& args, int max_m_blocks, hipStream_t stre
 // tile, R = 128, or 64 where experts hold few rows), 4 waves each own one
 // 64-column tile.
 //
-// Per 64-wide K chunk (two quant groups):
-//   * activations: 128 rows x 64 k (16 KB) staged in double-buffered LDS
-//     (rows padded to 72 bf16 against bank conflicts), loaded by all 256
-//     threads with 16-byte buffer loads two chunks ahead of use;
-//   * weights: one 16-byte load per lane per group (the decode kernel's
-//     pattern), transposed through a per-wave LDS slot, dequantised in
-//     registers; two chunks in flight;
-//   * 16 MFMA 32x32x16 per group per wave (4 row blocks x n0/n1 x 2 k-halves).
-// The loop is unrolled by two with named ping-pong buffers, so no register
-// copies are needed to rotate the prefetch; activation loads are issued
-// before weight loads so that waiting for the former leaves the latter in
-// flight (vector-memory counters retire in order).
+// What bounds it: the vector unit (79 instructions per 32-k group and wave, 64 of
+// them the exact dequant) beside the matrix pipe (4 MFMAs per group and 32-row
+// block, each of which also holds the vector unit's issue for about half its 32
+// cycles), so the loop's work is to keep the two side by side and everything else
+// out of their way:
+//   * activations, weights and scales go from memory straight to LDS (a ring of
+//     three or four 64-k stages, filled two or three chunks ahead): no staging
+//     registers, no LDS writes, and loads that no instruction waits for but one
+//     counted wait per chunk;
+//   * a wave's fragments are the words of its own weights, read in fragment order;
+//     the next group is dequantised between this group's MFMAs, a word per row block
+//     at R = 128;
+//   * one barrier per chunk: the activations are shared, the weights are not.
+// Against the register-staged form with the same tiles: Kimi's routed W13 + SwiGLU
+// and W2 under Zipf routing at 4096 tokens 479 -> 467 and 257 -> 254 us, at 1000
+// tokens 185 -> 178 and 101 -> 94 us (with 64-row tiles), DeepSeek-V2-Lite's at 2500
+// tokens 201 -> 196 and 111 -> 110 us.
 // ---------------------------------------------------------------------------
-constexpr int kPfChunk = 64;                 // k per LDS stage (2 quant groups)
-constexpr int kPfLdsStride = kPfChunk + 8;   // bf16 per LDS row (padding vs bank conflicts)
-// bf16 elements of the LDS area of an R-row tile: the two activation stages,
-// or the epilogue's 64-row staging ([64][264] bf16, or [2][64][65] words)
-constexpr int pf_lds_elems(int R) {
-  return 2 * R * kPfLdsStride > 64 * 264 ? 2 * R * kPfLdsStride : 64 * 264;
+constexpr int kPfChunk = 64;  // k per stage (2 quant groups)
+// Bytes of one stage beside the activations: per wave two groups' weight words
+// (1 KB each, as they lie in memory) and column scales (128 bytes each).
+constexpr int kPfWStage = 4 * 2048, kPfSStage = 4 * 256;
+constexpr int pf_stage_bytes(int RB) { return RB * 32 * kPfChunk * 2 + kPfWStage + kPfSStage; }
+// LDS of an R-row tile's ring: three workgroups of 64 rows or two of 128 rows fit a
+// CU's 160 KB with their other arrays.  The epilogue's staging (64 x 264 bf16, or
+// 2 x 64 x 65 words) and the tile scan lie in it too.
+constexpr int pf_ring_bytes(int R) { return R == 64 ? 53248 : 79872; }
+// Stages of the ring for a tile of RB routed row blocks: as many as fit, at most 4.
+constexpr int pf_stages(int RB, int R) {
+  return pf_ring_bytes(R) / pf_stage_bytes(RB) < 4 ? pf_ring_bytes(R) / pf_stage_bytes(RB) : 4;
 }
 
-struct PfB {
-  u32x4_t w[2];   // per group: the 4 words (th, w = 0..3) of this lane's k-tile
-  uint32_t s[2];  // per group: this lane's two column scales
+// Global memory straight to LDS: lane l's 16 (or 4) bytes at voff + soff go to
+// lds + 16 l (4 l).  In asm so that the compiler, which cannot tell the ring's
+// stages apart, does not drain every load in flight at each LDS read; the kernel
+// counts them itself (vm_wait) and no register is written.
+__device__ __forceinline__ void dma_b128(u32x4_t rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+}
+__device__ __forceinline__ void dma_b32(u32x4_t rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+               :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void vm_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
+}
+// Every wave's LDS reads have returned and its counted loads have landed.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+__device__ __forceinline__ u32x4_t rsrc_words(const void* base, uint32_t bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(base);
+  u32x4_t r = {static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a))),
+               static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a >> 32))) & 0xffffu,
+               bytes, 0x00020000u};
+  return r;
+}
+
+// One group's four B fragments (x1, x2, y1, y2), filled word by word: word jj holds
+// k = 2jj + {0, 1} in its "lo" pair and 2jj + {8, 9} in its "hi" pair.
+struct PfFrags {
+  uint32_t v[4][4];
+  __device__ __forceinline__ void put(int jj, const WordPairs& q) {
+    v[0][jj] = q.n0_lo;
+    v[1][jj] = q.n0_hi;
+    v[2][jj] = q.n1_lo;
+    v[3][jj] = q.n1_hi;
+  }
+  __device__ __forceinline__ bf16x8_t get(int i) const {
+    return as_bf16x8(v[i][0], v[i][1], v[i][2], v[i][3]);
+  }
 };
 
-// Main loop and epilogue of one wave for a tile with RB routed 32-row blocks
-// (RB = 0: a wave past the last column tile, which only helps stage the
-// activations).  A compile-time RB keeps every loop body branch-free and
+// Main loop and epilogue of one wave for a tile with RB routed 32-row blocks.
+// IDLE: a wave past the last column tile, which only stages its share of the
+// activations.  A compile-time RB keeps every loop body branch-free and
 // allocates only the accumulators in use.
-template <int RB, int R>
-__device__ __forceinline__ void prefill_tile(const GemmArgs& p, uint16_t* s_a, uint32_t* s_w_wave,
-                                             const int* s_sid, const float* s_tw, int expert,
-                                             int nt, int tx) {
-  constexpr int kStage = R * kPfLdsStride;  // bf16 per activation stage
-  constexpr int kPieces = R / 32;           // 16-byte activation pieces per thread per chunk
+template <int RB, int R, bool IDLE>
+__device__ __forceinline__ void prefill_tile(const GemmArgs& p, uint8_t* smem, const int* s_sid,
+                                             const float* s_tw, int expert, int nt, int tx) {
+  constexpr int NS = pf_stages(RB, R);
+  constexpr int kStage = pf_stage_bytes(RB);
+  constexpr int kAStage = RB * 32 * kPfChunk * 2;
+  constexpr int P = RB + (IDLE ? 0 : 3);  // loads per chunk
+  static_assert(NS >= 3 && NS * kStage <= pf_ring_bytes(R), "the ring fits");
+  static_assert(pf_ring_bytes(R) >= 64 * 264 * 2 && pf_ring_bytes(R) >= 2 * 64 * 65 * 4, "epilogue");
   const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 31, h = lane >> 5;
   const int K = p.size_k, N = p.size_n;
   const int n_tiles = N >> 6;
-  const int groups = K >> 5;
   const int chunks = K / kPfChunk;
   const int valid_limit = p.size_m * p.top_k;
-  const int ntc = RB > 0 ? nt : 0;
+  const int ntc = IDLE ? 0 : nt;
   const uint32_t expert_bytes = static_cast<uint32_t>(N) * static_cast<uint32_t>(K) / 2u;
-  const __amdgpu_buffer_rsrc_t wr = make_rsrc(
+  const u32x4_t wr = rsrc_words(
       p.qweight + static_cast<long long>(expert) * (expert_bytes / 4u), expert_bytes);
   const uint32_t tile_row_bytes = static_cast<uint32_t>(n_tiles) * 512u;
   const uint32_t w_voff = static_cast<uint32_t>(h) * tile_row_bytes +
                           static_cast<uint32_t>(ntc) * 512u + static_cast<uint32_t>(c) * 16u;
   const uint32_t w_step = 2u * tile_row_bytes;  // bytes per quant group
-  const uint32_t scale_bytes = static_cast<uint32_t>(groups) * static_cast<uint32_t>(N) * 2u;
-  const __amdgpu_buffer_rsrc_t sr = make_rsrc(
-      p.scales + static_cast<long long>(expert) * groups * N, scale_bytes);
-  const uint32_t s_voff = (static_cast<uint32_t>(ntc) * 64u + 8u * (c & 7) + 2u * (c >> 3)) * 2u;
   const uint32_t s_step = static_cast<uint32_t>(N) * 2u;
-  const __amdgpu_buffer_rsrc_t ar =
-      make_rsrc(p.input, static_cast<uint32_t>(p.size_m) * static_cast<uint32_t>(K) * 2u);
+  const u32x4_t sr = rsrc_words(p.scales + static_cast<long long>(expert) * (K >> 5) * N,
+                                static_cast<uint32_t>(K >> 5) * s_step);
+  // lanes 0..31 the first group's 32 dwords of column scales, 32..63 the second's
+  const uint32_t s_voff = static_cast<uint32_t>(h) * s_step + static_cast<uint32_t>(ntc) * 128u +
+                          4u * static_cast<uint32_t>(c);
+  const u32x4_t ar =
+      rsrc_words(p.input, static_cast<uint32_t>(p.size_m) * static_cast<uint32_t>(K) * 2u);
 
-  uint32_t* slot_w = s_w_wave + h * 160 + c;          // this lane's transpose write column
-  const uint32_t* slot_r = s_w_wave + h * 160 + 4 * c;  // this lane's 16-byte read
-
-  auto load_b = [&](PfB& b, int chunk) {
-    if constexpr (RB > 0) {
-      const uint32_t ch = static_cast<uint32_t>(min(chunk, chunks - 1));  // past the end: unused
+  // Activation staging: a row is 8 pieces of 16 bytes per chunk, piece q of row r at
+  // position q ^ (r % 8), so that the MFMA fragments' reads (32 rows, one piece) spread
+  // over the banks.  Load i of wave w brings rows 32 i + 8 w .. + 7, one row per 8 lanes;
+  // rows not routed here are out of range (zeros, or stale bytes: their products are
+  // never stored).
+  uint32_t a_voff[RB];
 #pragma unroll
-      for (int gg = 0; gg < 2; ++gg) {
-        const uint32_t g = 2u * ch + static_cast<uint32_t>(gg);
-        b.w[gg] = buf_load_b128(wr, w_voff, g * w_step);
-        b.s[gg] = buf_load_b32(sr, s_voff, g * s_step);
-      }
-    }
-  };
-
-  // Activation staging: R rows x 64 k = 8 R 16-byte pieces, R / 32 per thread;
-  // rows not routed here read zeros (out-of-range buffer offset).  A thread's
-  // piece i lies in 32-row block i, so a tile with RB < R / 32 routed blocks
-  // stages only its first RB blocks (the MFMAs read no other row); a wave past
-  // the last column tile (RB = 0) stages all of them, which covers whatever
-  // the workgroup's other waves need.
-  constexpr int kStaged = RB > 0 && RB < kPieces ? RB : kPieces;
-  uint32_t a_voff[kStaged];
-#pragma unroll
-  for (int i = 0; i < kStaged; ++i) {
-    const int piece = tid + 256 * i;
-    const int r = piece >> 3, q = piece & 7;
+  for (int i = 0; i < RB; ++i) {
+    const int r = 32 * i + 8 * wv + (lane >> 3);
     const int sid = s_sid[r];
     a_voff[i] = static_cast<unsigned>(sid) < static_cast<unsigned>(valid_limit)
-                    ? (static_cast<uint32_t>(sid / p.top_k) * static_cast<uint32_t>(K) + 8u * q) * 2u
+                    ? (static_cast<uint32_t>(sid / p.top_k) * static_cast<uint32_t>(K)) * 2u +
+                          16u * ((lane & 7) ^ (lane >> 3))
                     : kOutOfRange;
   }
-  // A chunk index past the end reads zeros (every lane out of range).
-  auto load_a = [&](u32x4_t (&st)[kStaged], int chunk) {
-    const uint32_t past = chunk < chunks ? 0u : kOutOfRange;
-    const uint32_t ch = static_cast<uint32_t>(min(chunk, chunks - 1));
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+      (__attribute__((address_space(3))) uint8_t*)smem));
+  auto stage_in = [&](int ch, int st) {
+    const uint32_t base = lds0 + static_cast<uint32_t>(st);
+    const uint32_t uch = static_cast<uint32_t>(ch);
+    if constexpr (!IDLE) {
 #pragma unroll
-    for (int i = 0; i < kStaged; ++i)
-      st[i] = buf_load_b128(ar, a_voff[i] | past, ch * (kPfChunk * 2u));
-  };
-  auto store_a = [&](const u32x4_t (&st)[kStaged], int buf) {
-#pragma unroll
-    for (int i = 0; i < kStaged; ++i) {
-      const int piece = tid + 256 * i;
-      const int r = piece >> 3, q = piece & 7;
-      *reinterpret_cast<u32x4_t*>(&s_a[buf * kStage + r * kPfLdsStride + 8 * q]) = st[i];
+      for (int gg = 0; gg < 2; ++gg)
+        dma_b128(wr, base + kAStage + 2048u * wv + 1024u * gg, w_voff, (2u * uch + gg) * w_step);
+      dma_b32(sr, base + kAStage + kPfWStage + 256u * wv, s_voff, 2u * uch * s_step);
     }
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+      dma_b128(ar, base + 4096u * i + 1024u * wv, a_voff[i], uch * (kPfChunk * 2u));
   };
 
-  constexpr int NACC = RB > 0 ? RB : 1;
+  // this lane's LDS addresses within a stage
+  const uint8_t* w_rd = smem + kAStage + 2048 * wv + 512 * h + 64 * (c & 7) + 4 * (c >> 3);
+  const uint8_t* s_rd = smem + kAStage + kPfWStage + 256 * wv + 16 * (c & 7) + 4 * (c >> 3);
+  const uint8_t* a_rd[4];  // pieces 4 gg + 2 h + e of row c
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    a_rd[i] = smem + 128 * c + 16 * ((4 * (i >> 1) + 2 * h + (i & 1)) ^ (c & 7));
+
+  constexpr int NACC = RB;
   floatx16_t accx[NACC], accy[NACC];
 #pragma unroll
   for (int rb = 0; rb < NACC; ++rb) {
@@ -798,63 +829,89 @@ __device__ __forceinline__ void prefill_tile(const GemmArgs& p, uint16_t* s_a, u
   }
   const DqConst dq = dq_consts();
 
-  auto compute = [&](const PfB& b, int buf) {
-    if constexpr (RB > 0) {
+  // words jj = 0..3 of this lane's column pair in group gg of a stage
+  auto read_w = [&](uint32_t (&w)[4], int st, int gg) {
 #pragma unroll
-      for (int gg = 0; gg < 2; ++gg) {
-        // transpose the tile words into fragment order through this wave's slot
-        slot_w[0] = b.w[gg][0];
-        slot_w[32] = b.w[gg][1];
-        slot_w[64] = b.w[gg][2];
-        slot_w[96] = b.w[gg][3];
-        const u32x4_t fw = *reinterpret_cast<const u32x4_t*>(slot_r);
-        const uint32_t w4[4] = {fw[0], fw[1], fw[2], fw[3]};
-        const BFrags f = make_b(w4, b.s[gg], dq);
+    for (int jj = 0; jj < 4; ++jj)
+      w[jj] = *reinterpret_cast<const uint32_t*>(w_rd + st + 1024 * gg + 16 * jj);
+  };
+  auto read_a = [&](bf16x8_t (&A)[2], int st, int gg, int rb) {
+    A[0] = *reinterpret_cast<const bf16x8_t*>(a_rd[2 * gg] + st + 4096 * rb);
+    A[1] = *reinterpret_cast<const bf16x8_t*>(a_rd[2 * gg + 1] + st + 4096 * rb);
+  };
+  // The products of group gg with its fragments f, and the dequantisation of the next
+  // group (words w, scale pair sp) into n, one row block's four MFMAs and a share of the
+  // words at a time: the scheduler keeps each share between its MFMAs, so that the
+  // matrix pipe and the vector unit run side by side within the wave.
+  auto half = [&](const PfFrags& f, int st, int gg, const uint32_t (&w)[4], uint32_t sp,
+                  PfFrags& n) {
+    const ColScale sa = col_scale(bf_lo(sp)), sb = col_scale(bf_hi(sp));
+    bf16x8_t A[2][2];
+    read_a(A[0], st, gg, 0);
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-          const uint16_t* ap = &s_a[buf * kStage + (32 * rb + c) * kPfLdsStride + 32 * gg + 16 * h];
-          const bf16x8_t A1 = *reinterpret_cast<const bf16x8_t*>(ap);
-          const bf16x8_t A2 = *reinterpret_cast<const bf16x8_t*>(ap + 8);
-          accx[rb] = mfma(A1, f.x1, accx[rb]);
-          accx[rb] = mfma(A2, f.x2, accx[rb]);
-          accy[rb] = mfma(A1, f.y1, accy[rb]);
-          accy[rb] = mfma(A2, f.y2, accy[rb]);
-        }
+    for (int rb = 0; rb < RB; ++rb) {
+      if (rb + 1 < RB) read_a(A[(rb + 1) & 1], st, gg, rb + 1);
+      const bf16x8_t A1 = A[rb & 1][0], A2 = A[rb & 1][1];
+      accx[rb] = mfma(A1, f.get(0), accx[rb]);
+      accy[rb] = mfma(A1, f.get(2), accy[rb]);
+      accx[rb] = mfma(A2, f.get(1), accx[rb]);
+      accy[rb] = mfma(A2, f.get(3), accy[rb]);
+#pragma unroll
+      for (int jj = 4 * rb / RB; jj < 4 * (rb + 1) / RB; ++jj) n.put(jj, dequant_word(w[jj], sa, sb, dq));
+      constexpr int kV = (84 + 4 * RB - 1) / (4 * RB);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        if (i == 0 && rb + 1 < RB) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, kV, 0);
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
-  PfB b_even, b_odd;
-  u32x4_t st_even[kStaged], st_odd[kStaged];
-  load_a(st_even, 0);
-  load_b(b_even, 0);
-  load_a(st_odd, 1);
-  load_b(b_odd, 1);
-  store_a(st_even, 0);
-  __syncthreads();
-  // Invariant at the top of each pair: s_a[0] holds chunk ch, st_odd holds
-  // (or is loading) chunk ch + 1, b_even / b_odd hold chunks ch / ch + 1.
-  // One exit only and no tail copy of the loop body, so the accumulators
-  // keep their registers.  With an odd chunk count the last pair's second
-  // chunk is past the end: its activations are zeros, and adding +0 to an
-  // accumulator that started at +0 changes nothing.
-  const int pairs = (chunks + 1) >> 1;
-  for (int pr = 0; pr < pairs; ++pr) {
-    const int ch = 2 * pr;
-    load_a(st_even, ch + 2);
-    compute(b_even, 0);
-    load_b(b_even, ch + 2);
-    // s_a[1] was last read in the previous pair, before the barrier that ended it
-    store_a(st_odd, 1);
-    __syncthreads();
-    load_a(st_odd, ch + 3);
-    compute(b_odd, 1);
-    load_b(b_odd, ch + 3);
-    // every wave finished reading s_a[0] (chunk ch) before the barrier above;
-    // past the last chunk this stages a clamped copy nobody reads
-    store_a(st_even, 0);
-    __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NS - 1; ++i)
+    if (i < chunks) stage_in(i, i * kStage);
+  if (chunks >= NS - 1) vm_wait<(NS - 2) * P>(); else vm_wait<0>();
+  PfFrags f0, f1;
+  uint32_t w0[4], w1[4], sc0 = 0, sc1 = 0;
+  if constexpr (!IDLE) {
+    read_w(w0, 0, 0);
+    sc0 = *reinterpret_cast<const uint32_t*>(s_rd);
+    sc1 = *reinterpret_cast<const uint32_t*>(s_rd + 128);
+    read_w(w1, 0, 1);
+    const ColScale sa = col_scale(bf_lo(sc0)), sb = col_scale(bf_hi(sc0));
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) f0.put(jj, dequant_word(w0[jj], sa, sb, dq));
   }
+  // Chunk ch lies in stage ch % NS.  At the top every wave has waited for its own part
+  // of the chunk, so the barrier makes the whole stage readable, and every wave is done
+  // with the stage of chunk ch - 1, which chunk ch + NS - 1 then overwrites.  A wave's
+  // weights are its own, so the next chunk's first group is dequantised beside this
+  // chunk's second group of products, ahead of the barrier.
+  int st = 0, st_in = (NS - 1) * kStage;
+  auto chunk = [&](int ch, auto more_c) {
+    constexpr bool more = decltype(more_c)::value;  // chunk ch + NS - 1 exists
+    lds_barrier();
+    if constexpr (more) stage_in(ch + NS - 1, st_in);
+    st_in = st;
+    const int st_next = st + kStage == NS * kStage ? 0 : st + kStage;
+    if constexpr (!IDLE) half(f0, st, 0, w1, sc1, f1);
+    vm_wait<more ? (NS - 2) * P : 0>();
+    if constexpr (!IDLE) {
+      read_w(w0, st_next, 0);
+      sc0 = *reinterpret_cast<const uint32_t*>(s_rd + st_next);
+      sc1 = *reinterpret_cast<const uint32_t*>(s_rd + st_next + 128);
+      read_w(w1, st_next, 1);
+      half(f1, st, 1, w0, sc0, f0);
+    }
+    st = st_next;
+  };
+  int ch = 0;
+  for (; ch + NS - 1 < chunks; ++ch) chunk(ch, std::true_type{});
+  for (; ch < chunks; ++ch) chunk(ch, std::false_type{});
+  lds_barrier();  // the epilogue's staging overwrites the ring
+  uint16_t* s_a = reinterpret_cast<uint16_t*>(smem);
 
   if (p.act != nullptr) {
     // W13 + SwiGLU in two row halves (rows 64 ph .. 64 ph + 63, the 32-row
@@ -872,7 +929,7 @@ __device__ __forceinline__ void prefill_tile(const GemmArgs& p, uint16_t* s_a, u
     const int gate_tiles = p.inter >> 6;
 #pragma unroll
     for (int ph = 0; ph < R / 64; ++ph) {
-      if constexpr (RB > 0) {
+      if constexpr (!IDLE) {
         const int pair = wave & 1, half = wave >> 1;  // half 0: gate, 1: up
         const int col = (c >> 3) * 16 + (c & 7);
 #pragma unroll
@@ -925,7 +982,7 @@ __device__ __forceinline__ void prefill_tile(const GemmArgs& p, uint16_t* s_a, u
   const int wave = threadIdx.x >> 6;
 #pragma unroll
   for (int ph = 0; ph < R / 64; ++ph) {
-    if constexpr (RB > 0) {
+    if constexpr (!IDLE) {
       const int col = wave * 64 + (c >> 3) * 16 + (c & 7);
 #pragma unroll
       for (int rbl = 0; rbl < 2; ++rbl) {
@@ -977,12 +1034,12 @@ constexpr int kPfScanSlab = 1024;  // block experts staged in LDS per scan pass
 // blocks, block order.
 template <int R>
 __device__ __forceinline__ void prefill_block(const GemmArgs& p, int tx, int ty) {
-  __shared__ __align__(16) uint16_t s_a[pf_lds_elems(R)];
-  __shared__ __align__(16) uint32_t s_w[4][kSlotDwords];
+  __shared__ __align__(1024) uint8_t smem[pf_ring_bytes(R)];
   __shared__ int s_sid[R];
   __shared__ float s_tw[R];  // with mul: the row's top-k weight rounded to bf16
-  __shared__ int s_e[kPfScanSlab];
-  __shared__ int s_tile;
+  int* s_e = reinterpret_cast<int*>(smem);  // the scan is over before the ring is filled
+  int& s_tile = s_e[kPfScanSlab];
+  static_assert(pf_ring_bytes(R) >= (kPfScanSlab + 1) * 4, "the scan's slab fits the ring");
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1108,27 +1165,21 @@ __device__ __forceinline__ void prefill_block(const GemmArgs& p, int tx, int ty)
     nt = tx * 4 + wave;
     tile_ok = nt < (p.size_n >> 6);
   }
-  const int rb = tile_ok ? __builtin_amdgcn_readfirstlane((row_end + 31) >> 5) : 0;
-  uint32_t* s_w_wave = s_w[wave];
-  if constexpr (R == 64) {
-    switch (rb) {
-      case 0: prefill_tile<0, R>(p, s_a, s_w_wave, s_sid, s_tw, expert, nt, tx); break;
-      case 1: prefill_tile<1, R>(p, s_a, s_w_wave, s_sid, s_tw, expert, nt, tx); break;
-      default: prefill_tile<2, R>(p, s_a, s_w_wave, s_sid, s_tw, expert, nt, tx); break;
-    }
-  } else {
-    switch (rb) {
-      case 0: prefill_tile<0, R>(p, s_a, s_w_wave, s_sid, s_tw, expert, nt, tx); break;
-      case 1: prefill_tile<1, R>(p, s_a, s_w_wave, s_sid, s_tw, expert, nt, tx); break;
-      case 2: prefill_tile<2, R>(p, s_a, s_w_wave, s_sid, s_tw, expert, nt, tx); break;
-      case 3: prefill_tile<3, R>(p, s_a, s_w_wave, s_sid, s_tw, expert, nt, tx); break;
-      default: prefill_tile<4, R>(p, s_a, s_w_wave, s_sid, s_tw, expert, nt, tx); break;
-    }
-  }
+  // the tile's routed 32-row blocks (wave- and workgroup-uniform): at least one is run
+  const int rb = __builtin_amdgcn_readfirstlane((row_end + 31) >> 5);
+  auto go = [&](auto RBc) {
+    constexpr int RB = decltype(RBc)::value;
+    if (tile_ok) prefill_tile<RB, R, false>(p, smem, s_sid, s_tw, expert, nt, tx);
+    else prefill_tile<RB, R, true>(p, smem, s_sid, s_tw, expert, nt, tx);
+  };
+  if (rb <= 1) go(std::integral_constant<int, 1>{});
+  else if (R == 64 || rb == 2) go(std::integral_constant<int, 2>{});
+  else if (rb == 3) go(std::integral_constant<int, R == 64 ? 2 : 3>{});
+  else go(std::integral_constant<int, R == 64 ? 2 : 4>{});
 }
 
 template <int R>
-__global__ __launch_bounds__(256, 2) void wna16_prefill_kernel(GemmArgs p) {
+__global__ __launch_bounds__(256, R == 64 ? 3 : 2) void wna16_prefill_kernel(GemmArgs p) {
   prefill_block<R>(p, blockIdx.x, blockIdx.y);
 }
 
@@ -1137,7 +1188,7 @@ __global__ __launch_bounds__(256, 2) void wna16_prefill_kernel(GemmArgs p) {
 // workgroups, then the second's, each in its own x-fastest order, so one
 // stream keeps both on the GPU at once.
 template <int R>
-__global__ __launch_bounds__(256, 2) void wna16_prefill_pair_kernel(
+__global__ __launch_bounds__(256, R == 64 ? 3 : 2) void wna16_prefill_pair_kernel(
     GemmArgs p0, GemmArgs p1, int x0, int n0, int x1) {
   const int l = static_cast<int>(blockIdx.x);
   if (l < n0)
@@ -1197,12 +1248,25 @@ __global__ void w13_swiglu_partials_kernel(GemmArgs p, uint16_t* __restrict__ ac
 
 bool valid_block_size(int bs) { return bs == 8 || (bs >= 16 && bs <= 64 && bs % 16 == 0); }
 
-// Prefill tile height: 64 rows when the routes could fill at most 64 rows per
-// expert on average, else 128.  Few rows per expert leave the 128-row tiles
-// mostly one or two 32-row blocks anyway, while a problem's large experts (a
-// shared expert in the same pair launch) would get tiles twice as long as the
-// rest, which then set the launch's last round.
-bool small_prefill_tiles(long long routes, long long experts) { return routes <= 64LL * experts; }
+// Whether the routes of a launch come to at most `rows` rows per expert on average.  A
+// launch sees every token's routes; 48 local experts are the EP8 share of a 384-expert
+// model (the only share the kimi_* entry points accept), which gets an eighth of them.
+bool mean_rows_at_most(long long routes, long long experts, long long rows) {
+  return routes <= rows * experts * (experts == 48 ? 8 : 1);
+}
+
+// Prefill tile height: 64 rows (three workgroups a CU instead of two) when the
+// routes come to few rows per expert, else 128.  Few rows per expert leave the
+// 128-row tiles mostly one or two 32-row blocks anyway, while a problem's large
+// experts (a shared expert in the same pair launch) would get tiles twice as long
+// as the rest, which then set the launch's last round.  An eighth share's mean is
+// only expected, and skewed routing fills some experts far past it, so there the
+// line is lower: Kimi's MoE block at 1000 tokens (21 rows) 473 us with 64-row tiles
+// against 491, its routed experts under Zipf routing 381 against 393; at 1500 tokens
+// (31 rows) 597 against 613, but 460 against 444 under Zipf.
+bool small_prefill_tiles(long long routes, long long experts) {
+  return mean_rows_at_most(routes, experts, experts == 48 ? 24 : 64);
+}
 
 // The kernels address one expert's weights and the activations through
 // 32-bit buffer ranges.  The activation range must also stay at or below
@@ -1270,8 +1334,9 @@ int wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long long 
     return launch_status("wna16_gemm (decode)");
   }
   if (max_m_blocks > 65535) return fail(kNotSupported, "wna16_gemm: too many m-blocks");
+  const long long rows = static_cast<long long>(size_m) * top_k;
   const dim3 grid(ceil_div(n_tiles, 4), max_m_blocks);
-  if (small_prefill_tiles(static_cast<long long>(size_m) * top_k, local_experts))
+  if (small_prefill_tiles(rows, local_experts))
     hipLaunchKernelGGL(wna16_prefill_kernel<64>, grid, dim3(256), 0, stream, args);
   else
     hipLaunchKernelGGL(wna16_prefill_kernel<128>, grid, dim3(256), 0, stream, args);
@@ -1322,8 +1387,9 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
                   b_scales, nullptr, sorted_token_ids, expert_ids, num_tokens_post_padded,
                   nullptr, sorted_token_ids_len, moe_block_size, top_k, 0, size_m, size_n,
                   size_k, local_experts, 1, nullptr, act, inter};
+    const long long rows = static_cast<long long>(size_m) * top_k;
     const dim3 grid(ceil_div(inter / 64, 2), max_m_blocks);
-    if (small_prefill_tiles(static_cast<long long>(size_m) * top_k, local_experts))
+    if (small_prefill_tiles(rows, local_experts))
       hipLaunchKernelGGL(wna16_prefill_kernel<64>, grid, dim3(256), 0, stream, args);
     else
       hipLaunchKernelGGL(wna16_prefill_kernel<128>, grid, dim3(256), 0, stream, args);
