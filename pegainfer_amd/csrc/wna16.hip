@@ -626,6 +626,166 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 6) void wna16_decode16_k
   }
 }
 
+// ---------------------------------------------------------------------------
+// Decode kernel for blocks of 32 to 64 rows that hold few routed ones: the
+// 32-row kernel above with all 32 MFMA rows in use (two 16-byte activation
+// loads per lane and group, k 0..7 and 8..15 of its half).  blockIdx.z is the
+// 32-row part of the block; parts without a routed row leave at once.  Bound by
+// the dequant's vector instructions like the kernels above; 120 VGPRs, four waves
+// per SIMD, so two 8-wave W13 workgroups a CU.  Kimi W13 + SwiGLU / W2 at 160
+// tokens (35 experts touched): 122 us (4.7 TB/s) / 68 us against 158 / 65 with the
+// tile kernel, whose 560 workgroups of 100 us each left most CUs idle for the last
+// third of the launch.
+struct GroupRegs32 {
+  u32x4_t raw;
+  uint32_t sp;
+  u32x4_t a0, a1;
+};
+
+template <int WK, int D, bool kPair = false>
+__global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 4) void wna16_decode32_kernel(GemmArgs p) {
+  static_assert(D % 2 == 0, "the two transpose slots alternate with the ring position");
+  constexpr int kWaves = WK * (kPair ? 2 : 1);
+  __shared__ int s_sid[32];
+  // the transpose slots ([wave][2][kSlotDwords]), then the reduction ([wave][32][64])
+  __shared__ __align__(16) uint32_t s_mem[kWaves * 32 * 64];
+  static_assert(2 * kSlotDwords <= 32 * 64, "the slots fit the reduction buffer");
+
+  const int n_tiles = p.size_n >> 6;
+  const int n_units = kPair ? (p.inter >> 6) : n_tiles;
+  const int split = blockIdx.x / n_units;
+  const int mb = blockIdx.y, row0 = 32 * blockIdx.z;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int valid_limit = p.size_m * p.top_k;
+  int sid = valid_limit;
+  if (lane < 32 && row0 + lane < p.bs && mb * p.bs + row0 + lane < p.sorted_len)
+    sid = p.sorted_ids[mb * p.bs + row0 + lane];
+  const int expert = __builtin_amdgcn_readfirstlane(p.expert_ids[mb]);
+  const int ntp = min(p.ntp[0], p.sorted_len);
+  // every wave holds the part's 32 ids, so the part with no routed row is left by all
+  const bool routed = __ballot(static_cast<unsigned>(sid) < static_cast<unsigned>(valid_limit)) != 0;
+  if (ntp < (mb + 1) * p.bs || expert < 0 || expert >= p.num_experts || !routed) return;
+
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kw = wave % WK;
+  const int half = wave / WK;
+  const int nt = blockIdx.x % n_units + (kPair ? half * (p.inter >> 6) : 0);
+  if (tid < 32) s_sid[tid] = sid;
+  const int c = lane & 31, h = lane >> 5;
+  const int my_sid = __builtin_amdgcn_ds_bpermute(c << 2, sid);
+  const int K = p.size_k, N = p.size_n;
+  const int groups = K >> 5;
+  const int gs0 = (groups * split) / p.splits, gs1 = (groups * (split + 1)) / p.splits;
+  const int g0 = gs0 + ((gs1 - gs0) * kw) / WK, g1 = gs0 + ((gs1 - gs0) * (kw + 1)) / WK;
+
+  const uint32_t expert_bytes = static_cast<uint32_t>(N) * static_cast<uint32_t>(K) / 2u;
+  const __amdgpu_buffer_rsrc_t wr = make_rsrc(
+      p.qweight + static_cast<long long>(expert) * (expert_bytes / 4u), expert_bytes);
+  const uint32_t tile_row_bytes = static_cast<uint32_t>(n_tiles) * 512u;
+  const uint32_t w_voff = static_cast<uint32_t>(h) * tile_row_bytes +
+                          static_cast<uint32_t>(nt) * 512u + static_cast<uint32_t>(c) * 16u;
+  const uint32_t w_step = 2u * tile_row_bytes;
+  const uint32_t scale_bytes = static_cast<uint32_t>(groups) * static_cast<uint32_t>(N) * 2u;
+  const __amdgpu_buffer_rsrc_t sr = make_rsrc(
+      p.scales + static_cast<long long>(expert) * groups * N, scale_bytes);
+  const uint32_t s_voff = (static_cast<uint32_t>(nt) * 64u + 8u * (c & 7) + 2u * (c >> 3)) * 2u;
+  const uint32_t s_step = static_cast<uint32_t>(N) * 2u;
+  const __amdgpu_buffer_rsrc_t ar =
+      make_rsrc(p.input, static_cast<uint32_t>(p.size_m) * static_cast<uint32_t>(K) * 2u);
+  const uint32_t a_voff =
+      static_cast<unsigned>(my_sid) < static_cast<unsigned>(valid_limit)
+          ? (static_cast<uint32_t>(my_sid / p.top_k) * static_cast<uint32_t>(K) + 16u * h) * 2u
+          : kOutOfRange;
+
+  uint32_t* slots = s_mem + wave * 2 * kSlotDwords;
+  uint32_t* slot_w0 = slots + h * 160 + c;
+  const uint32_t* slot_r0 = slots + h * 160 + 4 * c;
+
+  auto load_group = [&](GroupRegs32& r, int g) {
+    g = min(max(g, 0), groups - 1);
+    r.raw = buf_load_b128<kStream>(wr, w_voff, static_cast<uint32_t>(g) * w_step);
+    r.sp = buf_load_b32<kStream>(sr, s_voff, static_cast<uint32_t>(g) * s_step);
+    r.a0 = buf_load_b128(ar, a_voff, static_cast<uint32_t>(g) * 64u);
+    r.a1 = buf_load_b128(ar, a_voff + 16u, static_cast<uint32_t>(g) * 64u);
+  };
+
+  const DqConst dq = dq_consts();
+  floatx16_t accx = {}, accy = {};
+  GroupRegs32 slot[D];
+#pragma unroll
+  for (int q = 0; q < D; ++q) {
+    load_group(slot[q], g0 + q < g1 ? g0 + q : g1 - 1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  auto write_tr = [&](const GroupRegs32& r, int par) {
+    uint32_t* sw = slot_w0 + par * kSlotDwords;
+    sw[0] = r.raw[0];
+    sw[32] = r.raw[1];
+    sw[64] = r.raw[2];
+    sw[96] = r.raw[3];
+  };
+  auto compute_group = [&](const GroupRegs32& r, int par) {
+    const u32x4_t fw = *reinterpret_cast<const u32x4_t*>(slot_r0 + par * kSlotDwords);
+    const uint32_t w4[4] = {fw[0], fw[1], fw[2], fw[3]};
+    const BFrags b = make_b(w4, r.sp, dq);
+    const bf16x8_t A1 = __builtin_bit_cast(bf16x8_t, r.a0);
+    const bf16x8_t A2 = __builtin_bit_cast(bf16x8_t, r.a1);
+    accx = mfma(A1, b.x1, accx);
+    accy = mfma(A1, b.y1, accy);
+    accx = mfma(A2, b.x2, accx);
+    accy = mfma(A2, b.y2, accy);
+  };
+
+  const int rounds = (g1 - g0) / D;
+  int g = g0;
+  write_tr(slot[0], 0);
+  for (int r = 0; r < rounds; ++r, g += D) {
+#pragma unroll
+    for (int q = 0; q < D; ++q) {
+      write_tr(slot[(q + 1) % D], (q + 1) & 1);
+      compute_group(slot[q], q & 1);
+      load_group(slot[q], min(g + q + D, g1 - 1));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < D - 1; ++q) {
+    if (g + q < g1) {
+      if (q + 1 < D - 1 && g + q + 1 < g1) write_tr(slot[q + 1], (q + 1) & 1);
+      compute_group(slot[q], q & 1);
+    }
+  }
+
+  float* s_red = reinterpret_cast<float*>(s_mem);
+  __syncthreads();  // every wave is done with its slots
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    s_red[(wave * 32 + i) * 64 + lane] = accx[i];
+    s_red[(wave * 32 + 16 + i) * 64 + lane] = accy[i];
+  }
+  __syncthreads();
+
+  const int col0 = (c >> 3) * 16 + (c & 7);
+  for (int j = wave; j < 32; j += kWaves) {
+    float sg = 0.0f, su = 0.0f;
+#pragma unroll
+    for (int w = 0; w < WK; ++w) {
+      sg += s_red[(w * 32 + j) * 64 + lane];
+      if constexpr (kPair) su += s_red[((WK + w) * 32 + j) * 64 + lane];
+    }
+    const int rsid = s_sid[acc_row(j & 15, h)];
+    if (static_cast<unsigned>(rsid) >= static_cast<unsigned>(valid_limit)) continue;
+    const int col = (blockIdx.x % n_units) * 64 + col0 + (j < 16 ? 0 : 8);
+    if constexpr (kPair)
+      p.act[static_cast<long long>(rsid) * p.inter + col] =
+          swiglu_one(bf2f(f2bf(sg)), bf2f(f2bf(su)));
+    else if (p.partial)
+      p.partial[(static_cast<long long>(split) * valid_limit + rsid) * N + col] = sg;
+    else
+      p.output[static_cast<long long>(rsid) * N + col] = epilogue_value(sg, rsid, p);
+  }
+}
+
 constexpr int kDecodeDepth = 4;
 
 // WK = 4 runs the 16x16x32 kernel, the other share counts the 32-row one
@@ -633,7 +793,12 @@ constexpr int kDecodeDepth = 4;
 // its extra scale work cost C1/C2 2-4%).
 template <int WK>
 void launch_decode(const GemmArgs& args, int max_m_blocks, hipStream_t stream) {
-  const dim3 grid(args.size_n / 64 * args.splits, max_m_blocks);
+  const dim3 grid(args.size_n / 64 * args.splits, max_m_blocks, ceil_div(args.bs, 32));
+  if (args.bs > 16) {
+    hipLaunchKernelGGL((wna16_decode32_kernel<WK, kDecodeDepth>), grid, dim3(64 * WK), 0, stream,
+                       args);
+    return;
+  }
   if constexpr (WK == 4) {
     hipLaunchKernelGGL((wna16_decode16_kernel<WK, kDecodeDepth>), grid, dim3(64 * WK), 0, stream,
                        args);
@@ -649,7 +814,12 @@ void launch_decode(const GemmArgs& args, int max_m_blocks, hipStream_t stream) {
 
 template <int WK>
 void launch_decode_pair(const GemmArgs& args, int max_m_blocks, hipStream_t stream) {
-  const dim3 grid(args.inter / 64, max_m_blocks);
+  const dim3 grid(args.inter / 64, max_m_blocks, ceil_div(args.bs, 32));
+  if (args.bs > 16) {
+    hipLaunchKernelGGL((wna16_decode32_kernel<WK, kDecodeDepth, true>), grid, dim3(128 * WK), 0,
+                       stream, args);
+    return;
+  }
   if constexpr (WK == 4) {
     hipLaunchKernelGGL((wna16_decode16_kernel<WK, kDecodeDepth, true>), grid, dim3(128 * WK), 0,
                        stream, args);
@@ -1268,6 +1438,29 @@ bool small_prefill_tiles(long long routes, long long experts) {
   return mean_rows_at_most(routes, experts, experts == 48 ? 24 : 64);
 }
 
+// Launches at block sizes above 16 that take the decode kernel's 32-row form instead
+// of the tile kernel: its units are a column tile's K shares, an eighth of a tile
+// workgroup's work, so few rows or few tiles still balance over the CUs, but every
+// column tile reads the activations again, which rules out many rows.
+//   * Few rows per expert on average (a decode batch on an eighth share: Kimi's decode
+//     layer at 110 / 180 / 220 / 256 tokens 242 / 286 / 316 / 313 us against
+//     271 / 310 / 336 / 317 with tiles; at 400 tokens, 8 rows, 393 against 364).
+//   * One expert whose 32-row parts and column tiles are at most three workgroups a CU:
+//     the tile kernel would leave CUs idle for its whole chain over K (9728 x 2560,
+//     40 / 90 rows 18 / 23 against 34 / 39 us; 2048 x 7168, 64 rows 27 against 82; 14336 x
+//     4096, 128 rows, 3.5 a CU, 62 against 60).  Up to 128 rows, so that the shared
+//     expert of a prefill chunk stays with the routed experts' launch.
+bool few_rows(long long routes, long long experts, int n_tiles, int cu_count) {
+  if (experts == 1) return routes <= 128 && (routes + 31) / 32 * n_tiles <= 3LL * cu_count;
+  return mean_rows_at_most(routes, experts, 6);
+}
+// K shares (waves per column tile) of that form: four once the tiles of the 32-row
+// parts fill half the GPU's workgroup slots, else eight.
+int few_rows_waves(long long routes, long long experts, int n_tiles, int cu_count) {
+  const long long parts = experts == 1 ? (routes + 31) / 32 : std::min(routes, experts);
+  return parts * n_tiles >= 2LL * cu_count ? 4 : 8;
+}
+
 // The kernels address one expert's weights and the activations through
 // 32-bit buffer ranges.  The activation range must also stay at or below
 // 2^31 bytes: offset 0x80000000 is how rows not routed here read zeros.
@@ -1335,6 +1528,13 @@ int wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long long 
   }
   if (max_m_blocks > 65535) return fail(kNotSupported, "wna16_gemm: too many m-blocks");
   const long long rows = static_cast<long long>(size_m) * top_k;
+  if (few_rows(rows, local_experts, n_tiles, cu_count)) {
+    if (few_rows_waves(rows, local_experts, n_tiles, cu_count) == 4)
+      launch_decode<4>(args, max_m_blocks, stream);
+    else
+      launch_decode<8>(args, max_m_blocks, stream);
+    return launch_status("wna16_gemm (few rows)");
+  }
   const dim3 grid(ceil_div(n_tiles, 4), max_m_blocks);
   if (small_prefill_tiles(rows, local_experts))
     hipLaunchKernelGGL(wna16_prefill_kernel<64>, grid, dim3(256), 0, stream, args);
@@ -1387,7 +1587,16 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
                   b_scales, nullptr, sorted_token_ids, expert_ids, num_tokens_post_padded,
                   nullptr, sorted_token_ids_len, moe_block_size, top_k, 0, size_m, size_n,
                   size_k, local_experts, 1, nullptr, act, inter};
+    if (cu_count <= 0) cu_count = current_cu_count();
+    if (cu_count <= 0) return fail(kInvalidValue, "w13_swiglu: no device");
     const long long rows = static_cast<long long>(size_m) * top_k;
+    if (few_rows(rows, local_experts, size_n / 64, cu_count)) {
+      if (few_rows_waves(rows, local_experts, size_n / 64, cu_count) == 4)
+        launch_decode_pair<4>(args, max_m_blocks, stream);
+      else
+        launch_decode_pair<8>(args, max_m_blocks, stream);
+      return launch_status("w13_swiglu (few rows)");
+    }
     const dim3 grid(ceil_div(inter / 64, 2), max_m_blocks);
     if (small_prefill_tiles(rows, local_experts))
       hipLaunchKernelGGL(wna16_prefill_kernel<64>, grid, dim3(256), 0, stream, args);
@@ -1498,6 +1707,23 @@ int prefill_problem(const pega_wna16_problem* q, const char* which, GemmArgs& ar
   return kSuccess;
 }
 
+// A checked problem as its own launch.  Weights that are not multiplied are not read, so a
+// NULL there is replaced by a pointer the single entry's null check accepts.
+int single_problem(const pega_wna16_problem* q, int cu_count, hipStream_t stream) {
+  if (q->act != nullptr)
+    return wna16_w13_swiglu(q->input, q->act, nullptr, 0, q->b_qweight, q->b_scales,
+                            q->sorted_token_ids, q->expert_ids, q->num_tokens_post_padded,
+                            q->sorted_token_ids_len, q->moe_block_size, q->top_k, q->size_m,
+                            q->size_n / 2, q->size_k, q->local_experts, q->group_size, cu_count,
+                            stream);
+  const float* tw = q->topk_weights ? q->topk_weights : reinterpret_cast<const float*>(q->input);
+  return wna16_gemm(q->input, q->output, nullptr, 0, q->b_qweight, q->b_scales, nullptr, 0,
+                    q->sorted_token_ids, q->expert_ids, q->num_tokens_post_padded, tw,
+                    q->sorted_token_ids_len, q->moe_block_size, q->top_k,
+                    q->mul_topk_weights != 0, q->size_m, q->size_n, q->size_k, q->local_experts,
+                    q->group_size, cu_count, stream);
+}
+
 }  // namespace
 
 int wna16_prefill_pair(const pega_wna16_problem* first, const pega_wna16_problem* second,
@@ -1508,6 +1734,18 @@ int wna16_prefill_pair(const pega_wna16_problem* first, const pega_wna16_problem
   if (rc != kSuccess) return rc;
   rc = prefill_problem(second, "second", a1, x1, y1);
   if (rc != kSuccess) return rc;
+  // A problem that its own launch would not run on tiles: both run as their own launches,
+  // so that each output keeps the bits of its single launch.
+  const int cu_count = current_cu_count();
+  if (cu_count <= 0) return fail(kInvalidValue, "wna16_prefill_pair: no device");
+  const bool grids_fit = y0 <= 65535 && y1 <= 65535;  // of the single launches
+  if (grids_fit && (few_rows(static_cast<long long>(a0.size_m) * a0.top_k, a0.num_experts,
+                             a0.size_n / 64, cu_count) ||
+                    few_rows(static_cast<long long>(a1.size_m) * a1.top_k, a1.num_experts,
+                             a1.size_n / 64, cu_count))) {
+    rc = single_problem(first, cu_count, stream);
+    return rc != kSuccess ? rc : single_problem(second, cu_count, stream);
+  }
   const long long n0 = static_cast<long long>(x0) * y0, n1 = static_cast<long long>(x1) * y1;
   if (n0 + n1 > 0x7fffffffLL)
     return fail(kNotSupported, "wna16_prefill_pair: %lld workgroups exceed the grid", n0 + n1);

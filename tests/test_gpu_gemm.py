@@ -501,3 +501,67 @@ def test_decode16_uneven_and_empty_k_shares(oracle, K):
     got_act = host(act)
     assert np.array_equal(got_act[local], oracle.swiglu(ref13, inter)[local]), f"W13 K={K}"
     assert (got_act[~local] == 0x4040).all()
+
+
+@pytest.mark.parametrize("E,T,topk,bs,N,K,mul", [
+    (48, 20, 8, 32, 128, 64, False),     # two groups for eight K shares, one column tile pair
+    (48, 100, 8, 48, 192, 160 * 2, True),  # odd tile count, a 48-row block's second, half part
+    (48, 250, 8, 64, 4096, 512, True),   # four K shares
+    (1, 17, 1, 64, 640, 192, False), (1, 31, 1, 64, 640, 192, True), (1, 32, 1, 64, 640, 192, False),
+    (1, 33, 1, 64, 640, 448, True),      # second 32-row part with one row
+    (1, 65, 1, 64, 128, 1024, False),    # second block
+    (1, 128, 1, 32, 128, 2048, True), (6, 30, 1, 32, 256, 256, True)])
+def test_few_rows_form_exact(oracle, E, T, topk, bs, N, K, mul):
+    """Block sizes above 16 with few rows (the decode kernel's 32-row form): exact inputs, so
+    both the GEMM and W13 + SwiGLU equal the oracle bit for bit whatever the K shares; rows not
+    routed here keep their contents."""
+    from pegainfer_amd import ops
+    g = np.random.default_rng(E * 1000 + T + K)
+    q = g.integers(-8, 8, size=(E, N, K))
+    scale_bits = oracle.f32_to_bf16(
+        (2.0 ** g.integers(-6, -2, size=(E, N, K // 32))).astype(np.float32))
+    a_bits = oracle.f32_to_bf16(g.integers(-2, 3, size=(T, K)).astype(np.float32))
+    # an eighth of the routes local for 48 experts, with one expert that takes many rows
+    idx = g.integers(0, 8 * E if E > 1 else 1, size=(T, topk)).astype(np.int32)
+    if E > 1:
+        idx[: T // 2, 0] = 2
+    tw = (2.0 ** g.integers(-2, 2, size=(T, topk))).astype(np.float32)
+    got, ref = _run(oracle, E=E, N=N, K=K, T=T, topk=topk, bs=bs, mul=mul, a_bits=a_bits, q=q,
+                    scale_bits=scale_bits, idx=idx, tw=tw)
+    assert np.array_equal(got, ref)
+    if N % 128:
+        return
+    inter = N // 2
+    w, packed = _setup(E, N, K, q, scale_bits)
+    ws = ops.KimiMarlinRouteWorkspace(T, bs, topk=topk, local_experts=E)
+    routing = ops.moe_align_block_size(ws, dev(idx.reshape(-1)), T, T, 0)
+    gws = ops.KimiMarlinWna16Workspace(ws.max_m_blocks, N, bs)
+    act = torch.full((T * topk, inter), 3.0, dtype=torch.bfloat16, device="cuda")
+    ops.wna16_w13_swiglu(gws, routing, dev(a_bits), w, act, top_k=topk, size_m=T)
+    r = {k: host(v) for k, v in (("sorted_token_ids", routing.sorted_token_ids),
+                                 ("expert_ids", routing.expert_ids),
+                                 ("num_tokens_post_padded", routing.num_tokens_post_padded))}
+    ref13 = oracle.wna16_gemm(a_bits, packed, scale_bits, r, tw, moe_block_size=bs, top_k=topk,
+                              mul_topk_weights=False, size_m=T, size_n=N, size_k=K, threads=16)
+    local = idx.reshape(-1) < E
+    assert np.array_equal(host(act)[local], oracle.swiglu(ref13, inter)[local])
+    assert (host(act)[~local] == 0x4040).all()
+
+
+@pytest.mark.parametrize("R_rows", [1, 32, 33, 64, 65, 96, 97, 128, 129])
+@pytest.mark.parametrize("K", [64, 128, 192, 320, 512])
+def test_tile_kernel_rows_and_chunks_exact(oracle, R_rows, K):
+    """The prefill tile kernel at every routed 32-row block count of a tile and at chunk counts
+    below, at and past its ring's stages; a column tile count that leaves idle waves."""
+    g = np.random.default_rng(R_rows * 7 + K)
+    E, N, T = 2, 320, 400
+    q = g.integers(-8, 8, size=(E, N, K))
+    scale_bits = oracle.f32_to_bf16(
+        (2.0 ** g.integers(-6, -2, size=(E, N, K // 32))).astype(np.float32))
+    a_bits = oracle.f32_to_bf16(g.integers(-2, 3, size=(T, K)).astype(np.float32))
+    idx = np.zeros((T, 1), np.int32)
+    idx[g.permutation(T)[:R_rows], 0] = 1
+    for bs in (32, 64):
+        got, ref = _run(oracle, E=E, N=N, K=K, T=T, topk=1, bs=bs, mul=False, a_bits=a_bits, q=q,
+                        scale_bits=scale_bits, idx=idx, tw=np.ones((T, 1), np.float32))
+        assert np.array_equal(got, ref)
