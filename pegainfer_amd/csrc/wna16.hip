@@ -852,10 +852,12 @@ void launch_decode_pair(const GemmArgs& args, int max_m_blocks, hipStream_t stre
 //     the next group is dequantised between this group's MFMAs, a word per row block
 //     at R = 128;
 //   * one barrier per chunk: the activations are shared, the weights are not.
-// Against the register-staged form with the same tiles: Kimi's routed W13 + SwiGLU
-// and W2 under Zipf routing at 4096 tokens 479 -> 467 and 257 -> 254 us, at 1000
-// tokens 185 -> 178 and 101 -> 94 us (with 64-row tiles), DeepSeek-V2-Lite's at 2500
-// tokens 201 -> 196 and 111 -> 110 us.
+//   * a chunk's chain is kept short: activation fragments are read one row block ahead,
+//     through both groups, and the next chunk's first words half a chunk ahead.
+// Against the register-staged form with the same tiles, whole layers: Kimi's routed
+// experts under Zipf routing, 4096 tokens, 794 -> 760 us; DeepSeek-V2-Lite's layer at 512 /
+// 2500 tokens 171 -> 163 / 455 -> 437 us; Kimi's MoE block at 1000 tokens (64-row tiles)
+// 512 -> 483 us.
 // ---------------------------------------------------------------------------
 constexpr int kPfChunk = 64;  // k per stage (2 quant groups)
 // Bytes of one stage beside the activations: per wave two groups' weight words
@@ -1013,15 +1015,18 @@ __device__ __forceinline__ void prefill_tile(const GemmArgs& p, uint8_t* smem, c
   // group (words w, scale pair sp) into n, one row block's four MFMAs and a share of the
   // words at a time: the scheduler keeps each share between its MFMAs, so that the
   // matrix pipe and the vector unit run side by side within the wave.
-  auto half = [&](const PfFrags& f, int st, int gg, const uint32_t (&w)[4], uint32_t sp,
+  bf16x8_t A[2][2];  // the activation fragments of a row block, read one block ahead
+  auto half = [&](const PfFrags& f, int st, auto gg_c, const uint32_t (&w)[4], uint32_t sp,
                   PfFrags& n) {
+    constexpr int gg = decltype(gg_c)::value;
+    constexpr int first = gg * RB;  // row blocks of the chunk's two groups, in turn
     const ColScale sa = col_scale(bf_lo(sp)), sb = col_scale(bf_hi(sp));
-    bf16x8_t A[2][2];
-    read_a(A[0], st, gg, 0);
+    if (gg == 0) read_a(A[0], st, 0, 0);
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
-      if (rb + 1 < RB) read_a(A[(rb + 1) & 1], st, gg, rb + 1);
-      const bf16x8_t A1 = A[rb & 1][0], A2 = A[rb & 1][1];
+      const int q = first + rb, q1 = q + 1;
+      if (q1 < 2 * RB) read_a(A[q1 & 1], st, q1 / RB, q1 % RB);
+      const bf16x8_t A1 = A[q & 1][0], A2 = A[q & 1][1];
       accx[rb] = mfma(A1, f.get(0), accx[rb]);
       accy[rb] = mfma(A1, f.get(2), accy[rb]);
       accx[rb] = mfma(A2, f.get(1), accx[rb]);
@@ -1032,7 +1037,7 @@ __device__ __forceinline__ void prefill_tile(const GemmArgs& p, uint8_t* smem, c
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-        if (i == 0 && rb + 1 < RB) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        if (i == 0 && q1 < 2 * RB) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
         __builtin_amdgcn_sched_group_barrier(0x2, kV, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -1066,14 +1071,16 @@ __device__ __forceinline__ void prefill_tile(const GemmArgs& p, uint8_t* smem, c
     if constexpr (more) stage_in(ch + NS - 1, st_in);
     st_in = st;
     const int st_next = st + kStage == NS * kStage ? 0 : st + kStage;
-    if constexpr (!IDLE) half(f0, st, 0, w1, sc1, f1);
-    vm_wait<more ? (NS - 2) * P : 0>();
+    vm_wait<more ? (NS - 2) * P : 0>();  // this wave's part of chunk ch + 1
     if constexpr (!IDLE) {
       read_w(w0, st_next, 0);
       sc0 = *reinterpret_cast<const uint32_t*>(s_rd + st_next);
-      sc1 = *reinterpret_cast<const uint32_t*>(s_rd + st_next + 128);
+      half(f0, st, std::integral_constant<int, 0>{}, w1, sc1, f1);
+    }
+    if constexpr (!IDLE) {
       read_w(w1, st_next, 1);
-      half(f1, st, 1, w0, sc0, f0);
+      sc1 = *reinterpret_cast<const uint32_t*>(s_rd + st_next + 128);
+      half(f1, st, std::integral_constant<int, 1>{}, w0, sc0, f0);
     }
     st = st_next;
   };
