@@ -153,6 +153,38 @@ __device__ __forceinline__ uint16_t swiglu_one(float g, float u) {
   return f2bf(bf2f(f2bf(silu)) * u);
 }
 
+// ---------------------------------------------------------------- loads straight to LDS
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
+
+// Global memory straight to LDS: lane l's 16 (or 4) bytes at voff + soff go to
+// lds + 16 l (4 l).  In asm so that the compiler, which cannot tell a ring's
+// stages apart, does not drain every load in flight at each LDS read; the kernels
+// count them themselves (vm_wait) and no register is written.  The resource is four
+// words (rsrc_words); lanes out of its range bring zeros.
+__device__ __forceinline__ void dma_b128(u32x4_t rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+}
+__device__ __forceinline__ void dma_b32(u32x4_t rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+               :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void vm_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
+}
+// Every wave's LDS reads have returned and its counted loads have landed.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+__device__ __forceinline__ u32x4_t rsrc_words(const void* base, uint32_t bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(base);
+  u32x4_t r = {static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a))),
+               static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a >> 32))) & 0xffffu,
+               bytes, 0x00020000u};
+  return r;
+}
+
 __host__ __device__ constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 }  // namespace pega

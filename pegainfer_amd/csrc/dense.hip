@@ -19,7 +19,7 @@
 // A permuted k order that reads 256 contiguous bytes per row per step instead
 // quadruples the lines per instruction and ran 2.3x slower.
 //
-// The decode-sized token counts this serves make the GEMM a weight stream:
+// The first kernel below serves up to 32 tokens, where the GEMM is a weight stream:
 // one workgroup owns 16 MR output features for 16 RB tokens (the host picks
 // the shape); its WK waves split K and are reduced through LDS in wave order
 // (deterministic).  Per 32-k step a lane issues one 16-byte load of W per
@@ -44,7 +44,6 @@ namespace {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
 
 constexpr uint32_t kOutOfRange = 0x80000000u;  // voffset that fails every range check
 // W loads are cached too: a step reads 64 bytes of each of 16 rows, so the
@@ -86,7 +85,7 @@ __global__ __launch_bounds__(64 * WK) void dense_gemm_kernel(const uint16_t* __r
   static_assert(!SWIGLU || MR == 2, "SwiGLU pairs one gate and one up tile");
   static_assert(!(SWIGLU && F32), "the SwiGLU epilogue writes bf16");
   uint16_t* __restrict__ Y = static_cast<uint16_t*>(Yv);
-  constexpr int D = MR + RB <= 5 ? 4 : 3;  // the ring fits 128 VGPRs at WK = 16
+  constexpr int D = 4;  // the ring fits 128 VGPRs at WK = 16
   __shared__ float s_red[WK][RB * 4][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -218,12 +217,10 @@ template <int WK, int MR, bool SWIGLU, bool F32>
 void launch_dense_rb(int rb, dim3 grid, const uint16_t* W, const uint16_t* X, void* Y, int M,
                      int N, int K, int stride, hipStream_t stream) {
   const dim3 block(64 * WK);
-  switch (rb) {
-    case 1: hipLaunchKernelGGL((dense_gemm_kernel<WK, MR, 1, SWIGLU, F32>), grid, block, 0, stream, W, X, Y, M, N, K, stride); break;
-    case 2: hipLaunchKernelGGL((dense_gemm_kernel<WK, MR, 2, SWIGLU, F32>), grid, block, 0, stream, W, X, Y, M, N, K, stride); break;
-    case 3: hipLaunchKernelGGL((dense_gemm_kernel<WK, MR, 3, SWIGLU, F32>), grid, block, 0, stream, W, X, Y, M, N, K, stride); break;
-    default: hipLaunchKernelGGL((dense_gemm_kernel<WK, MR, 4, SWIGLU, F32>), grid, block, 0, stream, W, X, Y, M, N, K, stride); break;
-  }
+  if (rb == 1)
+    hipLaunchKernelGGL((dense_gemm_kernel<WK, MR, 1, SWIGLU, F32>), grid, block, 0, stream, W, X, Y, M, N, K, stride);
+  else
+    hipLaunchKernelGGL((dense_gemm_kernel<WK, MR, 2, SWIGLU, F32>), grid, block, 0, stream, W, X, Y, M, N, K, stride);
 }
 
 template <int WK, bool SWIGLU, bool F32>
@@ -236,18 +233,18 @@ void launch_dense(int mr, int rb, dim3 grid, const uint16_t* W, const uint16_t* 
 }
 
 // Row tiles per wave: two where M allows (each X fragment then feeds two
-// MFMAs).  Token blocks per workgroup: up to four, halved once when the grid
-// would leave CUs idle.  Filling the CUs is worth more than reading each W row
-// once: the workgroups that share W rows sit at the same blockIdx.x, and since
-// the row-tile count is a multiple of 8 on the shapes this serves (4096, 7168
-// features) they land on the same XCD and find the rows in its L2 (Kimi
-// gate/up, 64 tokens: 128 workgroups of 64 tokens 26.4 us, 256 of 32 tokens
-// 20.4 us).
+// MFMAs).  Token blocks per workgroup: two above 16 tokens, unless that would
+// leave CUs idle: filling the CUs is worth more than reading each W row once (the
+// workgroups that share W rows sit at the same blockIdx.x, and since the row-tile
+// count is a multiple of 8 on the shapes this serves they land on the same XCD and
+// find the rows in its L2).
 int pick_token_blocks(long long row_groups, int N, int cu) {
-  int rb = N <= 16 ? 1 : N <= 32 ? 2 : N <= 48 ? 3 : 4;
-  if (rb > 1 && row_groups * ceil_div(N, 16 * rb) < cu) rb = (rb + 1) / 2;
-  return rb;
+  return N <= 16 || row_groups < cu ? 1 : 2;
 }
+
+template <bool SWIGLU, bool F32>
+int dense_tile(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M, int N, int K, int cu,
+               hipStream_t stream, const char* name);
 
 // Shared checks and launch.  rows = W rows read (M, or 2 I for SwiGLU),
 // M = output features per token row of Y.
@@ -272,19 +269,22 @@ int dense_launch(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M,
                 K);
   const int cu = current_cu_count();
   if (cu <= 0) return fail(kInvalidValue, "%s: no device", name);
+  if (ceil_div(N, 64) > 65535)
+    return fail(kNotSupported, "%s: too many token blocks (N=%d)", name, N);
+  // More than 32 tokens: the LDS-tiled kernel below.  From 5 tokens too where its 32-feature
+  // tiles give the CUs a workgroup each (7168 x 2048, 16 / 32 tokens: 7.5 / 7.6 us against
+  // 8.8 / 9.5 for the kernel above; 4096 rows, 128 workgroups: 20.6 / 21.1 against 21.4 /
+  // 19.8 us).
+  if (N > 32 || (N > 4 && ceil_div(rows, 32) >= cu * 3 / 4))
+    return dense_tile<SWIGLU, F32>(W, X, Y, rows, M, N, K, cu, stream, name);
   const int mr = SWIGLU ? 2 : (M % 32 == 0 ? 2 : 1);
   const int gx = SWIGLU ? M / 16 : M / (16 * mr);
   const int rb = pick_token_blocks(gx, N, cu);
-  const int ny = ceil_div(N, 16 * rb);
-  if (ny > 65535) return fail(kNotSupported, "%s: too many token blocks (N=%d)", name, N);
-  const dim3 grid(gx, ny);
+  const dim3 grid(gx, ceil_div(N, 16 * rb));
   const int stride = SWIGLU ? M : 16;
   // Few workgroups: more waves each, splitting K (at least one step a wave).
   // Once the grid has a workgroup per CU, fewer and longer K shares (at least
-  // 64 steps a wave) stream faster: Kimi's shared expert at 64 tokens, gate/up
-  // 7168 x 4096 with SwiGLU (256 workgroups) 20.4 / 19.5 / 19.0 / 17.9 us at
-  // 16 / 8 / 4 / 2 waves, down 2048 x 7168 (448 workgroups) 15.5 / 12.5 / 11.8 /
-  // 11.5 us at 8 / 4 / 2 / 1 (graph replays over 4 weight copies, one box).
+  // 64 steps a wave) stream faster.
   const long long wgs = static_cast<long long>(grid.x) * grid.y;
   int wk = wgs <= cu ? 16 : (wgs <= 2LL * cu ? 8 : 4);
   if (wgs >= cu)
@@ -298,6 +298,254 @@ int dense_launch(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M,
     default: launch_dense<1, SWIGLU, F32>(mr, rb, grid, W, X, Y, M, N, K, stride, stream); break;
   }
   return launch_status(name);
+}
+
+// ---------------------------------------------------------------- many tokens
+// The same GEMM for more tokens: a workgroup of eight waves owns
+// BM features x BN tokens and brings both operands straight from memory to a ring of
+// LDS stages of KC = 16 KS k.  The waves split each chunk's k into KS slices of 16
+// (and, with WM = 2, the features into halves), so that every byte of a stage is read
+// from LDS once or twice in all; each wave holds its slice's sums for the whole tile
+// (TM x TN 32x32 accumulators), and the slices are added through LDS in slice order at
+// the end.  A wave reads the next chunk's fragments while this chunk's MFMAs run; one
+// barrier per chunk.
+//
+// Kimi's shared expert (gate/up with SwiGLU 4096 x 7168, down 7168 x 2048) at 64 / 100 / 160 /
+// 250 tokens: gate/up 21.3 / 21.6 / 27.5 / 31.2 us, down 8.4 / 10.2 / 16.7 / 18.7 us, against
+// 22.6 / 29.9 / 44.6 / 55.9 and 12.1 / 17.0 / 21.6 / 30.7 us with the streaming kernel above,
+// whose fragments cross lanes through ds_bpermute; the router's logits (384 x 7168, fp32) at
+// 1000 / 4096 tokens 24.6 / 60.3 against 40.4 / 90.3 us.
+//
+// A row's 16-byte pieces are stored at slot piece ^ (row % pieces), which spreads the
+// fragment reads (32 rows, one piece) over the banks.  Bound by what a CU can bring in
+// from L2 (64 bytes a cycle) at few tokens, by the matrix pipe and LDS at many.
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16_t;
+
+template <int WM_, int TM_, int TN_, int KS_, int NS_>
+struct TileShape {
+  static constexpr int WM = WM_, TM = TM_, TN = TN_, KS = KS_, NS = NS_;
+  static constexpr int KC = 16 * KS, kRowBytes = 2 * KC, kPieces = kRowBytes / 16;
+  static constexpr int BM = 32 * WM * TM, BN = 32 * TN;
+  static constexpr int kStage = (BM + BN) * kRowBytes;
+  static constexpr int kRowsPerLoad = 1024 / kRowBytes;
+  static constexpr int P = (BM + BN) / kRowsPerLoad / 8;  // loads per wave and chunk
+  // token blocks whose partial sums fit LDS at once, and their bytes
+  static constexpr int TNR = KS * 32 * TN * (BM + 8) * 4 <= 160 * 1024 ? TN : TN / 2;
+  static constexpr int kRed = KS * 32 * TNR * (BM + 8) * 4;
+  static constexpr int kLds = NS * kStage > kRed ? NS * kStage : kRed;
+  static_assert(WM * KS == 8 && P * 8 * kRowsPerLoad == BM + BN && TN % TNR == 0, "tile shape");
+  static_assert(kLds <= 160 * 1024 && NS >= 3 && (kPieces & (kPieces - 1)) == 0, "tile shape");
+};
+
+// wide: Y is aligned to four of its elements.  M: output features of a token row of Y
+// (inter with SWIGLU, whose W has 2 M rows: the tile's first half holds gate features, its
+// second half the matching up features).
+template <typename S, bool SWIGLU, bool F32>
+__global__ __launch_bounds__(512, 2) void dense_tile_kernel(const uint16_t* __restrict__ W,
+                                                            const uint16_t* __restrict__ X,
+                                                            void* __restrict__ Yv, int M, int N,
+                                                            int K, bool wide) {
+  constexpr int BM = S::BM, BN = S::BN, NS = S::NS, P = S::P, TM = S::TM, TN = S::TN;
+  constexpr int BMO = SWIGLU ? BM / 2 : BM;  // output features of the tile
+  __shared__ __align__(1024) uint8_t smem[S::kLds];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / S::KS, ks = wave % S::KS;
+  const int c = lane & 31, h = lane >> 5;
+  const int m0 = blockIdx.x * BMO, n0 = blockIdx.y * BN;
+  const int chunks = ceil_div(K, S::KC);
+  const uint32_t row_bytes = static_cast<uint32_t>(K) * 2u;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+      (__attribute__((address_space(3))) uint8_t*)smem));
+
+  // This wave's loads of a chunk: each brings kRowsPerLoad rows of the stage, all gate, up
+  // or token rows.  Rows past the last feature or token are out of their resource's range.
+  u32x4_t rsrc[P];
+  uint32_t dst[P], voff[P];
+  int piece_k[P];  // the first k of this lane's piece within a chunk
+#pragma unroll
+  for (int j = 0; j < P; ++j) {
+    const int r0 = (wave * P + j) * S::kRowsPerLoad;
+    const bool token = r0 >= BM, up = SWIGLU && !token && r0 >= BMO;
+    const int part0 = token ? BM : up ? BMO : 0;  // the part's first row of the stage
+    const long long first = token ? n0 : up ? M + m0 : m0;
+    const int rows = token ? min(BN, N - n0) : min(BMO, M - m0);
+    rsrc[j] = rsrc_words((token ? X : W) + first * K,
+                         static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
+                             rows * static_cast<int>(row_bytes))));
+    const int r = r0 + lane / S::kPieces;
+    const int piece = (lane % S::kPieces) ^ (r % S::kPieces);
+    dst[j] = lds0 + static_cast<uint32_t>(r0 * S::kRowBytes);
+    voff[j] = static_cast<uint32_t>(r - part0) * row_bytes + 16u * piece;
+    piece_k[j] = 8 * piece;
+  }
+  auto stage_in = [&](int ch, int st) {
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+      // pieces past K (the last chunk of a K that is not whole chunks) bring zeros
+      const uint32_t past = piece_k[j] + ch * S::KC < K ? 0u : kOutOfRange;
+      dma_b128(rsrc[j], dst[j] + static_cast<uint32_t>(st), voff[j] | past,
+               static_cast<uint32_t>(ch) * S::kRowBytes);
+    }
+  };
+  const int slot = 16 * ((2 * ks + h) ^ (c % S::kPieces));
+  const uint8_t* w_rd = smem + (wm * TM * 32 + c) * S::kRowBytes + slot;
+  const uint8_t* x_rd = smem + (BM + c) * S::kRowBytes + slot;
+  struct Frags {
+    bf16x8_t w[TM], x[TN];
+  };
+  auto read = [&](Frags& f, int st) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      f.w[i] = *reinterpret_cast<const bf16x8_t*>(w_rd + st + 32 * S::kRowBytes * i);
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+      f.x[i] = *reinterpret_cast<const bf16x8_t*>(x_rd + st + 32 * S::kRowBytes * i);
+  };
+  floatx16_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = floatx16_t{};
+  auto products = [&](const Frags& f) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.x[j], f.w[i], acc[i][j], 0, 0, 0);
+  };
+
+#pragma unroll
+  for (int i = 0; i < NS - 1; ++i)
+    if (i < chunks) stage_in(i, i * S::kStage);
+  if (chunks >= NS - 1) vm_wait<(NS - 2) * P>(); else vm_wait<0>();
+  lds_barrier();
+  Frags f0, f1;
+  read(f0, 0);
+  // Step ch: chunk ch + 1 lands, chunk ch + NS - 1 goes into the stage of chunk ch - 1
+  // (every wave has its fragments of it, and this barrier follows its last read), the
+  // next fragments are read and this chunk's products run.
+  int st_rd = S::kStage, st_in = (NS - 1) * S::kStage;
+  auto next = [](int st) { return st + S::kStage == NS * S::kStage ? 0 : st + S::kStage; };
+  auto step = [&](const Frags& cur, Frags& nxt, int ch) {
+    if (ch + NS - 2 < chunks) vm_wait<(NS - 3) * P>(); else vm_wait<0>();
+    lds_barrier();
+    if (ch + NS - 1 < chunks) stage_in(ch + NS - 1, st_in);
+    read(nxt, st_rd);  // past the last chunk: a stage whose words are not used
+    st_in = next(st_in);
+    st_rd = next(st_rd);
+    products(cur);
+  };
+  for (int ch = 0; ch < chunks; ch += 2) {
+    step(f0, f1, ch);
+    if (ch + 1 < chunks) step(f1, f0, ch + 1);
+  }
+
+  // The KS slices' sums through LDS, TNR token blocks at a time, then four output
+  // features per thread, slices in order.
+  constexpr int kPitch = BM + 8;
+  float* red = reinterpret_cast<float*>(smem);
+#pragma unroll
+  for (int t0 = 0; t0 < TN; t0 += S::TNR) {
+    lds_barrier();  // the ring, or the previous blocks' sums, are read
+#pragma unroll
+    for (int j = 0; j < S::TNR; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          red[(ks * 32 * S::TNR + 32 * j + 8 * (e >> 2) + 4 * h + (e & 3)) * kPitch +
+              (wm * TM + i) * 32 + c] = acc[i][t0 + j][e];
+    __syncthreads();
+    for (int o = tid; o < 32 * S::TNR * (BMO / 4); o += 512) {
+      const int r = o / (BMO / 4), f = (o % (BMO / 4)) * 4;
+      const int n = n0 + 32 * t0 + r;
+      if (n >= N || m0 + f >= M) continue;
+      float g[4] = {0, 0, 0, 0}, u[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (int s = 0; s < S::KS; ++s) {
+        const float* src = red + (s * 32 * S::TNR + r) * kPitch + f;
+        const float4 v = *reinterpret_cast<const float4*>(src);
+        g[0] += v.x;
+        g[1] += v.y;
+        g[2] += v.z;
+        g[3] += v.w;
+        if constexpr (SWIGLU) {
+          const float4 w = *reinterpret_cast<const float4*>(src + BMO);
+          u[0] += w.x;
+          u[1] += w.y;
+          u[2] += w.z;
+          u[3] += w.w;
+        }
+      }
+      const long long at = static_cast<long long>(n) * M + m0 + f;
+      if constexpr (F32) {
+        float* y = static_cast<float*>(Yv) + at;
+        if (wide) {
+          *reinterpret_cast<float4*>(y) = make_float4(g[0], g[1], g[2], g[3]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[e] = g[e];
+        }
+      } else {
+        uint16_t* y = static_cast<uint16_t*>(Yv) + at;
+        uint16_t b[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          b[e] = SWIGLU ? swiglu_one(bf2f(f2bf(g[e])), bf2f(f2bf(u[e]))) : f2bf(g[e]);
+        if (wide) {
+          *reinterpret_cast<uint2*>(y) = make_uint2(b[0] | (static_cast<uint32_t>(b[1]) << 16),
+                                                    b[2] | (static_cast<uint32_t>(b[3]) << 16));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[e] = b[e];
+        }
+      }
+    }
+  }
+}
+
+template <typename S, bool SWIGLU, bool F32>
+int launch_tile(const uint16_t* W, const uint16_t* X, void* Y, int M, int N, int K,
+                hipStream_t stream, const char* name) {
+  const dim3 grid(ceil_div(M, SWIGLU ? S::BM / 2 : S::BM), ceil_div(N, S::BN));
+  // four outputs of a row per store where Y's alignment allows it
+  const bool wide = (reinterpret_cast<uintptr_t>(Y) & (F32 ? 15u : 7u)) == 0;
+  hipLaunchKernelGGL((dense_tile_kernel<S, SWIGLU, F32>), grid, dim3(512), 0, stream, W, X, Y, M, N,
+                     K, wide);
+  return launch_status(name);
+}
+
+// The tile shape whose slowest CU brings in the fewest bytes: a CU's workgroups times the
+// rows of a stage, since all of these shapes read their operands at about the same rate
+// (15-17 TB/s over the GPU: what bounds them).  On a tie the larger tile.  At 4096 weight
+// rows of 7168 (with SwiGLU) 32 x 32 / 32 x 64 / 32 x 96 / 64 x 64 take 21.2 / 23.3 / 26.1 /
+// 31.1 us at 64 tokens, 26.1 / 21.6 / 26.1 / 28.6 at 100, 41.1 / 38.2 / 27.5 / 28.8 at 160,
+// 47.4 / 40.3 / 48.4 / 31.8 at 250.
+template <bool SWIGLU, bool F32>
+int dense_tile(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M, int N, int K, int cu,
+               hipStream_t stream, const char* name) {
+  // BM, BN in order of preference
+  constexpr int kShapes[6][2] = {{128, 128}, {64, 64}, {64, 32}, {32, 64}, {32, 96}, {32, 32}};
+  int pick = 0;
+  long long best = -1;
+  for (int i = 0; i < 6; ++i) {
+    const long long wgs = static_cast<long long>(ceil_div(rows, kShapes[i][0])) *
+                          ceil_div(N, kShapes[i][1]);
+    const long long cost = (wgs + cu - 1) / cu * (kShapes[i][0] + kShapes[i][1]);
+    if (best < 0 || cost < best) {
+      best = cost;
+      pick = i;
+    }
+  }
+  switch (pick) {
+    case 0: return launch_tile<TileShape<2, 2, 4, 4, 4>, SWIGLU, F32>(W, X, Y, M, N, K, stream, name);
+    case 1: return launch_tile<TileShape<1, 2, 2, 8, 4>, SWIGLU, F32>(W, X, Y, M, N, K, stream, name);
+    case 2: return launch_tile<TileShape<1, 2, 1, 8, 6>, SWIGLU, F32>(W, X, Y, M, N, K, stream, name);
+    case 3: return launch_tile<TileShape<1, 1, 2, 8, 6>, SWIGLU, F32>(W, X, Y, M, N, K, stream, name);
+    case 4: return launch_tile<TileShape<1, 1, 3, 8, 4>, SWIGLU, F32>(W, X, Y, M, N, K, stream, name);
+    default: return launch_tile<TileShape<1, 1, 1, 8, 4>, SWIGLU, F32>(W, X, Y, M, N, K, stream, name);
+  }
 }
 
 // ---------------------------------------------------------------- prefill sizes

@@ -92,7 +92,6 @@ __device__ __forceinline__ WordPairs dequant_word(uint32_t x, const ColScale& a,
 }
 
 __device__ __forceinline__ bf16x8_t as_bf16x8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
-  typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
   u32x4_t v = {a, b, c, d};
   return __builtin_bit_cast(bf16x8_t, v);
 }
@@ -159,7 +158,6 @@ __device__ __forceinline__ uint16_t epilogue_value(float acc, int sid, const Gem
 // per-iteration scalar offset, and hardware range checking (reads at or past
 // `bytes` return zero, which is how rows that are not routed here read zeros
 // without a branch).
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
 constexpr uint32_t kOutOfRange = 0x80000000u;  // voffset that fails every range check
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
@@ -871,34 +869,6 @@ constexpr int pf_ring_bytes(int R) { return R == 64 ? 53248 : 79872; }
 // Stages of the ring for a tile of RB routed row blocks: as many as fit, at most 4.
 constexpr int pf_stages(int RB, int R) {
   return pf_ring_bytes(R) / pf_stage_bytes(RB) < 4 ? pf_ring_bytes(R) / pf_stage_bytes(RB) : 4;
-}
-
-// Global memory straight to LDS: lane l's 16 (or 4) bytes at voff + soff go to
-// lds + 16 l (4 l).  In asm so that the compiler, which cannot tell the ring's
-// stages apart, does not drain every load in flight at each LDS read; the kernel
-// counts them itself (vm_wait) and no register is written.
-__device__ __forceinline__ void dma_b128(u32x4_t rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
-__device__ __forceinline__ void dma_b32(u32x4_t rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-               :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void vm_wait() {
-  asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
-}
-// Every wave's LDS reads have returned and its counted loads have landed.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-__device__ __forceinline__ u32x4_t rsrc_words(const void* base, uint32_t bytes) {
-  const uint64_t a = reinterpret_cast<uint64_t>(base);
-  u32x4_t r = {static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a))),
-               static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a >> 32))) & 0xffffu,
-               bytes, 0x00020000u};
-  return r;
 }
 
 // One group's four B fragments (x1, x2, y1, y2), filled word by word: word jj holds

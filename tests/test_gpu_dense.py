@@ -282,3 +282,60 @@ def test_kimi_shared_expert_prefill_path(oracle):
         graph.replay()
         torch.cuda.synchronize()
         assert np.array_equal(host(out), got)
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 33, 32), (48, 64, 96), (80, 65, 160), (112, 97, 224),
+                                   (208, 129, 2080), (4096, 65, 512), (4096, 100, 96),
+                                   (4096, 200, 352), (4096, 255, 64), (7168, 100, 160),
+                                   (7168, 5, 160), (8192, 255, 288)])
+def test_dense_tile_shapes_exact(oracle, M, N, K):
+    """The LDS-tiled kernel's tile shapes (the shapes pick each of them) at ragged features,
+    tokens and k chunks, with Y aligned to its stores and two bytes off; exact operands, so
+    every summation order gives the fp32 product's bits."""
+    from pegainfer_amd import _lib
+    g = np.random.default_rng(M + N + K)
+    w = oracle.f32_to_bf16(np.ldexp(g.integers(-8, 8, (M, K)), g.integers(-4, 0, (M, K)))
+                           .astype(np.float32))
+    x = oracle.f32_to_bf16(g.integers(-3, 4, (N, K)).astype(np.float32))
+    ref = oracle.f32_to_bf16(oracle.bf16_to_f32(x) @ oracle.bf16_to_f32(w).T)
+    wd, xd = dev(w), dev(x)
+    for off in (0, 1):
+        y = torch.full((N * M + 2,), 7.0, dtype=torch.bfloat16, device="cuda")
+        _lib.call("gemm_graphsafe_cuda", wd.data_ptr(), xd.data_ptr(), y.data_ptr() + 2 * off, M, N,
+                  K, torch.cuda.current_stream().cuda_stream)
+        got = host(y)
+        assert np.array_equal(got[off:off + N * M].reshape(N, M), ref), off
+        assert (got[:off] == 0x40E0).all() and (got[off + N * M:] == 0x40E0).all()
+
+
+@pytest.mark.parametrize("I,N,K", [(16, 33, 32), (48, 100, 160), (80, 129, 96), (2048, 70, 352),
+                                   (2048, 255, 96), (2064, 160, 64)])
+def test_dense_tile_swiglu_equals_gemm_then_swiglu(oracle, I, N, K):
+    """Gate and up features of one tile, ragged in both halves: the bits of the two calls."""
+    from pegainfer_amd import ops
+    g = np.random.default_rng(I + N + K)
+    w = dev(oracle.f32_to_bf16((g.standard_normal((2 * I, K)) * 0.1).astype(np.float32)))
+    x = dev(oracle.f32_to_bf16(g.standard_normal((N, K)).astype(np.float32)))
+    fused = torch.full((N, I), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ops.dense_w13_swiglu(w, x, fused)
+    gu = torch.zeros(N, 2 * I, dtype=torch.bfloat16, device="cuda")
+    ops.gemm_graphsafe(w, x, gu)
+    chain = torch.zeros(N, I, dtype=torch.bfloat16, device="cuda")
+    ops.kimi_marlin_w13_swiglu(gu, chain, N, I)
+    assert np.array_equal(host(fused), host(chain))
+
+
+@pytest.mark.parametrize("N,K", [(33, 96), (100, 2080), (700, 160), (1500, 64), (4100, 32)])
+def test_dense_tile_router_logits_exact(oracle, N, K):
+    """The fp32 epilogue through the router entry point, on exact operands."""
+    from pegainfer_amd import ops
+    g = np.random.default_rng(N + K)
+    M = 384
+    w = oracle.f32_to_bf16(np.ldexp(g.integers(-8, 8, (M, K)), g.integers(-4, 0, (M, K)))
+                           .astype(np.float32))
+    x = oracle.f32_to_bf16(g.integers(-3, 4, (N, K)).astype(np.float32))
+    logits = torch.zeros(N, M, device="cuda")
+    tw = torch.zeros(N, 8, device="cuda")
+    ti = torch.zeros(N, 8, dtype=torch.int32, device="cuda")
+    ops.kimi_k2_router_noaux_tc(dev(x), dev(w), torch.zeros(M, device="cuda"), logits, tw, ti, N, N)
+    assert np.array_equal(host(logits), oracle.bf16_to_f32(x) @ oracle.bf16_to_f32(w).T)
