@@ -146,6 +146,10 @@ struct GemmArgs {
                     // instead of the bf16 output (finished by the consumer kernel)
   uint16_t* act;    // prefill, non-null: W13 + SwiGLU, act[sid][inter] instead of the output
   int inter;        // with act: gate columns [0, inter), up columns [inter, 2 inter)
+  // 16-row decode kernel at block size 8: pair the blocks of an expert
+  __host__ __device__ bool pair_blocks() const {
+    return bs == 8 && static_cast<long long>(size_m) * top_k >= 4LL * num_experts;
+  }
 };
 
 __device__ __forceinline__ uint16_t epilogue_value(float acc, int sid, const GemmArgs& p) {
@@ -433,6 +437,10 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 4) void wna16_decode_ker
 // instead of 2: 65.4 -> 64.0 us (three interleaved rounds, one box).  The swap's
 // output goes into the fragment with no per-lane select (both k halves find the
 // swapped bytes in the same registers): 121.9 -> 117.0 us and 64.6 -> 62.9 us.
+// Blocks of 8 rows run two to a workgroup where an expert has several, so that its
+// weights are dequantised once per 16 rows (512 rows in blocks of 8 over 48 experts, W13 /
+// W2: 267 / 165 -> 186 / 121 us); from four routes per expert on, since looking the run up
+// costs about half a microsecond (Kimi's decode layer at 3 tokens 80.4 -> 81.6 us).
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
 
 __device__ __forceinline__ floatx4_t mfma16(bf16x8_t a, bf16x8_t b, floatx4_t c) {
@@ -456,14 +464,34 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 6) void wna16_decode16_k
   const int n_tiles = p.size_n >> 6;
   const int n_units = kPair ? (p.inter >> 6) : n_tiles;
   const int split = blockIdx.x / n_units;
-  const int mb = blockIdx.y;
+  const int mb = blockIdx.y, m_blocks = gridDim.y;
   const int tid = threadIdx.x, lane = tid & 63;
   const int valid_limit = p.size_m * p.top_k;
   int sid = valid_limit;
-  if (tid < p.bs && mb * p.bs + tid < p.sorted_len) sid = p.sorted_ids[mb * p.bs + tid];
+  if (tid < 16 && mb * p.bs + tid < p.sorted_len) sid = p.sorted_ids[mb * p.bs + tid];
   const int expert = __builtin_amdgcn_readfirstlane(p.expert_ids[mb]);
+  // with paired blocks, the experts of this block and the 63 before it and of the next
+  const bool paired = p.pair_blocks();
+  const int before = paired ? p.expert_ids[max(mb - lane, 0)] : expert;
+  const int after = paired ? p.expert_ids[min(mb + 1, m_blocks - 1)] : -1;
   const int ntp = min(p.ntp[0], p.sorted_len);
   if (ntp < (mb + 1) * p.bs || expert < 0 || expert >= p.num_experts) return;
+  int rows = p.bs;
+  if (paired) {
+    // Two blocks of 8 rows of one expert share the MFMA's 16: in a run of blocks of one
+    // expert the even ones take the next block's rows along, the odd ones have been taken.
+    int run = 0;  // blocks of this expert up to this one
+    for (int first = mb;; first -= 64) {
+      const int e = first == mb ? before : p.expert_ids[max(first - lane, 0)];
+      const uint64_t same = __ballot(first - lane >= 0 && e == expert);
+      const int n = same == ~0ull ? 64 : __builtin_ctzll(~same);
+      run += n;
+      if (n < 64) break;
+    }
+    if ((run - 1) & 1) return;
+    if (mb + 1 < m_blocks && ntp >= (mb + 2) * 8 && after == expert) rows = 16;
+  }
+  if (tid >= rows) sid = valid_limit;
 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kw = wave % WK;
@@ -596,7 +624,7 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 6) void wna16_decode16_k
       }
       const int row = 4 * kb + (e & 3);
       const int col = colb + 8 * (e >> 2);
-      if (row < p.bs) {
+      if (row < rows) {
         const int rsid = s_sid[row];
         if (static_cast<unsigned>(rsid) < static_cast<unsigned>(valid_limit))
           p.act[static_cast<long long>(rsid) * p.inter + col] =
@@ -612,7 +640,7 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 6) void wna16_decode16_k
     for (int w = 0; w < WK; ++w) s += s_red[w][e][lane];
     const int row = 4 * kb + (e & 3);
     const int n = colb + 8 * (e >> 2);
-    if (row < p.bs) {
+    if (row < rows) {
       const int rsid = s_sid[row];
       if (static_cast<unsigned>(rsid) < static_cast<unsigned>(valid_limit)) {
         if (p.partial)

@@ -565,3 +565,40 @@ def test_tile_kernel_rows_and_chunks_exact(oracle, R_rows, K):
         got, ref = _run(oracle, E=E, N=N, K=K, T=T, topk=1, bs=bs, mul=False, a_bits=a_bits, q=q,
                         scale_bits=scale_bits, idx=idx, tw=np.ones((T, 1), np.float32))
         assert np.array_equal(got, ref)
+
+
+def test_decode_merges_blocks_of_eight_rows(oracle):
+    """Blocks of 8 rows, two to a workgroup within an expert's run of blocks: runs of 1 to 140
+    blocks (longer than the 64 looked back at once), odd and even, one expert in two runs, -1
+    blocks between, a last block whose partner lies past the routed total.  Exact inputs;
+    rows of -1 blocks and past the total keep their contents."""
+    from pegainfer_amd import _lib
+    g = np.random.default_rng(21)
+    E, N, K, bs = 6, 4096, 128, 8
+    runs = [(3, 1), (1, 2), (0, 3), (-1, 2), (0, 5), (2, 140), (1, 4), (-1, 1), (5, 67), (4, 2)]
+    expert_ids = np.concatenate([[e] * n for e, n in runs]).astype(np.int32)
+    blocks = len(expert_ids)
+    T = blocks * bs
+    sorted_ids = g.permutation(T).astype(np.int32)
+    pad = g.random(T) < 0.1  # padding anywhere in a block
+    sorted_ids = np.where(pad, T, sorted_ids).astype(np.int32)
+    ntp = (blocks - 1) * bs  # the last block lies past the total
+    q = g.integers(-8, 8, size=(E, N, K))
+    scale_bits = oracle.f32_to_bf16(
+        (2.0 ** g.integers(-6, -2, size=(E, N, K // 32))).astype(np.float32))
+    a_bits = oracle.f32_to_bf16(g.integers(-2, 3, size=(T, K)).astype(np.float32))
+    w, packed = _setup(E, N, K, q, scale_bits)
+    out = torch.full((T, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    tw = np.ones((T, 1), np.float32)
+    sid, eid, nt, twd, a = (dev(sorted_ids), dev(expert_ids), dev(np.array([ntp], np.int32)),
+                            dev(tw.reshape(-1)), dev(a_bits))
+    _lib.call("pega_wna16_gemm", a.data_ptr(), out.data_ptr(), None, 0,
+              w.weight_packed_uint4b8.data_ptr(), w.weight_scale_permuted.data_ptr(), None, 0,
+              sid.data_ptr(), eid.data_ptr(), nt.data_ptr(), twd.data_ptr(), T, bs, 1, False, T, N,
+              K, E, 32, 0, torch.cuda.current_stream().cuda_stream)
+    ref = oracle.wna16_gemm(a_bits, packed, scale_bits,
+                            dict(sorted_token_ids=sorted_ids, expert_ids=expert_ids,
+                                 num_tokens_post_padded=np.array([ntp], np.int32)), tw,
+                            moe_block_size=bs, top_k=1, mul_topk_weights=False, size_m=T, size_n=N,
+                            size_k=K, output=np.full((T, N), 0x40E0, np.uint16), threads=8)
+    assert np.array_equal(host(out), ref)
