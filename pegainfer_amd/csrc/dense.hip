@@ -19,14 +19,12 @@
 // A permuted k order that reads 256 contiguous bytes per row per step instead
 // quadruples the lines per instruction and ran 2.3x slower.
 //
-// The first kernel below serves up to 32 tokens, where the GEMM is a weight stream:
-// one workgroup owns 16 MR output features for 16 RB tokens (the host picks
-// the shape); its WK waves split K and are reduced through LDS in wave order
-// (deterministic).  Per 32-k step a lane issues one 16-byte load of W per
-// 16-feature row tile and one of X per 16-token row block; after the lane
-// exchange, lane (c, q) holds feature m0 + 16 mr + c, k 8q..8q+7 (the B
-// fragment of a 16x16x32 MFMA) and the token blocks' A fragments, and one
-// v_mfma_f32_16x16x32_bf16 runs per (row tile, token block).  A and B take
+// The first kernel below serves few tokens, where the GEMM is a weight stream: one
+// workgroup owns 16 rows of W for 16 RB tokens; its WK waves split K and are reduced
+// through LDS in wave order (deterministic).  Per 32-k step a lane issues one 16-byte
+// load of W and one of X per 16-token block; after the lane exchange, lane (c, q) holds
+// row c of the tile, k 8q..8q+7 (the B fragment of a 16x16x32 MFMA) and the token blocks'
+// A fragments, and one v_mfma_f32_16x16x32_bf16 runs per token block.  A and B take
 // the same k slots per lane, so the product is exact whatever k order the
 // MFMA assigns to them.  Token rows past N read zeros through an
 // out-of-range buffer offset and are never stored.
@@ -63,49 +61,51 @@ __device__ __forceinline__ u32x4_t load16(__amdgpu_buffer_rsrc_t r, uint32_t vof
                                                kPolicy);
 }
 
-template <int MR, int RB>
+template <int RB>
 struct StepRegs {
-  u32x4_t w[MR];  // W[m0 + 16 mr + l / 4][k0 + 8 (l % 4) .. +7] (lane l)
+  u32x4_t w;      // row l / 4 of the tile, W[..][k0 + 8 (l % 4) .. +7] (lane l)
   u32x4_t x[RB];  // X[n0 + 16 rb + l / 4][k0 + 8 (l % 4) .. +7]
 };
 
-// One workgroup per (16 MR output features, 16 RB tokens); WK waves split the
-// K/32 steps; D steps per wave in flight.  Each X fragment feeds MR MFMAs and
-// each W fragment RB.  A wave's row tiles start tile_stride rows apart.
-// SWIGLU (MR = 2): tile 0 holds gate features m0..m0+15 and tile 1 the
-// matching up features (tile_stride = I); the epilogue rounds both sums to
-// bf16 as the GEMM's output would be, applies SwiGLU and writes act[n][m0+c]
-// (Y row stride M = I).  F32: Y is fp32 and takes the sums unrounded (the
+// One workgroup per (16 rows of W, 16 RB tokens); WK waves split the K/32 steps; D steps
+// per wave in flight.  SWIGLU: the tile holds gate features m0..m0+7 and the matching up
+// features (I rows further on), so a tile completes eight outputs by itself; the epilogue
+// rounds both sums to bf16 as the GEMM's output would be, applies SwiGLU and writes
+// act[n][m0+c] (Y row stride M = I).  F32: Y is fp32 and takes the sums unrounded (the
 // router's logits GEMM, cublasGemmEx with CUDA_R_32F output).
-template <int WK, int MR, int RB, bool SWIGLU, bool F32 = false>
+//
+// A stream of W with few bytes per CU: what counts is that every CU has a workgroup and
+// that the first loads are out early.  Kimi's shared expert, 3 tokens, gate/up (58.7 MB)
+// / down (29.4 MB): 17.2 / 7.5 us with 16 waves on 32-row tiles (128 and 224 workgroups,
+// half the CUs idle in the first), 16.7 / 6.7 with eight waves on them, 12.4 / 6.7 with
+// eight and 11.8 / 6.0 us with four waves on 16-row ones (5.0 and 4.9 TB/s).  Two waves:
+// 15.9 / 6.0; eight steps in flight instead of four: 11.9 / 6.3.
+template <int WK, int RB, bool SWIGLU, bool F32>
 __global__ __launch_bounds__(64 * WK) void dense_gemm_kernel(const uint16_t* __restrict__ W,
                                                              const uint16_t* __restrict__ X,
                                                              void* __restrict__ Yv, int M,
-                                                             int N, int K, int tile_stride) {
-  static_assert(!SWIGLU || MR == 2, "SwiGLU pairs one gate and one up tile");
+                                                             int N, int K) {
   static_assert(!(SWIGLU && F32), "the SwiGLU epilogue writes bf16");
-  uint16_t* __restrict__ Y = static_cast<uint16_t*>(Yv);
-  constexpr int D = 4;  // the ring fits 128 VGPRs at WK = 16
+  constexpr int D = 4;
   __shared__ float s_red[WK][RB * 4][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, q = lane >> 4;
-  const int m0 = blockIdx.x * (SWIGLU ? 16 : 16 * MR);
+  const int m0 = blockIdx.x * (SWIGLU ? 8 : 16);
   const int n0 = blockIdx.y * (16 * RB);
   const int steps = K >> 5;
   const int s0 = (steps * wave) / WK, s1 = (steps * (wave + 1)) / WK;
 
-  const __amdgpu_buffer_rsrc_t wr = make_rsrc(
-      W + static_cast<long long>(m0) * K,
-      (static_cast<uint32_t>(tile_stride) * (MR - 1) + 16u) * static_cast<uint32_t>(K) * 2u);
+  const uint32_t span = SWIGLU ? static_cast<uint32_t>(M) + 8u : 16u;
+  const __amdgpu_buffer_rsrc_t wr =
+      make_rsrc(W + static_cast<long long>(m0) * K, span * static_cast<uint32_t>(K) * 2u);
   // Loads run along k: lane l fetches row l / 4, k 8 (l % 4) .. +7, so four
   // neighbouring lanes read 64 contiguous bytes of one row (one line request
   // per lane quad, 16 per load); ds_bpermute then hands lane (c, q) the
   // 16 bytes of row c, k 8q .. +7 that its fragment needs, from lane 4c + q.
   const uint32_t lr = static_cast<uint32_t>(lane >> 2), lp = static_cast<uint32_t>(lane & 3);
-  uint32_t w_voff[MR];
-#pragma unroll
-  for (int mr = 0; mr < MR; ++mr) w_voff[mr] = ((static_cast<uint32_t>(tile_stride) * mr + lr) * K + 8u * lp) * 2u;
+  const uint32_t w_row = SWIGLU ? (lr & 7u) + (lr >> 3) * static_cast<uint32_t>(M) : lr;
+  const uint32_t w_voff = (w_row * static_cast<uint32_t>(K) + 8u * lp) * 2u;
   const int src_lane_bytes = (4 * c + q) * 4;
   const __amdgpu_buffer_rsrc_t xr =
       make_rsrc(X, static_cast<uint32_t>(N) * static_cast<uint32_t>(K) * 2u);
@@ -124,33 +124,27 @@ __global__ __launch_bounds__(64 * WK) void dense_gemm_kernel(const uint16_t* __r
     return __builtin_bit_cast(bf16x8_t, f);
   };
 
-  auto load_step = [&](StepRegs<MR, RB>& r, int s) {
+  auto load_step = [&](StepRegs<RB>& r, int s) {
     s = min(max(s, 0), steps - 1);  // every scalar offset stays inside the rows
     const uint32_t soff = static_cast<uint32_t>(s) * 64u;
-#pragma unroll
-    for (int mr = 0; mr < MR; ++mr) r.w[mr] = load16<kCached>(wr, w_voff[mr], soff);
+    r.w = load16<kCached>(wr, w_voff, soff);
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) r.x[rb] = load16<kCached>(xr, x_voff[rb], soff);
   };
-  floatx4_t acc[MR][RB];
+  floatx4_t acc[RB];
 #pragma unroll
-  for (int mr = 0; mr < MR; ++mr)
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) acc[mr][rb] = floatx4_t{};
-  auto compute_step = [&](const StepRegs<MR, RB>& r) {
+  for (int rb = 0; rb < RB; ++rb) acc[rb] = floatx4_t{};
+  auto compute_step = [&](const StepRegs<RB>& r) {
     bf16x8_t a[RB];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) a[rb] = to_fragment(r.x[rb]);
+    const bf16x8_t b = to_fragment(r.w);
 #pragma unroll
-    for (int mr = 0; mr < MR; ++mr) {
-      const bf16x8_t b = to_fragment(r.w[mr]);
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
-        acc[mr][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rb], b, acc[mr][rb], 0, 0, 0);
-    }
+    for (int rb = 0; rb < RB; ++rb)
+      acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rb], b, acc[rb], 0, 0, 0);
   };
 
-  StepRegs<MR, RB> slot[D];
+  StepRegs<RB> slot[D];
 #pragma unroll
   for (int j = 0; j < D; ++j) {
     load_step(slot[j], s0 + j < s1 ? s0 + j : s1 - 1);
@@ -173,73 +167,41 @@ __global__ __launch_bounds__(64 * WK) void dense_gemm_kernel(const uint16_t* __r
   for (int j = 0; j < D - 1; ++j)
     if (s + j < s1) compute_step(slot[j]);
 
-  // Reduction over the WK waves in wave order, one row tile at a time.
-  // Accumulator element e of (mr, rb) holds token n0 + 16 rb + 4 q + e,
-  // feature m0 + tile_stride mr + c.  Every tile gives a lane the same j
-  // values, so a SwiGLU lane keeps its gate sums in gsum for the up pass.
-  constexpr int kJ = (RB * 4 + WK - 1) / WK;
-  float gsum[kJ];
+  // Reduction over the WK waves in wave order.  Accumulator element e of block rb holds
+  // token n0 + 16 rb + 4 q + e, tile row c.
 #pragma unroll
-  for (int mr = 0; mr < MR; ++mr) {
-    if (mr > 0) __syncthreads();  // the previous tile's sums are read
+  for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
+    for (int e = 0; e < 4; ++e) s_red[wave][rb * 4 + e][lane] = acc[rb][e];
+  __syncthreads();
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s_red[wave][rb * 4 + e][lane] = acc[mr][rb][e];
-    __syncthreads();
+  for (int j = wave; j < RB * 4; j += WK) {
+    float sum = 0.0f;
 #pragma unroll
-    for (int i = 0; i < kJ; ++i) {
-      const int j = wave + i * WK;
-      if (j >= RB * 4) break;
-      float sum = 0.0f;
-#pragma unroll
-      for (int w = 0; w < WK; ++w) sum += s_red[w][j][lane];
-      const int n = n0 + 16 * (j >> 2) + 4 * q + (j & 3);
-      if constexpr (SWIGLU) {
-        if (mr == 0) {
-          gsum[i] = sum;
-        } else if (n < N) {
-          Y[static_cast<long long>(n) * M + m0 + c] =
-              swiglu_one(bf2f(f2bf(gsum[i])), bf2f(f2bf(sum)));
-        }
-      } else if (n < N) {
-        const long long o = static_cast<long long>(n) * M + m0 + 16 * mr + c;
-        if constexpr (F32)
-          static_cast<float*>(Yv)[o] = sum;
-        else
-          Y[o] = f2bf(sum);
-      }
+    for (int w = 0; w < WK; ++w) sum += s_red[w][j][lane];
+    const int n = n0 + 16 * (j >> 2) + 4 * q + (j & 3);
+    const long long o = static_cast<long long>(n) * M + m0 + c;
+    if constexpr (SWIGLU) {
+      const float up = __shfl_xor(sum, 8);  // tile rows 8..15
+      if (n < N && c < 8)
+        static_cast<uint16_t*>(Yv)[o] = swiglu_one(bf2f(f2bf(sum)), bf2f(f2bf(up)));
+    } else if (n < N) {
+      if constexpr (F32)
+        static_cast<float*>(Yv)[o] = sum;
+      else
+        static_cast<uint16_t*>(Yv)[o] = f2bf(sum);
     }
   }
 }
 
-template <int WK, int MR, bool SWIGLU, bool F32>
-void launch_dense_rb(int rb, dim3 grid, const uint16_t* W, const uint16_t* X, void* Y, int M,
-                     int N, int K, int stride, hipStream_t stream) {
-  const dim3 block(64 * WK);
-  if (rb == 1)
-    hipLaunchKernelGGL((dense_gemm_kernel<WK, MR, 1, SWIGLU, F32>), grid, block, 0, stream, W, X, Y, M, N, K, stride);
-  else
-    hipLaunchKernelGGL((dense_gemm_kernel<WK, MR, 2, SWIGLU, F32>), grid, block, 0, stream, W, X, Y, M, N, K, stride);
-}
-
 template <int WK, bool SWIGLU, bool F32>
-void launch_dense(int mr, int rb, dim3 grid, const uint16_t* W, const uint16_t* X, void* Y,
-                  int M, int N, int K, int stride, hipStream_t stream) {
-  if (SWIGLU || mr == 2)
-    launch_dense_rb<WK, 2, SWIGLU, F32>(rb, grid, W, X, Y, M, N, K, stride, stream);
+void launch_dense(int rb, int row_tiles, const uint16_t* W, const uint16_t* X, void* Y, int M,
+                  int N, int K, hipStream_t stream) {
+  const dim3 grid(row_tiles, ceil_div(N, 16 * rb)), block(64 * WK);
+  if (rb == 1)
+    hipLaunchKernelGGL((dense_gemm_kernel<WK, 1, SWIGLU, F32>), grid, block, 0, stream, W, X, Y, M, N, K);
   else
-    launch_dense_rb<WK, 1, false, F32>(rb, grid, W, X, Y, M, N, K, stride, stream);
-}
-
-// Row tiles per wave: two where M allows (each X fragment then feeds two
-// MFMAs).  Token blocks per workgroup: two above 16 tokens, unless that would
-// leave CUs idle: filling the CUs is worth more than reading each W row once (the
-// workgroups that share W rows sit at the same blockIdx.x, and since the row-tile
-// count is a multiple of 8 on the shapes this serves they land on the same XCD and
-// find the rows in its L2).
-int pick_token_blocks(long long row_groups, int N, int cu) {
-  return N <= 16 || row_groups < cu ? 1 : 2;
+    hipLaunchKernelGGL((dense_gemm_kernel<WK, 2, SWIGLU, F32>), grid, block, 0, stream, W, X, Y, M, N, K);
 }
 
 template <bool SWIGLU, bool F32>
@@ -271,32 +233,28 @@ int dense_launch(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M,
   if (cu <= 0) return fail(kInvalidValue, "%s: no device", name);
   if (ceil_div(N, 64) > 65535)
     return fail(kNotSupported, "%s: too many token blocks (N=%d)", name, N);
-  // More than 32 tokens: the LDS-tiled kernel below.  From 5 tokens too where its 32-feature
-  // tiles give the CUs a workgroup each (7168 x 2048, 16 / 32 tokens: 7.5 / 7.6 us against
-  // 8.8 / 9.5 for the kernel above; 4096 rows, 128 workgroups: 20.6 / 21.1 against 21.4 /
-  // 19.8 us).
-  if (N > 32 || (N > 4 && ceil_div(rows, 32) >= cu * 3 / 4))
+  // The streaming kernel while its workgroups fit one per CU, on the smaller token blocks
+  // if those do; a second workgroup per CU costs more than reading each fragment for two
+  // token blocks (2048 x 2816, 24 tokens, 256 workgroups of 16 or 128 of 32 tokens: 4.5 /
+  // 5.7 us; 64 tokens, 512 or 256: 7.3 / 6.0).  With more workgroups, the LDS-tiled kernel
+  // below from 33 tokens on, and from 17 where its own tiles give the CUs a workgroup each
+  // (us here / there: 7168 x 2048, 20 tokens 8.1 / 7.6, 32 tokens 9.5 / 7.7; 2048 x 2816, 96
+  // tokens 9.1 / 7.5; the router's logits, 384 x 7168 fp32, which stay here, at 33 / 128
+  // tokens 12.3 / 19.6 and 12.8 / 19.6).  Its tiles read X for 32 features at a time, not
+  // 16, which also counts for fewer tokens where the weights are many: from 32 MB at 9 to
+  // 16 tokens (5120 x 5120, 16 tokens 20.6 / 17.2; 16384 x 4096, 10 tokens 27.4 / 26.1;
+  // below, 7168 x 2048 10 tokens 6.7 / 7.4), from 256 MB at 5 to 8 (gate/up 36864 x 7168
+  // 116 / 106; below, 7168 x 18432 53 / 58).
+  const long long tiles = rows / 16, w_bytes = 2LL * rows * K;
+  const int rb = N <= 16 || tiles * ceil_div(N, 16) <= cu ? 1 : 2;
+  const bool many = N > 16 || (N > 8 && w_bytes >= (32LL << 20)) ||
+                    (N > 4 && w_bytes >= (256LL << 20));
+  if (tiles * ceil_div(N, 16 * rb) > cu && (N > 32 || (many && tiles >= cu * 5LL / 4)))
     return dense_tile<SWIGLU, F32>(W, X, Y, rows, M, N, K, cu, stream, name);
-  const int mr = SWIGLU ? 2 : (M % 32 == 0 ? 2 : 1);
-  const int gx = SWIGLU ? M / 16 : M / (16 * mr);
-  const int rb = pick_token_blocks(gx, N, cu);
-  const dim3 grid(gx, ceil_div(N, 16 * rb));
-  const int stride = SWIGLU ? M : 16;
-  // Few workgroups: more waves each, splitting K (at least one step a wave).
-  // Once the grid has a workgroup per CU, fewer and longer K shares (at least
-  // 64 steps a wave) stream faster.
-  const long long wgs = static_cast<long long>(grid.x) * grid.y;
-  int wk = wgs <= cu ? 16 : (wgs <= 2LL * cu ? 8 : 4);
-  if (wgs >= cu)
-    while (wk > 1 && K / 32 < 64 * wk) wk >>= 1;
-  while (wk > 1 && K / 32 < wk) wk >>= 1;
-  switch (wk) {
-    case 16: launch_dense<16, SWIGLU, F32>(mr, rb, grid, W, X, Y, M, N, K, stride, stream); break;
-    case 8: launch_dense<8, SWIGLU, F32>(mr, rb, grid, W, X, Y, M, N, K, stride, stream); break;
-    case 4: launch_dense<4, SWIGLU, F32>(mr, rb, grid, W, X, Y, M, N, K, stride, stream); break;
-    case 2: launch_dense<2, SWIGLU, F32>(mr, rb, grid, W, X, Y, M, N, K, stride, stream); break;
-    default: launch_dense<1, SWIGLU, F32>(mr, rb, grid, W, X, Y, M, N, K, stride, stream); break;
-  }
+  if (K >= 4 * 32)  // a step per wave at least
+    launch_dense<4, SWIGLU, F32>(rb, static_cast<int>(tiles), W, X, Y, M, N, K, stream);
+  else
+    launch_dense<1, SWIGLU, F32>(rb, static_cast<int>(tiles), W, X, Y, M, N, K, stream);
   return launch_status(name);
 }
 

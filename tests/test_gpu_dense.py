@@ -339,3 +339,28 @@ def test_dense_tile_router_logits_exact(oracle, N, K):
     ti = torch.zeros(N, 8, dtype=torch.int32, device="cuda")
     ops.kimi_k2_router_noaux_tc(dev(x), dev(w), torch.zeros(M, device="cuda"), logits, tw, ti, N, N)
     assert np.array_equal(host(logits), oracle.bf16_to_f32(x) @ oracle.bf16_to_f32(w).T)
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 1, 32), (16, 17, 96), (48, 16, 128), (48, 33, 160),
+                                   (384, 170, 2080), (2048, 32, 352), (2048, 33, 128),
+                                   (4096, 31, 160), (5120, 16, 160), (7168, 9, 2368)])
+def test_dense_stream_shapes_exact(oracle, M, N, K):
+    """The streaming kernel at its least K (one wave; four waves of a step), at token blocks of
+    16 and 32 with remainders, and on both sides of the line to the LDS-tiled kernel: plain
+    and SwiGLU, on exact operands (every summation order gives the fp32 product's bits)."""
+    from pegainfer_amd import ops
+    g = np.random.default_rng(M + N + K)
+    w = oracle.f32_to_bf16(np.ldexp(g.integers(-8, 8, (M, K)), g.integers(-4, 0, (M, K)))
+                           .astype(np.float32))
+    x = oracle.f32_to_bf16(g.integers(-3, 4, (N, K)).astype(np.float32))
+    wd, xd = dev(w), dev(x)
+    y = torch.full((N + 1, M), 7.0, dtype=torch.bfloat16, device="cuda")
+    ops.gemm_graphsafe(wd, xd, y[:N])
+    ref = oracle.f32_to_bf16(oracle.bf16_to_f32(x) @ oracle.bf16_to_f32(w).T)
+    assert np.array_equal(host(y[:N]), ref) and bool((y[N] == 7.0).all())
+    if M % 32 == 0:
+        fused = torch.full((N + 1, M // 2), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops.dense_w13_swiglu(wd, xd, fused[:N])
+        chain = torch.zeros(N, M // 2, dtype=torch.bfloat16, device="cuda")
+        ops.kimi_marlin_w13_swiglu(y[:N], chain, N, M // 2)
+        assert np.array_equal(host(fused[:N]), host(chain)) and bool((fused[N] == 7.0).all())
