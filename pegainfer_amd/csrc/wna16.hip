@@ -1430,6 +1430,21 @@ bool mean_rows_at_most(long long routes, long long experts, long long rows) {
   return routes <= rows * experts * (experts == 48 ? 8 : 1);
 }
 
+// Blocks that a decode launch is expected to find work for: at most one per route, and an
+// eighth of that on a 48-expert share.
+long long live_blocks(long long routes, long long experts, long long max_m_blocks) {
+  return std::min(experts == 48 ? (routes + 7) / 8 : routes, max_m_blocks);
+}
+
+// Waves that share a workgroup's K: four from a workgroup per CU on, more below that, where
+// the CUs have no other work to hide a wave's latency behind.  Kimi W2 with one live block
+// (112 workgroups) in a decode layer at one token: 16 / 8 / 4 waves 55 / 51.7 / 53 us, with
+// three (336) 75 / 69.4 / 69.5 at 3 tokens; 28672 x 4096, one row (448) 19.4 / 16.1 / 16.1
+// us; 2560 x 9728, one row (40) 16.0 / 16.8 / 20.8.
+int decode_waves(long long wgs, int cu_count) {
+  return wgs >= cu_count ? 4 : (wgs >= cu_count * 3LL / 8 ? 8 : 16);
+}
+
 // Prefill tile height: 64 rows (three workgroups a CU instead of two) when the
 // routes come to few rows per expert, else 128.  Few rows per expert leave the
 // 128-row tiles mostly one or two 32-row blocks anyway, while a problem's large
@@ -1521,9 +1536,9 @@ int wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long long 
     // more waves per workgroup splitting K, so the chip stays busy.
     const int groups = size_k / 32;
     const long long routes = static_cast<long long>(size_m) * top_k;
-    const long long est_blocks = routes < max_m_blocks ? routes : max_m_blocks;
+    const long long est_blocks = live_blocks(routes, local_experts, max_m_blocks);
     const long long wgs = est_blocks * n_tiles;
-    int wk = wgs >= 4LL * cu_count ? 4 : (wgs >= 2LL * cu_count ? 8 : 16);
+    int wk = decode_waves(wgs, cu_count);
     while (wk > 4 && groups < wk) wk >>= 1;  // waves past the last group idle
     if (max_m_blocks > 65535) return fail(kNotSupported, "wna16_gemm: too many m-blocks");
     if (wk == 4) launch_decode<4>(args, max_m_blocks, stream);
@@ -1614,12 +1629,17 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
   const long long routes = static_cast<long long>(size_m) * top_k;
   const int n_tiles = size_n / 64;
   const int groups = size_k / 32;
-  const long long est_blocks = routes < max_m_blocks ? routes : max_m_blocks;
+  const long long est_blocks = live_blocks(routes, local_experts, max_m_blocks);
   const long long wgs = est_blocks * n_tiles;
-  // shares: about two workgroups per CU, at least 8 groups (two per wave) each,
-  // as many as the partials buffer holds
-  long long sp = (2LL * cu_count + wgs - 1) / wgs;
-  if (sp > 16) sp = 16;
+  // Shares: about two workgroups per CU, at least 8 groups (two per wave) each, as many as
+  // the partials buffer holds.  On a 48-expert share four per CU, since the routes that fall
+  // on it vary, and at most four shares, since most workgroups of its grid find no block
+  // and each share dispatches them again (decode layer at 1 / 3 / 12 tokens: one share 62.5
+  // / 69.5 / 98 us, two 55.7 / 62.4 / 96, four 53 / 59.5 / 95, eight 57 / 65 / -).
+  const bool share48 = local_experts == 48;
+  const long long aim = (share48 ? 4LL : 2LL) * cu_count;
+  long long sp = (aim + wgs - 1) / wgs;
+  if (sp > (share48 ? 4 : 16)) sp = share48 ? 4 : 16;
   if (sp > groups / 8) sp = groups / 8;
   const long long cap = partials ? partials_len / (routes * size_n) : 0;
   if (sp > cap) sp = cap;
@@ -1643,7 +1663,7 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
                 sorted_token_ids_len, moe_block_size, top_k, 0, size_m, size_n, size_k,
                 local_experts, splits, partials};
   const long long total_wgs = wgs * splits;
-  int wk = total_wgs >= 4LL * cu_count ? 4 : (total_wgs >= 2LL * cu_count ? 8 : 16);
+  int wk = decode_waves(total_wgs, cu_count);
   while (wk > 4 && groups / splits < 2 * wk) wk >>= 1;  // keep >= 2 groups per wave
   if (wk == 4) launch_decode<4>(args, max_m_blocks, stream);
   else if (wk == 8) launch_decode<8>(args, max_m_blocks, stream);
