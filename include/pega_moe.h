@@ -129,10 +129,12 @@ int pega_wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long 
  * route row; here act = [size_m * top_k, intermediate_dim] bf16 gets SwiGLU of the W13 sums
  * rounded to bf16 as the W13 output is, for the routed rows only (other rows are left as they
  * are), and the W13 output never reaches HBM.  The bits are the pair's whenever both add the
- * fp32 products over the same K shares: always at block sizes 32-64 (one wave covers all of
- * K), and at block sizes 8/16 when the W13 GEMM has at least two workgroups per CU and K is at
- * least 512 (C3's decode layer, for one).  Otherwise the shares differ (the K split below, or
- * 8 waves where the GEMM runs 16), and the sums may differ from the pair's in the last fp32
+ * fp32 products over the same K shares: always at block sizes 32-64 (both take the same form
+ * and the same split of K), and at block sizes 8/16 when the launch expects at least two (block,
+ * 64-column tile) units per CU, or four on a 48-expert share, and K is at least 512 (the Kimi
+ * decode layer from 16 tokens on, for one).  A launch expects one block per route, and one per
+ * eight routes on a 48-expert share.  Otherwise the shares differ (the K split below, or 8
+ * waves where the GEMM runs 16), and the sums may differ from the pair's in the last fp32
  * bit, within the same summation error bound.
  *  - Block size 8 or 16 (decode): when the (block, tile) units are too few to fill the GPU
  *    (one expert at batch 1-8), K is split across workgroups; the fp32 partials (partials:
@@ -142,9 +144,9 @@ int pega_wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long 
  *    to split) a workgroup takes a gate tile and its up tile and applies SwiGLU in its
  *    epilogue.
  *  - Block size 32, 48 or 64 (prefill): the tile GEMM (128-row tiles, or 64-row tiles when
- *    the routes fill at most 64 rows per expert on average) takes each gate tile and its up
- *    tile in one workgroup and applies SwiGLU in its epilogue; partials is not used (may be
- *    NULL, partials_len 0). */
+ *    the routes are few per expert), or where they are fewer still a 32-row form of the decode
+ *    kernel, takes each gate tile and its up tile in one workgroup and applies SwiGLU in its
+ *    epilogue; partials is not used (may be NULL, partials_len 0). */
 int pega_wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials,
                           long long partials_len, const uint8_t* b_qweight,
                           const uint16_t* b_scales, const int32_t* sorted_token_ids,
@@ -199,7 +201,8 @@ typedef struct pega_wna16_problem {
 /* No reference counterpart: two independent prefill-size GEMMs in one launch, e.g. a layer's
  * shared expert (first) and its routed experts (second).  The workgroups of the first problem
  * are dispatched first, and the second problem's fill the rest of the GPU, so one stream keeps
- * both running at once; each problem's output has the bits its own single launch gives.
+ * both running at once; each problem's output has the bits its own single launch gives.  When
+ * a problem has too few routed rows for the tile kernel, each gets its own launch instead.
  * Returns 801 when a problem's block size is 8 or 16 (the decode kernels). */
 int pega_wna16_prefill_pair(const pega_wna16_problem* first, const pega_wna16_problem* second,
                             hipStream_t stream);

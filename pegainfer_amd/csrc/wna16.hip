@@ -1651,7 +1651,10 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
                   nullptr, sorted_token_ids_len, moe_block_size, top_k, 0, size_m, size_n,
                   size_k, local_experts, 1, nullptr, act, inter};
     const long long pair_wgs = est_blocks * (inter / 64);
-    int wk = pair_wgs >= 2LL * cu_count ? 4 : 8;
+    // As the plain GEMM's from two units per CU on, so that the two give the same bits there
+    // (DeepSeek-V2-Lite block at 3 / 8 tokens: 61.2 / 81.6 us with four waves, 63.9 / 81.9
+    // with eight).
+    int wk = pair_wgs >= cu_count ? 4 : 8;
     while (wk > 4 && groups < 2 * wk) wk >>= 1;  // keep >= 2 groups per wave
     if (wk == 4) launch_decode_pair<4>(args, max_m_blocks, stream);
     else launch_decode_pair<8>(args, max_m_blocks, stream);

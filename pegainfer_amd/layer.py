@@ -82,8 +82,8 @@ class RoutedExperts:
         GPUs are never read: W2 reads only local rows, and the combine skips
         non-local routes) and fuses SwiGLU into W13.  The two give the same bits
         whenever the fused and the plain W13 add over the same K shares (prefill
-        block sizes; decode grids of two or more W13 workgroups per CU with
-        K >= 512); a small decode grid splits K differently, and a W13 sum may then
+        block sizes; decode grids that expect two or more W13 (block, tile) units
+        per CU, four on a 48-expert share, with K >= 512); a small decode grid splits K differently, and a W13 sum may then
         differ in the last fp32 bit.
         `w13_timer` (optional) exposes start()/stop(mark) and is called around the
         W13 GEMM launch so a caller can time that kernel with stream events.
