@@ -19,20 +19,23 @@
 // A permuted k order that reads 256 contiguous bytes per row per step instead
 // quadruples the lines per instruction and ran 2.3x slower.
 //
+// Order of the sums, the same in both kernels below: K's 32-k steps in 1 to 16 contiguous
+// shares (k_shares), each share one chain of v_mfma_f32_16x16x32_bf16 in k order, the shares'
+// sums added in order in fp32.  A launch's bits then depend on its sizes alone, not on the
+// kernel or tile that a dispatch rule picks.  Lane (c, q) of an MFMA holds row c of the
+// tile, k 8q..8q+7 (tokens the A operand, features the B operand).
+//
 // The first kernel below serves few tokens, where the GEMM is a weight stream: one
-// workgroup owns 16 rows of W for 16 RB tokens; its WK waves split K and are reduced
-// through LDS in wave order (deterministic).  Per 32-k step a lane issues one 16-byte
-// load of W and one of X per 16-token block; after the lane exchange, lane (c, q) holds
-// row c of the tile, k 8q..8q+7 (the B fragment of a 16x16x32 MFMA) and the token blocks'
-// A fragments, and one v_mfma_f32_16x16x32_bf16 runs per token block.  A and B take
-// the same k slots per lane, so the product is exact whatever k order the
-// MFMA assigns to them.  Token rows past N read zeros through an
+// workgroup owns 16 rows of W for 16 RB tokens; its waves take the shares.  Per 32-k step a
+// lane issues one 16-byte load of W and one of X per 16-token block; after the lane exchange
+// one v_mfma_f32_16x16x32_bf16 runs per token block.  Token rows past N read zeros through an
 // out-of-range buffer offset and are never stored.
 #include <hipblaslt/hipblaslt.h>
 
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <type_traits>
 
 #include "common.h"
 #include "pega_moe.h"
@@ -44,6 +47,9 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
 
 constexpr uint32_t kOutOfRange = 0x80000000u;  // voffset that fails every range check
+constexpr int kMaxShares = 16;
+// First 32-k step of share w of 2^lg (share 2^lg starts where the last one ends).
+__device__ __forceinline__ int share_start(int steps, int w, int lg) { return (steps * w) >> lg; }
 // W loads are cached too: a step reads 64 bytes of each of 16 rows, so the
 // other half of every 128-byte line is the next step's, and a non-temporal
 // policy that does not keep the line costs 20% (44.9 against 37.3 us for
@@ -61,42 +67,49 @@ __device__ __forceinline__ u32x4_t load16(__amdgpu_buffer_rsrc_t r, uint32_t vof
                                                kPolicy);
 }
 
-template <int RB>
+template <int MR, int RB>
 struct StepRegs {
-  u32x4_t w;      // row l / 4 of the tile, W[..][k0 + 8 (l % 4) .. +7] (lane l)
+  u32x4_t w[MR];  // row l / 4 of the tile, W[..][k0 + 8 (l % 4) .. +7] (lane l)
   u32x4_t x[RB];  // X[n0 + 16 rb + l / 4][k0 + 8 (l % 4) .. +7]
 };
 
-// One workgroup per (16 rows of W, 16 RB tokens); WK waves split the K/32 steps; D steps
-// per wave in flight.  SWIGLU: the tile holds gate features m0..m0+7 and the matching up
-// features (I rows further on), so a tile completes eight outputs by itself; the epilogue
-// rounds both sums to bf16 as the GEMM's output would be, applies SwiGLU and writes
-// act[n][m0+c] (Y row stride M = I).  F32: Y is fp32 and takes the sums unrounded (the
-// router's logits GEMM, cublasGemmEx with CUDA_R_32F output).
+// One workgroup per (16 rows of W, 16 RB tokens); wave w of WV takes the shares
+// w shares / WV up to the next wave's, one after another, D steps in flight.  SWIGLU: the
+// tile holds gate features m0..m0+7 and the matching up features (I rows further on), so a
+// tile completes eight outputs by itself; the epilogue rounds both sums to bf16 as the GEMM's
+// output would be, applies SwiGLU and writes act[n][m0+c] (Y row stride M = I).  F32: Y is
+// fp32 and takes the sums unrounded (the router's logits GEMM, cublasGemmEx with CUDA_R_32F
+// output).
 //
 // A stream of W with few bytes per CU: what counts is that every CU has a workgroup and
-// that the first loads are out early.  Kimi's shared expert, 3 tokens, gate/up (58.7 MB)
-// / down (29.4 MB): 17.2 / 7.5 us with 16 waves on 32-row tiles (128 and 224 workgroups,
-// half the CUs idle in the first), 16.7 / 6.7 with eight waves on them, 12.4 / 6.7 with
-// eight and 11.8 / 6.0 us with four waves on 16-row ones (5.0 and 4.9 TB/s).  Two waves:
-// 15.9 / 6.0; eight steps in flight instead of four: 11.9 / 6.3.
-template <int WK, int RB, bool SWIGLU, bool F32>
-__global__ __launch_bounds__(64 * WK) void dense_gemm_kernel(const uint16_t* __restrict__ W,
+// that the first loads are out early.  Kimi's shared expert, 3 tokens, gate/up with SwiGLU
+// (58.7 MB) / down (29.4 MB), weights not in cache: 13.6 / 7.3 us, against 21.9 / 8.9 with a
+// wave per share on 32-row tiles (128 and 224 workgroups, half the CUs idle in the first); two
+// waves and eight steps in flight where there are two shares, 16384 x 4096 at one token, 28.8
+// (four steps: 32.4).
+template <int WV, int MR, int RB, bool SWIGLU, bool F32>
+__global__ __launch_bounds__(64 * WV) void dense_gemm_kernel(const uint16_t* __restrict__ W,
                                                              const uint16_t* __restrict__ X,
                                                              void* __restrict__ Yv, int M,
-                                                             int N, int K) {
+                                                             int N, int K, int lg_shares) {
   static_assert(!(SWIGLU && F32), "the SwiGLU epilogue writes bf16");
-  constexpr int D = 4;
-  __shared__ float s_red[WK][RB * 4][64];
+  constexpr int D = WV >= 4 || MR * RB > 3 ? 4 : 8;  // few waves: more loads in flight each
+  constexpr bool kOneShare = WV <= 2;                // launched with as many shares as waves
+  constexpr int kShares = kOneShare ? WV : kMaxShares;
+  __shared__ float s_red[kShares][MR * RB * 4][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, q = lane >> 4;
-  const int m0 = blockIdx.x * (SWIGLU ? 8 : 16);
+  constexpr int kOut = SWIGLU ? 8 : 16;  // outputs of a tile
+  const int m0 = blockIdx.x * (kOut * MR);
   const int n0 = blockIdx.y * (16 * RB);
   const int steps = K >> 5;
-  const int s0 = (steps * wave) / WK, s1 = (steps * (wave + 1)) / WK;
+  const int shares = 1 << lg_shares;
+  int sh = (shares * wave) / WV;  // this wave's first share, then the one it is in
+  const int s0 = share_start(steps, sh, lg_shares);
+  const int s1 = share_start(steps, (shares * (wave + 1)) / WV, lg_shares);
 
-  const uint32_t span = SWIGLU ? static_cast<uint32_t>(M) + 8u : 16u;
+  const uint32_t span = SWIGLU ? static_cast<uint32_t>(M) + 8u * MR : 16u * MR;
   const __amdgpu_buffer_rsrc_t wr =
       make_rsrc(W + static_cast<long long>(m0) * K, span * static_cast<uint32_t>(K) * 2u);
   // Loads run along k: lane l fetches row l / 4, k 8 (l % 4) .. +7, so four
@@ -105,7 +118,10 @@ __global__ __launch_bounds__(64 * WK) void dense_gemm_kernel(const uint16_t* __r
   // 16 bytes of row c, k 8q .. +7 that its fragment needs, from lane 4c + q.
   const uint32_t lr = static_cast<uint32_t>(lane >> 2), lp = static_cast<uint32_t>(lane & 3);
   const uint32_t w_row = SWIGLU ? (lr & 7u) + (lr >> 3) * static_cast<uint32_t>(M) : lr;
-  const uint32_t w_voff = (w_row * static_cast<uint32_t>(K) + 8u * lp) * 2u;
+  uint32_t w_voff[MR];
+#pragma unroll
+  for (int mr = 0; mr < MR; ++mr)
+    w_voff[mr] = ((w_row + kOut * mr) * static_cast<uint32_t>(K) + 8u * lp) * 2u;
   const int src_lane_bytes = (4 * c + q) * 4;
   const __amdgpu_buffer_rsrc_t xr =
       make_rsrc(X, static_cast<uint32_t>(N) * static_cast<uint32_t>(K) * 2u);
@@ -124,27 +140,50 @@ __global__ __launch_bounds__(64 * WK) void dense_gemm_kernel(const uint16_t* __r
     return __builtin_bit_cast(bf16x8_t, f);
   };
 
-  auto load_step = [&](StepRegs<RB>& r, int s) {
+  auto load_step = [&](StepRegs<MR, RB>& r, int s) {
     s = min(max(s, 0), steps - 1);  // every scalar offset stays inside the rows
     const uint32_t soff = static_cast<uint32_t>(s) * 64u;
-    r.w = load16<kCached>(wr, w_voff, soff);
+#pragma unroll
+    for (int mr = 0; mr < MR; ++mr) r.w[mr] = load16<kCached>(wr, w_voff[mr], soff);
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) r.x[rb] = load16<kCached>(xr, x_voff[rb], soff);
   };
-  floatx4_t acc[RB];
+  floatx4_t acc[MR][RB];
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) acc[rb] = floatx4_t{};
-  auto compute_step = [&](const StepRegs<RB>& r) {
+  for (int mr = 0; mr < MR; ++mr)
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) acc[mr][rb] = floatx4_t{};
+  // Accumulator element e of (mr, rb) holds token n0 + 16 rb + 4 q + e, row c of tile mr.
+  int bound = share_start(steps, sh + 1, lg_shares);
+  auto compute_step = [&](const StepRegs<MR, RB>& r) {
     bf16x8_t a[RB];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) a[rb] = to_fragment(r.x[rb]);
-    const bf16x8_t b = to_fragment(r.w);
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-      acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rb], b, acc[rb], 0, 0, 0);
+    for (int mr = 0; mr < MR; ++mr) {
+      const bf16x8_t b = to_fragment(r.w[mr]);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+        acc[mr][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rb], b, acc[mr][rb], 0, 0, 0);
+    }
+  };
+  auto flush = [&]() {
+#pragma unroll
+    for (int mr = 0; mr < MR; ++mr)
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s_red[sh][(mr * RB + rb) * 4 + e][lane] = acc[mr][rb][e];
+        acc[mr][rb] = floatx4_t{};
+      }
+  };
+  auto end_step = [&](int s) {
+    if (kOneShare || s + 1 != bound) return;  // else the share's last step
+    flush();
+    bound = share_start(steps, ++sh + 1, lg_shares);
   };
 
-  StepRegs<RB> slot[D];
+  StepRegs<MR, RB> slot[D];
 #pragma unroll
   for (int j = 0; j < D; ++j) {
     load_step(slot[j], s0 + j < s1 ? s0 + j : s1 - 1);
@@ -160,27 +199,32 @@ __global__ __launch_bounds__(64 * WK) void dense_gemm_kernel(const uint16_t* __r
     for (int j = 0; j < D; ++j) {
       compute_step(slot[j]);
       load_step(slot[j], min(s + j + D, s1 - 1));
+      end_step(s + j);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
 #pragma unroll
   for (int j = 0; j < D - 1; ++j)
-    if (s + j < s1) compute_step(slot[j]);
+    if (s + j < s1) {
+      compute_step(slot[j]);
+      end_step(s + j);
+    }
 
-  // Reduction over the WK waves in wave order.  Accumulator element e of block rb holds
-  // token n0 + 16 rb + 4 q + e, tile row c.
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) s_red[wave][rb * 4 + e][lane] = acc[rb][e];
+  if (kOneShare) flush();
+  // the shares' sums in share order
   __syncthreads();
+  constexpr int kJ = MR * RB * 4;
 #pragma unroll
-  for (int j = wave; j < RB * 4; j += WK) {
-    float sum = 0.0f;
+  for (int i = 0; i < (kJ + WV - 1) / WV; ++i) {
+    const int j = wave + i * WV;
+    if (j >= kJ) break;
+    float part[kShares], sum = 0.0f;
 #pragma unroll
-    for (int w = 0; w < WK; ++w) sum += s_red[w][j][lane];
-    const int n = n0 + 16 * (j >> 2) + 4 * q + (j & 3);
-    const long long o = static_cast<long long>(n) * M + m0 + c;
+    for (int w = 0; w < kShares; ++w) part[w] = s_red[min(w, shares - 1)][j][lane];
+#pragma unroll
+    for (int w = 0; w < kShares; ++w) sum = w < shares ? sum + part[w] : sum;
+    const int n = n0 + 16 * (j / 4 % RB) + 4 * q + (j & 3);
+    const long long o = static_cast<long long>(n) * M + m0 + kOut * (j / (4 * RB)) + c;
     if constexpr (SWIGLU) {
       const float up = __shfl_xor(sum, 8);  // tile rows 8..15
       if (n < N && c < 8)
@@ -194,19 +238,39 @@ __global__ __launch_bounds__(64 * WK) void dense_gemm_kernel(const uint16_t* __r
   }
 }
 
-template <int WK, bool SWIGLU, bool F32>
-void launch_dense(int rb, int row_tiles, const uint16_t* W, const uint16_t* X, void* Y, int M,
-                  int N, int K, hipStream_t stream) {
-  const dim3 grid(row_tiles, ceil_div(N, 16 * rb)), block(64 * WK);
-  if (rb == 1)
-    hipLaunchKernelGGL((dense_gemm_kernel<WK, 1, SWIGLU, F32>), grid, block, 0, stream, W, X, Y, M, N, K);
-  else
-    hipLaunchKernelGGL((dense_gemm_kernel<WK, 2, SWIGLU, F32>), grid, block, 0, stream, W, X, Y, M, N, K);
+template <int V>
+using Int = std::integral_constant<int, V>;
+
+int log2_shares(int shares) { return __builtin_ctz(static_cast<unsigned>(shares)); }
+
+template <int WV, int MR, int RB, bool SWIGLU, bool F32>
+void launch_dense(const uint16_t* W, const uint16_t* X, void* Y, int M, int N, int K, int shares,
+                  hipStream_t stream) {
+  const dim3 grid(M / ((SWIGLU ? 8 : 16) * MR), ceil_div(N, 16 * RB));
+  hipLaunchKernelGGL((dense_gemm_kernel<WV, MR, RB, SWIGLU, F32>), grid, dim3(64 * WV), 0, stream,
+                     W, X, Y, M, N, K, log2_shares(shares));
 }
 
 template <bool SWIGLU, bool F32>
-int dense_tile(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M, int N, int K, int cu,
-               hipStream_t stream, const char* name);
+int dense_tile(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M, int N, int K,
+               int shares, int cu, hipStream_t stream, const char* name);
+
+// The K shares of a launch (see "Order of the sums" above): 16 where few 32-feature by
+// 16..64-token units make up the output, else as many as keep 64 steps in a share.  The
+// numbers were chosen for a kernel whose waves took a share each, and are kept because they
+// are part of the results' bits; they no longer say how many waves run.
+int k_shares(bool swiglu, int M, int N, int K, int cu) {
+  const int units = swiglu ? M / 16 : M / (M % 32 == 0 ? 32 : 16);
+  int rb = N <= 16 ? 1 : N <= 32 ? 2 : N <= 48 ? 3 : 4;
+  if (rb > 1 && static_cast<long long>(units) * ceil_div(N, 16 * rb) < cu) rb = (rb + 1) / 2;
+  const long long n = static_cast<long long>(units) * ceil_div(N, 16 * rb);
+  const int steps = K / 32;
+  int shares = n <= cu ? 16 : (n <= 2LL * cu ? 8 : 4);
+  if (n >= cu)
+    while (shares > 1 && steps < 64 * shares) shares >>= 1;
+  while (shares > 1 && steps < shares) shares >>= 1;
+  return shares;
+}
 
 // Shared checks and launch.  rows = W rows read (M, or 2 I for SwiGLU),
 // M = output features per token row of Y.
@@ -221,9 +285,8 @@ int dense_launch(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M,
   if ((reinterpret_cast<uintptr_t>(W) & 15u) != 0 || (reinterpret_cast<uintptr_t>(X) & 15u) != 0)
     return fail(kNotSupported, "%s: W and X must be 16-byte aligned", name);
   // X is addressed through one 32-bit buffer range that must stay below the
-  // out-of-range offset, and so is a workgroup's W span: its 16 MR rows, or
-  // with SwiGLU its gate rows through its up rows (I + 16 rows).  The size of
-  // W as a whole does not matter.
+  // out-of-range offset, and so is a streaming workgroup's W span: 32 rows (it reads 16), or
+  // with SwiGLU its gate rows through its up rows.  The size of W as a whole does not matter.
   const long long w_span = SWIGLU ? static_cast<long long>(M) + 16 : 32;
   if (static_cast<long long>(N) * K * 2 >= static_cast<long long>(kOutOfRange) ||
       w_span * K * 2 >= static_cast<long long>(kOutOfRange))
@@ -233,65 +296,90 @@ int dense_launch(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M,
   if (cu <= 0) return fail(kInvalidValue, "%s: no device", name);
   if (ceil_div(N, 64) > 65535)
     return fail(kNotSupported, "%s: too many token blocks (N=%d)", name, N);
-  // The streaming kernel while its workgroups fit one per CU, on the smaller token blocks
-  // if those do; a second workgroup per CU costs more than reading each fragment for two
-  // token blocks (2048 x 2816, 24 tokens, 256 workgroups of 16 or 128 of 32 tokens: 4.5 /
-  // 5.7 us; 64 tokens, 512 or 256: 7.3 / 6.0).  With more workgroups, the LDS-tiled kernel
-  // below from 33 tokens on, and from 17 where its own tiles give the CUs a workgroup each
-  // (us here / there: 7168 x 2048, 20 tokens 8.1 / 7.6, 32 tokens 9.5 / 7.7; 2048 x 2816, 96
-  // tokens 9.1 / 7.5; the router's logits, 384 x 7168 fp32, which stay here, at 33 / 128
-  // tokens 12.3 / 19.6 and 12.8 / 19.6).  Its tiles read X for 32 features at a time, not
-  // 16, which also counts for fewer tokens where the weights are many: from 32 MB at 9 to
-  // 16 tokens (5120 x 5120, 16 tokens 20.6 / 17.2; 16384 x 4096, 10 tokens 27.4 / 26.1;
-  // below, 7168 x 2048 10 tokens 6.7 / 7.4), from 256 MB at 5 to 8 (gate/up 36864 x 7168
-  // 116 / 106; below, 7168 x 18432 53 / 58).
+  // The streaming kernel while its workgroups fit one per CU, on the smallest token blocks
+  // that do; a second workgroup per CU costs more than reading each fragment for two token
+  // blocks (2048 x 2816, 24 tokens, 256 workgroups of 16 or 128 of 32 tokens: 4.5 / 5.7 us;
+  // 64 tokens, 512 or 256: 7.3 / 6.0).  Blocks of 48 tokens only where the sums are in 16
+  // shares, whose short chunks cost the tile kernel most (router logits, 384 tokens, 23.8
+  // here / 29.9 there; with two shares, 4096 x 7168, 40 tokens, 23.7 / 21.1).
+  // With more workgroups, the LDS-tiled kernel below from 33 tokens on, and from 17 where its
+  // own tiles give the CUs a workgroup each; its tiles read X for 32 features at a time, not
+  // 16, which also counts for fewer tokens where the weights are many: from 64 MB at 9 to 16
+  // tokens, from 128 MB at 5 to 8 (7168 x 18432, 8 tokens 63 here / 53 there; 16384 x 4096, 9
+  // tokens 33 / 30; 5120 x 5120, 9 tokens, 19.0 / 20.0).
+  // Between the two, two feature tiles a workgroup, which halve the reads of X: at 5 to 16
+  // tokens from 32 MB of weights (5120 x 5120, 8 tokens, 21.0 with one / 18.7 with two; 8192 x
+  // 8192, 33.4 against 34.9 with the tile kernel), and for narrow outputs that fit the CUs only
+  // so (router logits at 512 tokens, 26.5 against 28 with the tile kernel; 1024 x 4096 at 250
+  // tokens, 11.2 / 12.9).
   const long long tiles = rows / 16, w_bytes = 2LL * rows * K;
-  const int rb = N <= 16 || tiles * ceil_div(N, 16) <= cu ? 1 : 2;
-  const bool many = N > 16 || (N > 8 && w_bytes >= (32LL << 20)) ||
-                    (N > 4 && w_bytes >= (256LL << 20));
-  if (tiles * ceil_div(N, 16 * rb) > cu && (N > 32 || (many && tiles >= cu * 5LL / 4)))
-    return dense_tile<SWIGLU, F32>(W, X, Y, rows, M, N, K, cu, stream, name);
-  if (K >= 4 * 32)  // a step per wave at least
-    launch_dense<4, SWIGLU, F32>(rb, static_cast<int>(tiles), W, X, Y, M, N, K, stream);
-  else
-    launch_dense<1, SWIGLU, F32>(rb, static_cast<int>(tiles), W, X, Y, M, N, K, stream);
+  const int shares = k_shares(SWIGLU, M, N, K, cu);
+  const auto fits = [&](int mr, int rb) { return tiles / mr * ceil_div(N, 16 * rb) <= cu; };
+  const int rb = N <= 16 || fits(1, 1) ? 1 : (shares == 16 && !fits(1, 2) && fits(1, 3) ? 3 : 2);
+  const bool many = N > 16 || (N > 8 && w_bytes >= (64LL << 20)) ||
+                    (N > 4 && w_bytes >= (128LL << 20));
+  bool two = false;
+  if (!fits(1, rb) && tiles % 2 == 0) {
+    if (rb == 1)
+      two = N > 4 && w_bytes >= (32LL << 20) && shares >= 4 &&
+            (!many || (shares == 4 && fits(2, 1)));
+    else if (rb == 2)
+      two = fits(2, 2) && (shares == 16 ? N > 32 : shares >= 2 && N > 128);
+  }
+  if (!two && !fits(1, rb) && (N > 32 || (many && tiles >= cu * 5LL / 4)))
+    return dense_tile<SWIGLU, F32>(W, X, Y, rows, M, N, K, shares, cu, stream, name);
+  const auto go = [&](auto wv, auto mr, auto rbc) {
+    launch_dense<decltype(wv)::value, decltype(mr)::value, decltype(rbc)::value, SWIGLU, F32>(
+        W, X, Y, M, N, K, shares, stream);
+  };
+  // waves: a share each, at most four (with two tiles eight)
+  const auto go_one = [&](auto wv) {
+    if (rb == 1) go(wv, Int<1>{}, Int<1>{});
+    else if (rb == 2) go(wv, Int<1>{}, Int<2>{});
+    else go(wv, Int<1>{}, Int<3>{});
+  };
+  const auto go_two = [&](auto wv) {
+    if (rb == 1) go(wv, Int<2>{}, Int<1>{});
+    else go(wv, Int<2>{}, Int<2>{});
+  };
+  if (two && shares >= 8) go_two(Int<8>{});
+  else if (two && shares == 4) go_two(Int<4>{});
+  else if (two) go(Int<2>{}, Int<2>{}, Int<2>{});
+  else if (shares >= 4) go_one(Int<4>{});
+  else if (shares == 2) go_one(Int<2>{});
+  else go_one(Int<1>{});
   return launch_status(name);
 }
 
 // ---------------------------------------------------------------- many tokens
-// The same GEMM for more tokens: a workgroup of eight waves owns
-// BM features x BN tokens and brings both operands straight from memory to a ring of
-// LDS stages of KC = 16 KS k.  The waves split each chunk's k into KS slices of 16
-// (and, with WM = 2, the features into halves), so that every byte of a stage is read
-// from LDS once or twice in all; each wave holds its slice's sums for the whole tile
-// (TM x TN 32x32 accumulators), and the slices are added through LDS in slice order at
-// the end.  A wave reads the next chunk's fragments while this chunk's MFMAs run; one
-// barrier per chunk.
+// The same GEMM for more tokens: a workgroup owns BM features x BN tokens and brings both
+// operands straight from memory to a ring of LDS stages of KC k.  Its waves own disjoint
+// blocks of the tile (TM x TN of 16 x 16) for all of K, so that the sums keep the order given
+// above: at a share's end a wave adds the share's sums to its totals.  One barrier per chunk.
 //
-// Kimi's shared expert (gate/up with SwiGLU 4096 x 7168, down 7168 x 2048) at 64 / 100 / 160 /
-// 250 tokens: gate/up 21.3 / 21.6 / 27.5 / 31.2 us, down 8.4 / 10.2 / 16.7 / 18.7 us, against
-// 22.6 / 29.9 / 44.6 / 55.9 and 12.1 / 17.0 / 21.6 / 30.7 us with the streaming kernel above,
-// whose fragments cross lanes through ds_bpermute; the router's logits (384 x 7168, fp32) at
-// 1000 / 4096 tokens 24.6 / 60.3 against 40.4 / 90.3 us.
+// Kimi's shared expert (gate/up with SwiGLU 4096 x 7168, down 7168 x 2048) at 64 / 160 / 250
+// tokens: gate/up 22.5 / 32.5 / 35.0 us, down 9.6 / 20.1 / 20.3 us, against 26.4 / 47.0 / 59.8
+// and 12.1 / 22.2 / 30.7 us with the streaming kernel, whose fragments cross lanes through
+// ds_bpermute; the router's logits (384 x 7168, fp32) at 1000 / 4096 tokens 27.9 / 67.8
+// against 41.0 / 90.6 us.
 //
 // A row's 16-byte pieces are stored at slot piece ^ (row % pieces), which spreads the
-// fragment reads (32 rows, one piece) over the banks.  Bound by what a CU can bring in
-// from L2 (64 bytes a cycle) at few tokens, by the matrix pipe and LDS at many.
-typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16_t;
-
-template <int WM_, int TM_, int TN_, int KS_, int NS_>
+// fragment reads (16 rows, one piece) over the banks.  Bound by what a CU can bring in
+// from L2 at few tokens, by LDS reads and the matrix pipe at many.
+template <int WM_, int WN_, int TM_, int TN_, int KC_, int NS_>
 struct TileShape {
-  static constexpr int WM = WM_, TM = TM_, TN = TN_, KS = KS_, NS = NS_;
-  static constexpr int KC = 16 * KS, kRowBytes = 2 * KC, kPieces = kRowBytes / 16;
-  static constexpr int BM = 32 * WM * TM, BN = 32 * TN;
+  static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, KC = KC_, NS = NS_;
+  static constexpr int kWaves = WM * WN, kThreads = 64 * kWaves;
+  static constexpr int kRowBytes = 2 * KC, kPieces = kRowBytes / 16;
+  static constexpr int BM = 16 * WM * TM, BN = 16 * WN * TN;
   static constexpr int kStage = (BM + BN) * kRowBytes;
   static constexpr int kRowsPerLoad = 1024 / kRowBytes;
-  static constexpr int P = (BM + BN) / kRowsPerLoad / 8;  // loads per wave and chunk
-  // token blocks whose partial sums fit LDS at once, and their bytes
-  static constexpr int TNR = KS * 32 * TN * (BM + 8) * 4 <= 160 * 1024 ? TN : TN / 2;
-  static constexpr int kRed = KS * 32 * TNR * (BM + 8) * 4;
-  static constexpr int kLds = NS * kStage > kRed ? NS * kStage : kRed;
-  static_assert(WM * KS == 8 && P * 8 * kRowsPerLoad == BM + BN && TN % TNR == 0, "tile shape");
+  static constexpr int P = (BM + BN) / kRowsPerLoad / kWaves;  // loads per wave and chunk
+  static constexpr int kPitch = BM + 8;                        // floats per row of the epilogue
+  static constexpr int kOut = BN * kPitch * 4;
+  static constexpr int kLds = NS * kStage > kOut ? NS * kStage : kOut;
+  static_assert(P * kWaves * kRowsPerLoad == BM + BN && KC % 32 == 0, "tile shape");
+  static_assert(BM / 2 % kRowsPerLoad == 0, "a load's rows are all gate, up or tokens");
   static_assert(kLds <= 160 * 1024 && NS >= 3 && (kPieces & (kPieces - 1)) == 0, "tile shape");
 };
 
@@ -299,19 +387,21 @@ struct TileShape {
 // (inter with SWIGLU, whose W has 2 M rows: the tile's first half holds gate features, its
 // second half the matching up features).
 template <typename S, bool SWIGLU, bool F32>
-__global__ __launch_bounds__(512, 2) void dense_tile_kernel(const uint16_t* __restrict__ W,
-                                                            const uint16_t* __restrict__ X,
-                                                            void* __restrict__ Yv, int M, int N,
-                                                            int K, bool wide) {
+__global__ __launch_bounds__(S::kThreads) void dense_tile_kernel(const uint16_t* __restrict__ W,
+                                                                 const uint16_t* __restrict__ X,
+                                                                 void* __restrict__ Yv, int M,
+                                                                 int N, int K, int lg_shares,
+                                                                 bool wide) {
   constexpr int BM = S::BM, BN = S::BN, NS = S::NS, P = S::P, TM = S::TM, TN = S::TN;
   constexpr int BMO = SWIGLU ? BM / 2 : BM;  // output features of the tile
+  constexpr int kSteps = S::KC / 32;         // 32-k steps per chunk
   __shared__ __align__(1024) uint8_t smem[S::kLds];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / S::KS, ks = wave % S::KS;
-  const int c = lane & 31, h = lane >> 5;
+  const int wm = wave % S::WM, wn = wave / S::WM;
+  const int c = lane & 15, q = lane >> 4;
   const int m0 = blockIdx.x * BMO, n0 = blockIdx.y * BN;
-  const int chunks = ceil_div(K, S::KC);
+  const int steps = K >> 5;
   const uint32_t row_bytes = static_cast<uint32_t>(K) * 2u;
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
       (__attribute__((address_space(3))) uint8_t*)smem));
@@ -337,152 +427,180 @@ __global__ __launch_bounds__(512, 2) void dense_tile_kernel(const uint16_t* __re
     voff[j] = static_cast<uint32_t>(r - part0) * row_bytes + 16u * piece;
     piece_k[j] = 8 * piece;
   }
-  auto stage_in = [&](int ch, int st) {
-#pragma unroll
-    for (int j = 0; j < P; ++j) {
-      // pieces past K (the last chunk of a K that is not whole chunks) bring zeros
-      const uint32_t past = piece_k[j] + ch * S::KC < K ? 0u : kOutOfRange;
-      dma_b128(rsrc[j], dst[j] + static_cast<uint32_t>(st), voff[j] | past,
-               static_cast<uint32_t>(ch) * S::kRowBytes);
+  // The chunks: whole KC from each share's first step on, the share's last chunk shorter.
+  struct Place {
+    int share, step, end;  // the chunk's share, first step, and the share's end
+  };
+  auto advance = [&](Place& p) {
+    p.step += kSteps;
+    if (p.step >= p.end) {
+      p.step = p.end;
+      p.end = share_start(steps, ++p.share + 1, lg_shares);
     }
   };
-  const int slot = 16 * ((2 * ks + h) ^ (c % S::kPieces));
-  const uint8_t* w_rd = smem + (wm * TM * 32 + c) * S::kRowBytes + slot;
-  const uint8_t* x_rd = smem + (BM + c) * S::kRowBytes + slot;
-  struct Frags {
-    bf16x8_t w[TM], x[TN];
+  const Place first{0, 0, share_start(steps, 1, lg_shares)};
+  int chunks = 0;
+  for (int w = 0; w < 1 << lg_shares; ++w)
+    chunks += (share_start(steps, w + 1, lg_shares) - share_start(steps, w, lg_shares) + kSteps - 1) /
+              kSteps;
+  auto stage_in = [&](const Place& p, int st) {
+    const int past_k = (p.end - p.step) * 32;
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+      // pieces past the share's end bring zeros, in both operands: their products are zeros
+      const uint32_t past = piece_k[j] < past_k ? 0u : kOutOfRange;
+      dma_b128(rsrc[j], dst[j] + static_cast<uint32_t>(st), voff[j] | past,
+               static_cast<uint32_t>(p.step) * 64u);
+    }
   };
+  struct Frags {  // of a chunk
+    bf16x8_t w[kSteps][TM], x[kSteps][TN];
+  };
+  const uint8_t* w_rd = smem + (wm * TM * 16 + c) * S::kRowBytes;
+  const uint8_t* x_rd = smem + (BM + wn * TN * 16 + c) * S::kRowBytes;
   auto read = [&](Frags& f, int st) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
-      f.w[i] = *reinterpret_cast<const bf16x8_t*>(w_rd + st + 32 * S::kRowBytes * i);
+    for (int i = 0; i < kSteps; ++i) {
+      const int slot = 16 * ((4 * i + q) ^ (c % S::kPieces)) + st;
 #pragma unroll
-    for (int i = 0; i < TN; ++i)
-      f.x[i] = *reinterpret_cast<const bf16x8_t*>(x_rd + st + 32 * S::kRowBytes * i);
+      for (int t = 0; t < TM; ++t)
+        f.w[i][t] = *reinterpret_cast<const bf16x8_t*>(w_rd + slot + 16 * S::kRowBytes * t);
+#pragma unroll
+      for (int t = 0; t < TN; ++t)
+        f.x[i][t] = *reinterpret_cast<const bf16x8_t*>(x_rd + slot + 16 * S::kRowBytes * t);
+    }
   };
-  floatx16_t acc[TM][TN];
+  floatx4_t acc[TM][TN], total[TM][TN];  // a share's sums; the sum of the shares before it
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = floatx16_t{};
+    for (int j = 0; j < TN; ++j) acc[i][j] = total[i][j] = floatx4_t{};
   auto products = [&](const Frags& f) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+    for (int i = 0; i < kSteps; ++i)
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.x[j], f.w[i], acc[i][j], 0, 0, 0);
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int t = 0; t < TM; ++t)
+          acc[t][j] =
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.x[i][j], f.w[i][t], acc[t][j], 0, 0, 0);
+  };
+  auto end_share = [&]() {
+#pragma unroll
+    for (int t = 0; t < TM; ++t)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) total[t][j][e] += acc[t][j][e];
+        acc[t][j] = floatx4_t{};
+      }
   };
 
+  Place in = first, at = first;  // of the next chunk to bring in, and to multiply
 #pragma unroll
   for (int i = 0; i < NS - 1; ++i)
-    if (i < chunks) stage_in(i, i * S::kStage);
+    if (i < chunks) {
+      stage_in(in, i * S::kStage);
+      advance(in);
+    }
   if (chunks >= NS - 1) vm_wait<(NS - 2) * P>(); else vm_wait<0>();
   lds_barrier();
   Frags f0, f1;
   read(f0, 0);
-  // Step ch: chunk ch + 1 lands, chunk ch + NS - 1 goes into the stage of chunk ch - 1
-  // (every wave has its fragments of it, and this barrier follows its last read), the
-  // next fragments are read and this chunk's products run.
+  // Chunk ch: the next chunk has landed (each wave waits for its own loads, the barrier for
+  // all), every wave has chunk ch - 1's fragments, whose stage chunk ch + NS - 1 then fills,
+  // and the next chunk's fragments are read while this chunk's products run.
   int st_rd = S::kStage, st_in = (NS - 1) * S::kStage;
   auto next = [](int st) { return st + S::kStage == NS * S::kStage ? 0 : st + S::kStage; };
-  auto step = [&](const Frags& cur, Frags& nxt, int ch) {
+  auto chunk = [&](const Frags& cur, Frags& nxt, int ch) {
     if (ch + NS - 2 < chunks) vm_wait<(NS - 3) * P>(); else vm_wait<0>();
     lds_barrier();
-    if (ch + NS - 1 < chunks) stage_in(ch + NS - 1, st_in);
+    if (ch + NS - 1 < chunks) {
+      stage_in(in, st_in);
+      advance(in);
+    }
     read(nxt, st_rd);  // past the last chunk: a stage whose words are not used
     st_in = next(st_in);
     st_rd = next(st_rd);
     products(cur);
+    const int share = at.share;
+    advance(at);
+    if (at.share != share) end_share();
   };
   for (int ch = 0; ch < chunks; ch += 2) {
-    step(f0, f1, ch);
-    if (ch + 1 < chunks) step(f1, f0, ch + 1);
+    chunk(f0, f1, ch);
+    if (ch + 1 < chunks) chunk(f1, f0, ch + 1);
   }
 
-  // The KS slices' sums through LDS, TNR token blocks at a time, then four output
-  // features per thread, slices in order.
-  constexpr int kPitch = BM + 8;
-  float* red = reinterpret_cast<float*>(smem);
+  // The totals through LDS as [token][feature], then four output features per thread.
+  float* out = reinterpret_cast<float*>(smem);
+  lds_barrier();  // the ring is read
 #pragma unroll
-  for (int t0 = 0; t0 < TN; t0 += S::TNR) {
-    lds_barrier();  // the ring, or the previous blocks' sums, are read
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < S::TNR; ++j)
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-          red[(ks * 32 * S::TNR + 32 * j + 8 * (e >> 2) + 4 * h + (e & 3)) * kPitch +
-              (wm * TM + i) * 32 + c] = acc[i][t0 + j][e];
-    __syncthreads();
-    for (int o = tid; o < 32 * S::TNR * (BMO / 4); o += 512) {
-      const int r = o / (BMO / 4), f = (o % (BMO / 4)) * 4;
-      const int n = n0 + 32 * t0 + r;
-      if (n >= N || m0 + f >= M) continue;
-      float g[4] = {0, 0, 0, 0}, u[4] = {0, 0, 0, 0};
-#pragma unroll
-      for (int s = 0; s < S::KS; ++s) {
-        const float* src = red + (s * 32 * S::TNR + r) * kPitch + f;
-        const float4 v = *reinterpret_cast<const float4*>(src);
-        g[0] += v.x;
-        g[1] += v.y;
-        g[2] += v.z;
-        g[3] += v.w;
-        if constexpr (SWIGLU) {
-          const float4 w = *reinterpret_cast<const float4*>(src + BMO);
-          u[0] += w.x;
-          u[1] += w.y;
-          u[2] += w.z;
-          u[3] += w.w;
-        }
-      }
-      const long long at = static_cast<long long>(n) * M + m0 + f;
-      if constexpr (F32) {
-        float* y = static_cast<float*>(Yv) + at;
-        if (wide) {
-          *reinterpret_cast<float4*>(y) = make_float4(g[0], g[1], g[2], g[3]);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) y[e] = g[e];
-        }
+      for (int e = 0; e < 4; ++e)
+        out[((wn * TN + j) * 16 + 4 * q + e) * S::kPitch + (wm * TM + i) * 16 + c] = total[i][j][e];
+  __syncthreads();
+  for (int o = tid; o < BN * (BMO / 4); o += S::kThreads) {
+    const int r = o / (BMO / 4), f = (o % (BMO / 4)) * 4;
+    const int n = n0 + r;
+    if (n >= N || m0 + f >= M) continue;
+    const float4 g4 = *reinterpret_cast<const float4*>(out + r * S::kPitch + f);
+    const long long at = static_cast<long long>(n) * M + m0 + f;
+    if constexpr (F32) {
+      float* y = static_cast<float*>(Yv) + at;
+      if (wide) {
+        *reinterpret_cast<float4*>(y) = g4;
       } else {
-        uint16_t* y = static_cast<uint16_t*>(Yv) + at;
-        uint16_t b[4];
+        y[0] = g4.x;
+        y[1] = g4.y;
+        y[2] = g4.z;
+        y[3] = g4.w;
+      }
+    } else {
+      uint16_t* y = static_cast<uint16_t*>(Yv) + at;
+      const float g[4] = {g4.x, g4.y, g4.z, g4.w};
+      uint16_t b[4];
+      if constexpr (SWIGLU) {
+        const float4 u4 = *reinterpret_cast<const float4*>(out + r * S::kPitch + f + BMO);
+        const float u[4] = {u4.x, u4.y, u4.z, u4.w};
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          b[e] = SWIGLU ? swiglu_one(bf2f(f2bf(g[e])), bf2f(f2bf(u[e]))) : f2bf(g[e]);
-        if (wide) {
-          *reinterpret_cast<uint2*>(y) = make_uint2(b[0] | (static_cast<uint32_t>(b[1]) << 16),
-                                                    b[2] | (static_cast<uint32_t>(b[3]) << 16));
-        } else {
+        for (int e = 0; e < 4; ++e) b[e] = swiglu_one(bf2f(f2bf(g[e])), bf2f(f2bf(u[e])));
+      } else {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) y[e] = b[e];
-        }
+        for (int e = 0; e < 4; ++e) b[e] = f2bf(g[e]);
+      }
+      if (wide) {
+        *reinterpret_cast<uint2*>(y) = make_uint2(b[0] | (static_cast<uint32_t>(b[1]) << 16),
+                                                  b[2] | (static_cast<uint32_t>(b[3]) << 16));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = b[e];
       }
     }
   }
 }
 
 template <typename S, bool SWIGLU, bool F32>
-int launch_tile(const uint16_t* W, const uint16_t* X, void* Y, int M, int N, int K,
+int launch_tile(const uint16_t* W, const uint16_t* X, void* Y, int M, int N, int K, int shares,
                 hipStream_t stream, const char* name) {
   const dim3 grid(ceil_div(M, SWIGLU ? S::BM / 2 : S::BM), ceil_div(N, S::BN));
   // four outputs of a row per store where Y's alignment allows it
   const bool wide = (reinterpret_cast<uintptr_t>(Y) & (F32 ? 15u : 7u)) == 0;
-  hipLaunchKernelGGL((dense_tile_kernel<S, SWIGLU, F32>), grid, dim3(512), 0, stream, W, X, Y, M, N,
-                     K, wide);
+  hipLaunchKernelGGL((dense_tile_kernel<S, SWIGLU, F32>), grid, dim3(S::kThreads), 0, stream, W, X,
+                     Y, M, N, K, log2_shares(shares), wide);
   return launch_status(name);
 }
 
 // The tile shape whose slowest CU brings in the fewest bytes: a CU's workgroups times the
 // rows of a stage, since all of these shapes read their operands at about the same rate
-// (15-17 TB/s over the GPU: what bounds them).  On a tie the larger tile.  At 4096 weight
-// rows of 7168 (with SwiGLU) 32 x 32 / 32 x 64 / 32 x 96 / 64 x 64 take 21.2 / 23.3 / 26.1 /
-// 31.1 us at 64 tokens, 26.1 / 21.6 / 26.1 / 28.6 at 100, 41.1 / 38.2 / 27.5 / 28.8 at 160,
-// 47.4 / 40.3 / 48.4 / 31.8 at 250.
+// (what bounds them).  On a tie the larger tile.  The 32 x 32 tile has eight stages: it brings
+// in the least per chunk (4096 x 7168, 40 tokens, four / eight stages 23.8 / 21.1 us).
 template <bool SWIGLU, bool F32>
-int dense_tile(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M, int N, int K, int cu,
-               hipStream_t stream, const char* name) {
+int dense_tile(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M, int N, int K,
+               int shares, int cu, hipStream_t stream, const char* name) {
   // BM, BN in order of preference
   constexpr int kShapes[6][2] = {{128, 128}, {64, 64}, {64, 32}, {32, 64}, {32, 96}, {32, 32}};
   int pick = 0;
@@ -496,13 +614,16 @@ int dense_tile(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M, i
       pick = i;
     }
   }
+  const auto go = [&](auto shape) {
+    return launch_tile<decltype(shape), SWIGLU, F32>(W, X, Y, M, N, K, shares, stream, name);
+  };
   switch (pick) {
-    case 0: return launch_tile<TileShape<2, 2, 4, 4, 4>, SWIGLU, F32>(W, X, Y, M, N, K, stream, name);
-    case 1: return launch_tile<TileShape<1, 2, 2, 8, 4>, SWIGLU, F32>(W, X, Y, M, N, K, stream, name);
-    case 2: return launch_tile<TileShape<1, 2, 1, 8, 6>, SWIGLU, F32>(W, X, Y, M, N, K, stream, name);
-    case 3: return launch_tile<TileShape<1, 1, 2, 8, 6>, SWIGLU, F32>(W, X, Y, M, N, K, stream, name);
-    case 4: return launch_tile<TileShape<1, 1, 3, 8, 4>, SWIGLU, F32>(W, X, Y, M, N, K, stream, name);
-    default: return launch_tile<TileShape<1, 1, 1, 8, 4>, SWIGLU, F32>(W, X, Y, M, N, K, stream, name);
+    case 0: return go(TileShape<4, 2, 2, 4, 64, 4>{});
+    case 1: return go(TileShape<2, 4, 2, 1, 128, 4>{});
+    case 2: return go(TileShape<4, 2, 1, 1, 128, 6>{});
+    case 3: return go(TileShape<2, 4, 1, 1, 128, 6>{});
+    case 4: return go(TileShape<2, 2, 1, 3, 128, 4>{});
+    default: return go(TileShape<2, 2, 1, 1, 128, 8>{});
   }
 }
 
@@ -622,8 +743,7 @@ using namespace pega;
 
 // Reference: pegainfer-kernels/src/ffi/shared.rs:220-228 (gemm_cuda) and
 // :230-238 (gemm_graphsafe_cuda); both compute the same GEMM.  Below 256
-// tokens this library's weight-streaming kernel runs; from 256 up, hipBLASLt
-// (no workspace).  Neither allocates device memory per call, so both are
+// tokens this library's kernels run; from 256 up, hipBLASLt (no workspace).  Neither allocates device memory per call, so both are
 // graph-safe once a shape has been called outside the capture (its first call
 // on a device makes the hipBLASLt handle and plan).
 PEGA_API int gemm_cuda(const uint16_t* W, const uint16_t* X, uint16_t* Y, int M, int N, int K,

@@ -364,3 +364,63 @@ def test_dense_stream_shapes_exact(oracle, M, N, K):
         chain = torch.zeros(N, M // 2, dtype=torch.bfloat16, device="cuda")
         ops.kimi_marlin_w13_swiglu(y[:N], chain, N, M // 2)
         assert np.array_equal(host(fused[:N]), host(chain)) and bool((fused[N] == 7.0).all())
+
+
+@pytest.mark.parametrize("M,N,K,shares", [
+    (384, 1, 7168, 16), (384, 33, 7168, 16), (384, 400, 7168, 16),  # router logits
+    (384, 1000, 7168, 2), (384, 4100, 4096, 2),
+    (2048, 96, 2816, 16), (4096, 5, 7168, 16), (4096, 24, 7168, 2), (4096, 64, 7168, 2),
+    (4096, 100, 4128, 2), (4096, 250, 7168, 2), (16384, 3, 16384, 8), (16384, 12, 4096, 2),
+    (16384, 100, 8192, 4), (48, 17, 544, 16), (48, 200, 352, 8), (5120, 7, 5120, 16),
+    (5120, 12, 5120, 16), (16384, 7, 4096, 2), (1024, 250, 4096, 2), (1024, 250, 8192, 4),
+    (2048, 65, 2048, 16)])
+def test_dense_sums_are_shares_of_k_in_order(oracle, M, N, K, shares):
+    """The order of the fp32 sums: `shares` contiguous parts of K's 32-k steps, added in order.
+    One nonzero k in each share makes a share's sum one exact product, and a large term that
+    a later share cancels makes the order of the additions show in every output format, so the
+    result equals the ordered fp32 sum bit for bit and another grouping's does not."""
+    from pegainfer_amd import ops
+    g = np.random.default_rng(M + N + K)
+    steps = K // 32
+    def bf16(*shape):
+        return oracle.bf16_to_f32(oracle.f32_to_bf16(g.uniform(0.5, 1, shape).astype(np.float32)))
+    if shares == 2:
+        # share 0: big + a small term, which its chain's sum loses; share 1: -big, then a small
+        # negative term, lost likewise
+        half = steps // 2 * 32
+        at = [0, 40, half + 16, half + 32 + (112 - half - 32) % 128]
+        col, xs = bf16(M, 4), bf16(N, 4)
+        col[:, 2] = col[:, 0]
+        xs[:, 0], xs[:, 2] = 2.0 ** 30, -2.0 ** 30
+        xs[:, 3] *= -1
+        ref = np.zeros((N, M), np.float32)
+    else:
+        at = [32 * int(g.integers(steps * s // shares, steps * (s + 1) // shares))
+              + int(g.integers(0, 32)) for s in range(shares)]
+        col, xs = bf16(M, shares), bf16(N, shares)
+        first, last = (int(v) for v in sorted(g.choice(shares, 2, replace=False)))
+        col[:, last] = col[:, first]
+        xs[:, first], xs[:, last] = 2.0 ** 20, -2.0 ** 20
+        ref = np.zeros((N, M), np.float32)
+        for s in range(shares):
+            ref = ref + xs[:, s:s + 1] * col[:, s]
+    w = torch.zeros(M, K, dtype=torch.bfloat16, device="cuda")
+    x = torch.zeros(N, K, dtype=torch.bfloat16, device="cuda")
+    w[:, at] = dev(col).to(torch.bfloat16)
+    x[:, at] = dev(xs).to(torch.bfloat16)
+    if M == 384:
+        got = torch.zeros(N, M, device="cuda")
+        ops.kimi_k2_router_noaux_tc(x, w, torch.zeros(M, device="cuda"), got,
+                                    torch.zeros(N, 8, device="cuda"),
+                                    torch.zeros(N, 8, dtype=torch.int32, device="cuda"), N, N)
+        assert np.array_equal(host(got), ref)
+    if N < 256:
+        y = torch.zeros(N, M, dtype=torch.bfloat16, device="cuda")
+        ops.gemm_graphsafe(w, x, y)
+        assert np.array_equal(host(y), oracle.f32_to_bf16(ref))
+        if M % 32 == 0:
+            act = torch.zeros(N, M // 2, dtype=torch.bfloat16, device="cuda")
+            ops.dense_w13_swiglu(w, x, act)
+            chain = torch.zeros_like(act)
+            ops.kimi_marlin_w13_swiglu(y, chain, N, M // 2)
+            assert np.array_equal(host(act), host(chain))
