@@ -91,6 +91,14 @@ __device__ __forceinline__ WordPairs dequant_word(uint32_t x, const ColScale& a,
   return r;
 }
 
+// Half of a word, as above for column n0 (n1 with the word shifted right by 8).
+__device__ __forceinline__ void dequant_half(uint32_t x, const ColScale& a, const DqConst& k,
+                                             uint32_t& lo, uint32_t& hi) {
+  const uint32_t p0 = x & k.m_lo, p1 = x & k.m_hi;
+  lo = pack_bf16x2(__builtin_fmaf(h_lo(p0), a.s24, a.c8), __builtin_fmaf(h_hi(p0), a.s24, a.c8));
+  hi = pack_bf16x2(__builtin_fmaf(h_lo(p1), a.s20, a.c8), __builtin_fmaf(h_hi(p1), a.s20, a.c8));
+}
+
 __device__ __forceinline__ bf16x8_t as_bf16x8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
   u32x4_t v = {a, b, c, d};
   return __builtin_bit_cast(bf16x8_t, v);
@@ -461,6 +469,7 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 6) void wna16_decode16_k
   __shared__ float s_red[kWaves][16][64];
   __shared__ __align__(16) uint32_t s_w[kWaves][2][kSlotDwords];
 
+  __builtin_amdgcn_s_setprio(1);  // ahead of the few-rows kernel's waves (see there)
   const int n_tiles = p.size_n >> 6;
   const int n_units = kPair ? (p.inter >> 6) : n_tiles;
   const int split = blockIdx.x / n_units;
@@ -656,30 +665,36 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 6) void wna16_decode16_k
 // Decode kernel for blocks of 32 to 64 rows that hold few routed ones: the
 // 32-row kernel above with all 32 MFMA rows in use (two 16-byte activation
 // loads per lane and group, k 0..7 and 8..15 of its half).  blockIdx.z is the
-// 32-row part of the block; parts without a routed row leave at once.  Bound by
-// the dequant's vector instructions like the kernels above; 120 VGPRs, four waves
-// per SIMD, so two 8-wave W13 workgroups a CU.  Kimi W13 + SwiGLU / W2 at 160
-// tokens (35 experts touched): 122 us (4.7 TB/s) / 68 us against 158 / 65 with the
-// tile kernel, whose 560 workgroups of 100 us each left most CUs idle for the last
-// third of the launch.
+// 32-row part of the block; parts without a routed row leave at once.  One wave per
+// (part, column tile) runs all of K, in the tile kernel's order, so a launch's bits do not
+// depend on which of the two a dispatch rule picks.  Bound by the dequant's vector
+// instructions like the kernels above; where few waves run, by one wave's chain, so the
+// next group is dequantised between this group's MFMAs (one expert, 2048 x 7168 at 64 rows:
+// 56 us without, 72 with the tile kernel; two waves a tile 39).  Kimi's MoE block, 160 tokens
+// (35 experts touched): 245 us against 289 with the tile kernel.
+// The other kernels of this file run at a wave priority of 1: a shared expert in this form
+// beside the routed experts, on another stream, then takes what they leave (DeepSeek-V2-Lite
+// layer at 64 / 100 tokens 106 / 114 us; at equal priority 116 / 126).
 struct GroupRegs32 {
   u32x4_t raw;
   uint32_t sp;
   u32x4_t a0, a1;
 };
 
-template <int WK, int D, bool kPair = false>
-__global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 4) void wna16_decode32_kernel(GemmArgs p) {
+// CS = 2: two waves per column tile, one of its n0 columns, one of its n1 columns.
+template <int D, bool kPair, int CS>
+__global__ __launch_bounds__(64 * (kPair ? 2 : CS), CS == 1 ? 3 : 2)
+void wna16_decode32_kernel(GemmArgs p) {
   static_assert(D % 2 == 0, "the two transpose slots alternate with the ring position");
-  constexpr int kWaves = WK * (kPair ? 2 : 1);
+  static_assert(!(kPair && CS == 2), "a pair has its two waves already");
+  constexpr int kWaves = kPair ? 2 : CS;  // kPair: a gate tile's wave, then its up tile's
+  constexpr int NB = 2 / CS;                    // 32-column MFMAs of a wave
   __shared__ int s_sid[32];
-  // the transpose slots ([wave][2][kSlotDwords]), then the reduction ([wave][32][64])
-  __shared__ __align__(16) uint32_t s_mem[kWaves * 32 * 64];
-  static_assert(2 * kSlotDwords <= 32 * 64, "the slots fit the reduction buffer");
+  // the transpose slots ([wave][2][kSlotDwords]), then the sums ([wave][16 NB][64])
+  __shared__ __align__(16) uint32_t s_mem[kWaves * 16 * NB * 64];
+  static_assert(2 * kSlotDwords <= 16 * NB * 64, "the slots fit the sums");
 
   const int n_tiles = p.size_n >> 6;
-  const int n_units = kPair ? (p.inter >> 6) : n_tiles;
-  const int split = blockIdx.x / n_units;
   const int mb = blockIdx.y, row0 = 32 * blockIdx.z;
   const int tid = threadIdx.x, lane = tid & 63;
   const int valid_limit = p.size_m * p.top_k;
@@ -693,16 +708,13 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 4) void wna16_decode32_k
   if (ntp < (mb + 1) * p.bs || expert < 0 || expert >= p.num_experts || !routed) return;
 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int kw = wave % WK;
-  const int half = wave / WK;
-  const int nt = blockIdx.x % n_units + (kPair ? half * (p.inter >> 6) : 0);
+  const int nt = blockIdx.x + (kPair ? wave * (p.inter >> 6) : 0);
+  const int cs = CS == 2 ? wave : 0;
   if (tid < 32) s_sid[tid] = sid;
   const int c = lane & 31, h = lane >> 5;
   const int my_sid = __builtin_amdgcn_ds_bpermute(c << 2, sid);
   const int K = p.size_k, N = p.size_n;
   const int groups = K >> 5;
-  const int gs0 = (groups * split) / p.splits, gs1 = (groups * (split + 1)) / p.splits;
-  const int g0 = gs0 + ((gs1 - gs0) * kw) / WK, g1 = gs0 + ((gs1 - gs0) * (kw + 1)) / WK;
 
   const uint32_t expert_bytes = static_cast<uint32_t>(N) * static_cast<uint32_t>(K) / 2u;
   const __amdgpu_buffer_rsrc_t wr = make_rsrc(
@@ -728,21 +740,12 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 4) void wna16_decode32_k
   const uint32_t* slot_r0 = slots + h * 160 + 4 * c;
 
   auto load_group = [&](GroupRegs32& r, int g) {
-    g = min(max(g, 0), groups - 1);
-    r.raw = buf_load_b128<kStream>(wr, w_voff, static_cast<uint32_t>(g) * w_step);
-    r.sp = buf_load_b32<kStream>(sr, s_voff, static_cast<uint32_t>(g) * s_step);
+    g = min(g, groups - 1);
+    r.raw = buf_load_b128<CS == 1 ? kStream : kCached>(wr, w_voff, static_cast<uint32_t>(g) * w_step);
+    r.sp = buf_load_b32<CS == 1 ? kStream : kCached>(sr, s_voff, static_cast<uint32_t>(g) * s_step);
     r.a0 = buf_load_b128(ar, a_voff, static_cast<uint32_t>(g) * 64u);
     r.a1 = buf_load_b128(ar, a_voff + 16u, static_cast<uint32_t>(g) * 64u);
   };
-
-  const DqConst dq = dq_consts();
-  floatx16_t accx = {}, accy = {};
-  GroupRegs32 slot[D];
-#pragma unroll
-  for (int q = 0; q < D; ++q) {
-    load_group(slot[q], g0 + q < g1 ? g0 + q : g1 - 1);
-    __builtin_amdgcn_sched_barrier(0);
-  }
   auto write_tr = [&](const GroupRegs32& r, int par) {
     uint32_t* sw = slot_w0 + par * kSlotDwords;
     sw[0] = r.raw[0];
@@ -750,65 +753,100 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 4) void wna16_decode32_k
     sw[64] = r.raw[2];
     sw[96] = r.raw[3];
   };
-  auto compute_group = [&](const GroupRegs32& r, int par) {
-    const u32x4_t fw = *reinterpret_cast<const u32x4_t*>(slot_r0 + par * kSlotDwords);
-    const uint32_t w4[4] = {fw[0], fw[1], fw[2], fw[3]};
-    const BFrags b = make_b(w4, r.sp, dq);
-    const bf16x8_t A1 = __builtin_bit_cast(bf16x8_t, r.a0);
-    const bf16x8_t A2 = __builtin_bit_cast(bf16x8_t, r.a1);
-    accx = mfma(A1, b.x1, accx);
-    accy = mfma(A1, b.y1, accy);
-    accx = mfma(A2, b.x2, accx);
-    accy = mfma(A2, b.y2, accy);
+  const DqConst dq = dq_consts();
+  // the B fragments of a group: per 32-column MFMA k 0..7 and k 8..15 of the lane's half
+  struct Frags {
+    bf16x8_t b[NB][2];
   };
-
-  const int rounds = (g1 - g0) / D;
-  int g = g0;
-  write_tr(slot[0], 0);
-  for (int r = 0; r < rounds; ++r, g += D) {
+  auto fragments = [&](Frags& f, uint32_t sp, int par) {
+    const u32x4_t fw = *reinterpret_cast<const u32x4_t*>(slot_r0 + par * kSlotDwords);
+    uint32_t w4[4] = {fw[0], fw[1], fw[2], fw[3]};
+    if constexpr (CS == 1) {
+      const BFrags b = make_b(w4, sp, dq);
+      f.b[0][0] = b.x1;
+      f.b[0][1] = b.x2;
+      f.b[NB - 1][0] = b.y1;
+      f.b[NB - 1][1] = b.y2;
+    } else {
+      const ColScale sc = col_scale(cs ? bf_hi(sp) : bf_lo(sp));
+      uint32_t lo[4], hi[4];
 #pragma unroll
-    for (int q = 0; q < D; ++q) {
-      write_tr(slot[(q + 1) % D], (q + 1) & 1);
-      compute_group(slot[q], q & 1);
-      load_group(slot[q], min(g + q + D, g1 - 1));
-      __builtin_amdgcn_sched_barrier(0);
+      for (int jj = 0; jj < 4; ++jj) dequant_half(w4[jj] >> (8 * cs), sc, dq, lo[jj], hi[jj]);
+      f.b[0][0] = as_bf16x8(lo[0], lo[1], lo[2], lo[3]);
+      f.b[0][1] = as_bf16x8(hi[0], hi[1], hi[2], hi[3]);
+    }
+  };
+  floatx16_t acc[NB];
+#pragma unroll
+  for (int n = 0; n < NB; ++n) acc[n] = floatx16_t{};
+  GroupRegs32 slot[D];
+#pragma unroll
+  for (int q = 0; q < D; ++q) {
+    load_group(slot[q], q);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // Step g: the products of group g, with the dequantisation of group g + 1 between them
+  // (its words were transposed a step earlier), the transpose of group g + 2, and the loads of
+  // group g + D in group g's registers.  Groups past the last are copies of it and are
+  // dropped.
+  Frags cur, nxt;
+  write_tr(slot[0], 0);
+  fragments(cur, slot[0].sp, 0);
+  write_tr(slot[1], 1);
+  auto step = [&](GroupRegs32& r, const GroupRegs32& r1, const GroupRegs32& r2, int par, int g,
+                  const Frags& f, Frags& n) {
+    const bf16x8_t A[2] = {__builtin_bit_cast(bf16x8_t, r.a0), __builtin_bit_cast(bf16x8_t, r.a1)};
+    write_tr(r2, par);
+    fragments(n, r1.sp, par ^ 1);
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[b] = mfma(A[e], f.b[b][e], acc[b]);
+    constexpr int kV = (NB == 2 ? 84 : 44) / (2 * NB) + 1;
+#pragma unroll
+    for (int i = 0; i < 2 * NB; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x2, kV, 0);
+    }
+    load_group(r, g + D);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int g = 0;
+  for (; g + D <= groups; g += D) {
+#pragma unroll
+    for (int q = 0; q < D; q += 2) {
+      step(slot[q], slot[q + 1], slot[(q + 2) % D], 0, g + q, cur, nxt);
+      step(slot[q + 1], slot[(q + 2) % D], slot[(q + 3) % D], 1, g + q + 1, nxt, cur);
     }
   }
 #pragma unroll
-  for (int q = 0; q < D - 1; ++q) {
-    if (g + q < g1) {
-      if (q + 1 < D - 1 && g + q + 1 < g1) write_tr(slot[q + 1], (q + 1) & 1);
-      compute_group(slot[q], q & 1);
-    }
+  for (int q = 0; q < D - 1; q += 2) {
+    if (g + q < groups) step(slot[q], slot[q + 1], slot[(q + 2) % D], 0, g + q, cur, nxt);
+    if (g + q + 1 < groups)
+      step(slot[q + 1], slot[(q + 2) % D], slot[(q + 3) % D], 1, g + q + 1, nxt, cur);
   }
 
   float* s_red = reinterpret_cast<float*>(s_mem);
   __syncthreads();  // every wave is done with its slots
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    s_red[(wave * 32 + i) * 64 + lane] = accx[i];
-    s_red[(wave * 32 + 16 + i) * 64 + lane] = accy[i];
-  }
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s_red[((wave * NB + b) * 16 + i) * 64 + lane] = acc[b][i];
   __syncthreads();
 
   const int col0 = (c >> 3) * 16 + (c & 7);
   for (int j = wave; j < 32; j += kWaves) {
-    float sg = 0.0f, su = 0.0f;
-#pragma unroll
-    for (int w = 0; w < WK; ++w) {
-      sg += s_red[(w * 32 + j) * 64 + lane];
-      if constexpr (kPair) su += s_red[((WK + w) * 32 + j) * 64 + lane];
-    }
     const int rsid = s_sid[acc_row(j & 15, h)];
     if (static_cast<unsigned>(rsid) >= static_cast<unsigned>(valid_limit)) continue;
-    const int col = (blockIdx.x % n_units) * 64 + col0 + (j < 16 ? 0 : 8);
-    if constexpr (kPair)
+    const int col = blockIdx.x * 64 + col0 + (j < 16 ? 0 : 8);
+    const float sg = s_red[j * 64 + lane];
+    if constexpr (kPair) {
+      const float su = s_red[(32 + j) * 64 + lane];
       p.act[static_cast<long long>(rsid) * p.inter + col] =
           swiglu_one(bf2f(f2bf(sg)), bf2f(f2bf(su)));
-    else if (p.partial)
-      p.partial[(static_cast<long long>(split) * valid_limit + rsid) * N + col] = sg;
-    else
+    } else {
       p.output[static_cast<long long>(rsid) * N + col] = epilogue_value(sg, rsid, p);
+    }
   }
 }
 
@@ -819,12 +857,7 @@ constexpr int kDecodeDepth = 4;
 // its extra scale work cost C1/C2 2-4%).
 template <int WK>
 void launch_decode(const GemmArgs& args, int max_m_blocks, hipStream_t stream) {
-  const dim3 grid(args.size_n / 64 * args.splits, max_m_blocks, ceil_div(args.bs, 32));
-  if (args.bs > 16) {
-    hipLaunchKernelGGL((wna16_decode32_kernel<WK, kDecodeDepth>), grid, dim3(64 * WK), 0, stream,
-                       args);
-    return;
-  }
+  const dim3 grid(args.size_n / 64 * args.splits, max_m_blocks);
   if constexpr (WK == 4) {
     hipLaunchKernelGGL((wna16_decode16_kernel<WK, kDecodeDepth>), grid, dim3(64 * WK), 0, stream,
                        args);
@@ -840,12 +873,7 @@ void launch_decode(const GemmArgs& args, int max_m_blocks, hipStream_t stream) {
 
 template <int WK>
 void launch_decode_pair(const GemmArgs& args, int max_m_blocks, hipStream_t stream) {
-  const dim3 grid(args.inter / 64, max_m_blocks, ceil_div(args.bs, 32));
-  if (args.bs > 16) {
-    hipLaunchKernelGGL((wna16_decode32_kernel<WK, kDecodeDepth, true>), grid, dim3(128 * WK), 0,
-                       stream, args);
-    return;
-  }
+  const dim3 grid(args.inter / 64, max_m_blocks);
   if constexpr (WK == 4) {
     hipLaunchKernelGGL((wna16_decode16_kernel<WK, kDecodeDepth, true>), grid, dim3(128 * WK), 0,
                        stream, args);
@@ -857,6 +885,27 @@ void launch_decode_pair(const GemmArgs& args, int max_m_blocks, hipStream_t stre
       hipLaunchKernelGGL((wna16_decode_kernel<WK, 8, kDecodeDepth, true>), grid, dim3(128 * WK),
                          0, stream, args);
   }
+}
+
+// W13 + SwiGLU with args.act, else the plain GEMM.  Two waves a column tile in a plain GEMM
+// where one expert's 32-row parts and tiles (units) are at most three quarters of the CUs, so
+// that each has a CU to itself (2048 x 7168, 64 rows, 64 units: 39 us against 56 with one wave; 9728 x
+// 2560, 17 rows, 152 units, 17.3 against 23.9; 64 rows, 304 units, 31.3 against 26.0).
+// W13 + SwiGLU has its two waves already (7168 x 2048 expert, 64 rows, both GEMMs, 74 us; with
+// four waves 88).
+void launch_few_rows(const GemmArgs& args, int max_m_blocks, int cu_count, hipStream_t stream) {
+  constexpr int D = 6;
+  const int z = ceil_div(args.bs, 32);
+  const auto go = [&](auto kernel, int tiles, int waves) {
+    hipLaunchKernelGGL(kernel, dim3(tiles, max_m_blocks, z), dim3(64 * waves), 0, stream, args);
+  };
+  const long long rows = static_cast<long long>(args.size_m) * args.top_k;
+  if (args.act != nullptr)
+    go(wna16_decode32_kernel<D, true, 1>, args.inter / 64, 2);
+  else if (args.num_experts == 1 && (rows + 31) / 32 * (args.size_n / 64) * 4 <= 3LL * cu_count)
+    go(wna16_decode32_kernel<D, false, 2>, args.size_n / 64, 2);
+  else
+    go(wna16_decode32_kernel<D, false, 1>, args.size_n / 64, 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -1209,6 +1258,7 @@ constexpr int kPfScanSlab = 1024;  // block experts staged in LDS per scan pass
 // blocks, block order.
 template <int R>
 __device__ __forceinline__ void prefill_block(const GemmArgs& p, int tx, int ty) {
+  __builtin_amdgcn_s_setprio(1);  // ahead of the few-rows kernel's waves (see there)
   __shared__ __align__(1024) uint8_t smem[pf_ring_bytes(R)];
   __shared__ int s_sid[R];
   __shared__ float s_tw[R];  // with mul: the row's top-k weight rounded to bf16
@@ -1474,13 +1524,6 @@ bool few_rows(long long routes, long long experts, int n_tiles, int cu_count) {
   if (experts == 1) return routes <= 128 && (routes + 31) / 32 * n_tiles <= 3LL * cu_count;
   return mean_rows_at_most(routes, experts, 6);
 }
-// K shares (waves per column tile) of that form: four once the tiles of the 32-row
-// parts fill half the GPU's workgroup slots, else eight.
-int few_rows_waves(long long routes, long long experts, int n_tiles, int cu_count) {
-  const long long parts = experts == 1 ? (routes + 31) / 32 : std::min(routes, experts);
-  return parts * n_tiles >= 2LL * cu_count ? 4 : 8;
-}
-
 // The kernels address one expert's weights and the activations through
 // 32-bit buffer ranges.  The activation range must also stay at or below
 // 2^31 bytes: offset 0x80000000 is how rows not routed here read zeros.
@@ -1549,10 +1592,7 @@ int wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long long 
   if (max_m_blocks > 65535) return fail(kNotSupported, "wna16_gemm: too many m-blocks");
   const long long rows = static_cast<long long>(size_m) * top_k;
   if (few_rows(rows, local_experts, n_tiles, cu_count)) {
-    if (few_rows_waves(rows, local_experts, n_tiles, cu_count) == 4)
-      launch_decode<4>(args, max_m_blocks, stream);
-    else
-      launch_decode<8>(args, max_m_blocks, stream);
+    launch_few_rows(args, max_m_blocks, cu_count, stream);
     return launch_status("wna16_gemm (few rows)");
   }
   const dim3 grid(ceil_div(n_tiles, 4), max_m_blocks);
@@ -1611,10 +1651,7 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
     if (cu_count <= 0) return fail(kInvalidValue, "w13_swiglu: no device");
     const long long rows = static_cast<long long>(size_m) * top_k;
     if (few_rows(rows, local_experts, size_n / 64, cu_count)) {
-      if (few_rows_waves(rows, local_experts, size_n / 64, cu_count) == 4)
-        launch_decode_pair<4>(args, max_m_blocks, stream);
-      else
-        launch_decode_pair<8>(args, max_m_blocks, stream);
+      launch_few_rows(args, max_m_blocks, cu_count, stream);
       return launch_status("w13_swiglu (few rows)");
     }
     const dim3 grid(ceil_div(inter / 64, 2), max_m_blocks);

@@ -548,6 +548,48 @@ def test_few_rows_form_exact(oracle, E, T, topk, bs, N, K, mul):
     assert (host(act)[~local] == 0x4040).all()
 
 
+@pytest.mark.parametrize("E,T,topk,bs,N,K", [
+    (1, 20, 1, 64, 1024, 7168), (1, 33, 1, 64, 2048, 2048), (1, 128, 1, 48, 640, 1088),
+    (48, 100, 8, 32, 512, 2048), (6, 30, 1, 32, 256, 4160)])
+def test_few_rows_form_gives_the_tile_kernels_bits(oracle, E, T, topk, bs, N, K):
+    """The few-rows form and the tile kernel add each sum in the same order: ordinary inputs
+    (sums that round) through the rule's form and through the tile kernel, which a launch over
+    more tokens selects (no id reaches the further ones), give the same bits, both for the
+    plain GEMM and for W13 + SwiGLU."""
+    from pegainfer_amd import _lib, ops
+    g = np.random.default_rng(E * 1000 + T + K)
+    q = g.integers(-8, 8, size=(E, N, K))
+    scale_bits = oracle.f32_to_bf16(np.abs(g.standard_normal((E, N, K // 32)) * 0.01)
+                                    .astype(np.float32))
+    a = dev(oracle.f32_to_bf16(g.standard_normal((T, K)).astype(np.float32)))
+    idx = g.integers(0, 8 * E if E > 1 else 1, size=(T, topk)).astype(np.int32)
+    tw = dev(g.random((T, topk)).astype(np.float32))
+    w, _ = _setup(E, N, K, q, scale_bits)
+    ws = ops.KimiMarlinRouteWorkspace(T, bs, topk=topk, local_experts=E)
+    r = ops.moe_align_block_size(ws, dev(idx.reshape(-1)), T, T, 0)
+    stream = torch.cuda.current_stream().cuda_stream
+    wide = 129 if E == 1 else 6 * E * 8 // topk + 8  # past every few-rows rule
+    x = torch.zeros(wide, K, dtype=torch.bfloat16, device="cuda")
+    x[:T] = a
+    outs = []
+    for rows in (T, wide):
+        out = torch.full((rows * topk, N), 7.0, dtype=torch.bfloat16, device="cuda")
+        act = torch.full((rows * topk, N // 2), 7.0, dtype=torch.bfloat16, device="cuda")
+        s = r.sorted_token_ids.clone()
+        s[s == T * topk] = rows * topk  # the padding's id
+        _lib.call("pega_wna16_gemm", x.data_ptr(), out.data_ptr(), None, 0,
+                  w.weight_packed_uint4b8.data_ptr(), w.weight_scale_permuted.data_ptr(), None, 0,
+                  s.data_ptr(), r.expert_ids.data_ptr(), r.num_tokens_post_padded.data_ptr(),
+                  tw.data_ptr(), s.numel(), bs, topk, False, rows, N, K, E, 32, 0, stream)
+        _lib.call("pega_wna16_w13_swiglu", x.data_ptr(), act.data_ptr(), None, 0,
+                  w.weight_packed_uint4b8.data_ptr(), w.weight_scale_permuted.data_ptr(),
+                  s.data_ptr(), r.expert_ids.data_ptr(), r.num_tokens_post_padded.data_ptr(),
+                  s.numel(), bs, topk, rows, N // 2, K, E, 32, 0, stream)
+        outs.append((host(out)[:T * topk], host(act)[:T * topk]))
+    assert np.array_equal(outs[0][0], outs[1][0])
+    assert np.array_equal(outs[0][1], outs[1][1])
+
+
 @pytest.mark.parametrize("R_rows", [1, 32, 33, 64, 65, 96, 97, 128, 129])
 @pytest.mark.parametrize("K", [64, 128, 192, 320, 512])
 def test_tile_kernel_rows_and_chunks_exact(oracle, R_rows, K):
