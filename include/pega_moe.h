@@ -131,9 +131,9 @@ int pega_wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long 
  * are), and the W13 output never reaches HBM.  The bits are the pair's whenever both add the
  * fp32 products over the same K shares: always at block sizes 32-64 (both take the same form
  * and the same split of K), and at block sizes 8/16 when the launch expects at least two (block,
- * 64-column tile) units per CU, or four on a 48-expert share, and K is at least 512 (the Kimi
- * decode layer from 16 tokens on, for one).  A launch expects one block per route, and one per
- * eight routes on a 48-expert share.  Otherwise the shares differ (the K split below, or 8
+ * 64-column tile) units per CU, or four on an expert-parallel share, and K is at least 512 (the
+ * Kimi decode layer from 16 tokens on, for one).  A launch expects one block per route (per
+ * ep_size routes in the _ep form below).  Otherwise the shares differ (the K split below, or 8
  * waves where the GEMM runs 16), and the sums may differ from the pair's in the last fp32
  * bit, within the same summation error bound.
  *  - Block size 8 or 16 (decode): when the (block, tile) units are too few to fill the GPU
@@ -154,6 +154,20 @@ int pega_wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials,
                           int sorted_token_ids_len, int moe_block_size, int top_k, int size_m,
                           int intermediate_dim, int size_k, int local_experts, int group_size,
                           int sm_count, hipStream_t stream);
+
+/* The same where the experts are one GPU's of ep_size (at least 1, which is the entry above)
+ * that the routes are spread over: the launch rules then expect one route in ep_size to be
+ * local.  The outputs are the entry's above within the bound stated there.
+ * kimi_marlin_wna16_gemm_cuda, whose 48 experts are one GPU's of eight, expects that by
+ * itself; pega_wna16_gemm takes every route to be local, and so do both for an expert-major
+ * launch (sorted_token_ids_len <= size_m * top_k). */
+int pega_wna16_w13_swiglu_ep(const uint16_t* input, uint16_t* act, float* partials,
+                             long long partials_len, const uint8_t* b_qweight,
+                             const uint16_t* b_scales, const int32_t* sorted_token_ids,
+                             const int32_t* expert_ids, const int32_t* num_tokens_post_padded,
+                             int sorted_token_ids_len, int moe_block_size, int top_k, int size_m,
+                             int intermediate_dim, int size_k, int local_experts, int ep_size,
+                             int group_size, int sm_count, hipStream_t stream);
 
 /* No reference counterpart; for callers that cannot allocate (code under HIP graph capture,
  * serving loops and harnesses that forbid hipMalloc): pega_wna16_w13_swiglu without the

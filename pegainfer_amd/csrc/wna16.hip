@@ -154,10 +154,7 @@ struct GemmArgs {
                     // instead of the bf16 output (finished by the consumer kernel)
   uint16_t* act;    // prefill, non-null: W13 + SwiGLU, act[sid][inter] instead of the output
   int inter;        // with act: gate columns [0, inter), up columns [inter, 2 inter)
-  // 16-row decode kernel at block size 8: pair the blocks of an expert
-  __host__ __device__ bool pair_blocks() const {
-    return bs == 8 && static_cast<long long>(size_m) * top_k >= 4LL * num_experts;
-  }
+  bool pair_blocks = false;  // 16-row decode kernel: pair the blocks of an expert's run
 };
 
 __device__ __forceinline__ uint16_t epilogue_value(float acc, int sid, const GemmArgs& p) {
@@ -480,7 +477,7 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 6) void wna16_decode16_k
   if (tid < 16 && mb * p.bs + tid < p.sorted_len) sid = p.sorted_ids[mb * p.bs + tid];
   const int expert = __builtin_amdgcn_readfirstlane(p.expert_ids[mb]);
   // with paired blocks, the experts of this block and the 63 before it and of the next
-  const bool paired = p.pair_blocks();
+  const bool paired = p.pair_blocks;
   const int before = paired ? p.expert_ids[max(mb - lane, 0)] : expert;
   const int after = paired ? p.expert_ids[min(mb + 1, m_blocks - 1)] : -1;
   const int ntp = min(p.ntp[0], p.sorted_len);
@@ -1473,17 +1470,26 @@ __global__ void w13_swiglu_partials_kernel(GemmArgs p, uint16_t* __restrict__ ac
 
 bool valid_block_size(int bs) { return bs == 8 || (bs >= 16 && bs <= 64 && bs % 16 == 0); }
 
-// Whether the routes of a launch come to at most `rows` rows per expert on average.  A
-// launch sees every token's routes; 48 local experts are the EP8 share of a 384-expert
-// model (the only share the kimi_* entry points accept), which gets an eighth of them.
-bool mean_rows_at_most(long long routes, long long experts, long long rows) {
-  return routes <= rows * experts * (experts == 48 ? 8 : 1);
+// What share of a launch's routes falls on its experts is not in the routing's sizes, so the
+// rules below count an expected `ep`-th of them: 8 where the caller says that the experts are
+// one GPU's of eight (kimi_marlin_wna16_gemm_cuda, whose 48 of 384 experts are that by
+// definition, and pega_wna16_w13_swiglu_ep), else 1.  An expert-major launch (identity ids, so
+// no room for padding beyond its rows) holds local rows alone, whoever issues it.
+int expected_share(int ep, int sorted_len, long long routes) { return sorted_len > routes ? ep : 1; }
+
+// Whether the routes of a launch come to at most `rows` rows per expert on average.
+bool mean_rows_at_most(long long routes, long long experts, int ep, long long rows) {
+  return routes <= rows * experts * ep;
 }
 
-// Blocks that a decode launch is expected to find work for: at most one per route, and an
-// eighth of that on a 48-expert share.
-long long live_blocks(long long routes, long long experts, long long max_m_blocks) {
-  return std::min(experts == 48 ? (routes + 7) / 8 : routes, max_m_blocks);
+// Blocks that a decode launch is expected to find work for: at most one per local route.
+long long live_blocks(long long routes, int ep, long long max_m_blocks) {
+  return std::min((routes + ep - 1) / ep, max_m_blocks);
+}
+
+// The 16-row decode kernel's two blocks a workgroup, from four local routes per expert on.
+bool pair_blocks(int bs, long long routes, int experts, int ep) {
+  return bs == 8 && routes >= 4LL * experts * ep;
 }
 
 // Waves that share a workgroup's K: four from a workgroup per CU on, more below that, where
@@ -1499,13 +1505,13 @@ int decode_waves(long long wgs, int cu_count) {
 // routes come to few rows per expert, else 128.  Few rows per expert leave the
 // 128-row tiles mostly one or two 32-row blocks anyway, while a problem's large
 // experts (a shared expert in the same pair launch) would get tiles twice as long
-// as the rest, which then set the launch's last round.  An eighth share's mean is
+// as the rest, which then set the launch's last round.  A share's mean is
 // only expected, and skewed routing fills some experts far past it, so there the
 // line is lower: Kimi's MoE block at 1000 tokens (21 rows) 473 us with 64-row tiles
 // against 491, its routed experts under Zipf routing 381 against 393; at 1500 tokens
 // (31 rows) 597 against 613, but 460 against 444 under Zipf.
-bool small_prefill_tiles(long long routes, long long experts) {
-  return mean_rows_at_most(routes, experts, experts == 48 ? 24 : 64);
+bool small_prefill_tiles(long long routes, long long experts, int ep) {
+  return mean_rows_at_most(routes, experts, ep, ep > 1 ? 24 : 64);
 }
 
 // Launches at block sizes above 16 that take the decode kernel's 32-row form instead
@@ -1520,9 +1526,9 @@ bool small_prefill_tiles(long long routes, long long experts) {
 //     40 / 90 rows 18 / 23 against 34 / 39 us; 2048 x 7168, 64 rows 27 against 82; 14336 x
 //     4096, 128 rows, 3.5 a CU, 62 against 60).  Up to 128 rows, so that the shared
 //     expert of a prefill chunk stays with the routed experts' launch.
-bool few_rows(long long routes, long long experts, int n_tiles, int cu_count) {
+bool few_rows(long long routes, long long experts, int ep, int n_tiles, int cu_count) {
   if (experts == 1) return routes <= 128 && (routes + 31) / 32 * n_tiles <= 3LL * cu_count;
-  return mean_rows_at_most(routes, experts, 6);
+  return mean_rows_at_most(routes, experts, ep, 6);
 }
 // The kernels address one expert's weights and the activations through
 // 32-bit buffer ranges.  The activation range must also stay at or below
@@ -1538,7 +1544,7 @@ int wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long long 
                int workspace_len, const int32_t* sorted_token_ids, const int32_t* expert_ids,
                const int32_t* num_tokens_post_padded, const float* topk_weights,
                int sorted_token_ids_len, int moe_block_size, int top_k, bool mul_topk_weights,
-               int size_m, int size_n, int size_k, int local_experts, int group_size,
+               int size_m, int size_n, int size_k, int local_experts, int ep, int group_size,
                int cu_count, hipStream_t stream) {
   if (!input || !output || !b_qweight || !b_scales || !sorted_token_ids || !expert_ids ||
       !num_tokens_post_padded || !topk_weights)
@@ -1569,6 +1575,8 @@ int wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long long 
 
   const int max_m_blocks = ceil_div(sorted_token_ids_len, moe_block_size);
   const int n_tiles = size_n / 64;
+  const long long routes = static_cast<long long>(size_m) * top_k;
+  ep = expected_share(ep, sorted_token_ids_len, routes);
   GemmArgs args{input, output, c_tmp, reinterpret_cast<const uint32_t*>(b_qweight), b_scales,
                 workspace, sorted_token_ids, expert_ids, num_tokens_post_padded, topk_weights,
                 sorted_token_ids_len, moe_block_size, top_k, mul_topk_weights ? 1 : 0, size_m,
@@ -1578,8 +1586,8 @@ int wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long long 
     // Decode: one workgroup per (m-block, tile).  Fewer expected workgroups ->
     // more waves per workgroup splitting K, so the chip stays busy.
     const int groups = size_k / 32;
-    const long long routes = static_cast<long long>(size_m) * top_k;
-    const long long est_blocks = live_blocks(routes, local_experts, max_m_blocks);
+    const long long est_blocks = live_blocks(routes, ep, max_m_blocks);
+    args.pair_blocks = pair_blocks(moe_block_size, routes, local_experts, ep);
     const long long wgs = est_blocks * n_tiles;
     int wk = decode_waves(wgs, cu_count);
     while (wk > 4 && groups < wk) wk >>= 1;  // waves past the last group idle
@@ -1590,13 +1598,12 @@ int wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long long 
     return launch_status("wna16_gemm (decode)");
   }
   if (max_m_blocks > 65535) return fail(kNotSupported, "wna16_gemm: too many m-blocks");
-  const long long rows = static_cast<long long>(size_m) * top_k;
-  if (few_rows(rows, local_experts, n_tiles, cu_count)) {
+  if (few_rows(routes, local_experts, ep, n_tiles, cu_count)) {
     launch_few_rows(args, max_m_blocks, cu_count, stream);
     return launch_status("wna16_gemm (few rows)");
   }
   const dim3 grid(ceil_div(n_tiles, 4), max_m_blocks);
-  if (small_prefill_tiles(rows, local_experts))
+  if (small_prefill_tiles(routes, local_experts, ep))
     hipLaunchKernelGGL(wna16_prefill_kernel<64>, grid, dim3(256), 0, stream, args);
   else
     hipLaunchKernelGGL(wna16_prefill_kernel<128>, grid, dim3(256), 0, stream, args);
@@ -1615,7 +1622,8 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
                      const int32_t* sorted_token_ids, const int32_t* expert_ids,
                      const int32_t* num_tokens_post_padded, int sorted_token_ids_len,
                      int moe_block_size, int top_k, int size_m, int inter, int size_k,
-                     int local_experts, int group_size, int cu_count, hipStream_t stream) {
+                     int local_experts, int ep, int group_size, int cu_count,
+                     hipStream_t stream) {
   if (!input || !act || !b_qweight || !b_scales || !sorted_token_ids || !expert_ids ||
       !num_tokens_post_padded)
     return fail(kInvalidValue, "w13_swiglu: null pointer");
@@ -1641,6 +1649,8 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
                 "2 GiB (m=%d inter=%d k=%d)", size_m, inter, size_k);
   const int max_m_blocks = ceil_div(sorted_token_ids_len, moe_block_size);
   if (max_m_blocks > 65535) return fail(kNotSupported, "w13_swiglu: too many m-blocks");
+  const long long routes = static_cast<long long>(size_m) * top_k;
+  ep = expected_share(ep, sorted_token_ids_len, routes);
   if (moe_block_size > 16) {
     // Prefill: the tile GEMM with the SwiGLU epilogue (partials not used).
     GemmArgs args{input, nullptr, nullptr, reinterpret_cast<const uint32_t*>(b_qweight),
@@ -1649,13 +1659,12 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
                   size_k, local_experts, 1, nullptr, act, inter};
     if (cu_count <= 0) cu_count = current_cu_count();
     if (cu_count <= 0) return fail(kInvalidValue, "w13_swiglu: no device");
-    const long long rows = static_cast<long long>(size_m) * top_k;
-    if (few_rows(rows, local_experts, size_n / 64, cu_count)) {
+    if (few_rows(routes, local_experts, ep, size_n / 64, cu_count)) {
       launch_few_rows(args, max_m_blocks, cu_count, stream);
       return launch_status("w13_swiglu (few rows)");
     }
     const dim3 grid(ceil_div(inter / 64, 2), max_m_blocks);
-    if (small_prefill_tiles(rows, local_experts))
+    if (small_prefill_tiles(routes, local_experts, ep))
       hipLaunchKernelGGL(wna16_prefill_kernel<64>, grid, dim3(256), 0, stream, args);
     else
       hipLaunchKernelGGL(wna16_prefill_kernel<128>, grid, dim3(256), 0, stream, args);
@@ -1663,20 +1672,18 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
   }
   if (cu_count <= 0) cu_count = current_cu_count();
   if (cu_count <= 0) return fail(kInvalidValue, "w13_swiglu: no device");
-  const long long routes = static_cast<long long>(size_m) * top_k;
   const int n_tiles = size_n / 64;
   const int groups = size_k / 32;
-  const long long est_blocks = live_blocks(routes, local_experts, max_m_blocks);
+  const long long est_blocks = live_blocks(routes, ep, max_m_blocks);
   const long long wgs = est_blocks * n_tiles;
   // Shares: about two workgroups per CU, at least 8 groups (two per wave) each, as many as
-  // the partials buffer holds.  On a 48-expert share four per CU, since the routes that fall
-  // on it vary, and at most four shares, since most workgroups of its grid find no block
+  // the partials buffer holds.  On an expert-parallel share four per CU, since the routes that
+  // fall on it vary, and at most four shares, since most workgroups of its grid find no block
   // and each share dispatches them again (decode layer at 1 / 3 / 12 tokens: one share 62.5
   // / 69.5 / 98 us, two 55.7 / 62.4 / 96, four 53 / 59.5 / 95, eight 57 / 65 / -).
-  const bool share48 = local_experts == 48;
-  const long long aim = (share48 ? 4LL : 2LL) * cu_count;
+  const long long aim = (ep > 1 ? 4LL : 2LL) * cu_count;
   long long sp = (aim + wgs - 1) / wgs;
-  if (sp > (share48 ? 4 : 16)) sp = share48 ? 4 : 16;
+  if (sp > (ep > 1 ? 4 : 16)) sp = ep > 1 ? 4 : 16;
   if (sp > groups / 8) sp = groups / 8;
   const long long cap = partials ? partials_len / (routes * size_n) : 0;
   if (sp > cap) sp = cap;
@@ -1687,6 +1694,7 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
                   b_scales, nullptr, sorted_token_ids, expert_ids, num_tokens_post_padded,
                   nullptr, sorted_token_ids_len, moe_block_size, top_k, 0, size_m, size_n,
                   size_k, local_experts, 1, nullptr, act, inter};
+    args.pair_blocks = pair_blocks(moe_block_size, routes, local_experts, ep);
     const long long pair_wgs = est_blocks * (inter / 64);
     // As the plain GEMM's from two units per CU on, so that the two give the same bits there
     // (DeepSeek-V2-Lite block at 3 / 8 tokens: 61.2 / 81.6 us with four waves, 63.9 / 81.9
@@ -1702,6 +1710,7 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
                 nullptr, sorted_token_ids, expert_ids, num_tokens_post_padded, nullptr,
                 sorted_token_ids_len, moe_block_size, top_k, 0, size_m, size_n, size_k,
                 local_experts, splits, partials};
+  args.pair_blocks = pair_blocks(moe_block_size, routes, local_experts, ep);
   const long long total_wgs = wgs * splits;
   int wk = decode_waves(total_wgs, cu_count);
   while (wk > 4 && groups / splits < 2 * wk) wk >>= 1;  // keep >= 2 groups per wave
@@ -1779,13 +1788,13 @@ int single_problem(const pega_wna16_problem* q, int cu_count, hipStream_t stream
     return wna16_w13_swiglu(q->input, q->act, nullptr, 0, q->b_qweight, q->b_scales,
                             q->sorted_token_ids, q->expert_ids, q->num_tokens_post_padded,
                             q->sorted_token_ids_len, q->moe_block_size, q->top_k, q->size_m,
-                            q->size_n / 2, q->size_k, q->local_experts, q->group_size, cu_count,
-                            stream);
+                            q->size_n / 2, q->size_k, q->local_experts, 1, q->group_size,
+                            cu_count, stream);
   const float* tw = q->topk_weights ? q->topk_weights : reinterpret_cast<const float*>(q->input);
   return wna16_gemm(q->input, q->output, nullptr, 0, q->b_qweight, q->b_scales, nullptr, 0,
                     q->sorted_token_ids, q->expert_ids, q->num_tokens_post_padded, tw,
                     q->sorted_token_ids_len, q->moe_block_size, q->top_k,
-                    q->mul_topk_weights != 0, q->size_m, q->size_n, q->size_k, q->local_experts,
+                    q->mul_topk_weights != 0, q->size_m, q->size_n, q->size_k, q->local_experts, 1,
                     q->group_size, cu_count, stream);
 }
 
@@ -1804,9 +1813,9 @@ int wna16_prefill_pair(const pega_wna16_problem* first, const pega_wna16_problem
   const int cu_count = current_cu_count();
   if (cu_count <= 0) return fail(kInvalidValue, "wna16_prefill_pair: no device");
   const bool grids_fit = y0 <= 65535 && y1 <= 65535;  // of the single launches
-  if (grids_fit && (few_rows(static_cast<long long>(a0.size_m) * a0.top_k, a0.num_experts,
+  if (grids_fit && (few_rows(static_cast<long long>(a0.size_m) * a0.top_k, a0.num_experts, 1,
                              a0.size_n / 64, cu_count) ||
-                    few_rows(static_cast<long long>(a1.size_m) * a1.top_k, a1.num_experts,
+                    few_rows(static_cast<long long>(a1.size_m) * a1.top_k, a1.num_experts, 1,
                              a1.size_n / 64, cu_count))) {
     rc = single_problem(first, cu_count, stream);
     return rc != kSuccess ? rc : single_problem(second, cu_count, stream);
@@ -1818,7 +1827,7 @@ int wna16_prefill_pair(const pega_wna16_problem* first, const pega_wna16_problem
   const long long routes = static_cast<long long>(a0.size_m) * a0.top_k +
                            static_cast<long long>(a1.size_m) * a1.top_k;
   const dim3 grid(static_cast<unsigned>(n0 + n1));
-  if (small_prefill_tiles(routes, static_cast<long long>(a0.num_experts) + a1.num_experts))
+  if (small_prefill_tiles(routes, static_cast<long long>(a0.num_experts) + a1.num_experts, 1))
     hipLaunchKernelGGL(wna16_prefill_pair_kernel<64>, grid, dim3(256), 0, stream, a0, a1, x0,
                        static_cast<int>(n0), x1);
   else
@@ -1836,6 +1845,10 @@ int wna16_prefill_pair(const pega_wna16_problem* first, const pega_wna16_problem
 // K reduction happens inside each workgroup, so c_tmp and the lock workspace
 // are validated but never read or written (a caller's zero-filled locks stay
 // zero).
+namespace {
+constexpr int kKimiEp = 8;  // the 48 experts are one GPU's of eight (pegainfer-kimi-k2's EP8)
+}  // namespace
+
 PEGA_API int kimi_marlin_wna16_gemm_cuda(
     const uint16_t* input, uint16_t* output, float* c_tmp, const uint8_t* b_qweight,
     const uint16_t* b_scales, int32_t* workspace, const int32_t* sorted_token_ids,
@@ -1876,8 +1889,8 @@ PEGA_API int kimi_marlin_wna16_gemm_cuda(
   return pega::wna16_gemm(input, output, c_tmp, c_tmp_len, b_qweight, b_scales, workspace,
                           workspace_len, sorted_token_ids, expert_ids, num_tokens_post_padded,
                           topk_weights, sorted_token_ids_len, moe_block_size, top_k,
-                          mul_topk_weights, size_m, size_n, size_k, local_experts, group_size,
-                          sm_count, stream);
+                          mul_topk_weights, size_m, size_n, size_k, local_experts, kKimiEp,
+                          group_size, sm_count, stream);
 }
 
 // Shape-general entry (any expert count; expert ids outside [0, local_experts)
@@ -1895,7 +1908,7 @@ PEGA_API int pega_wna16_gemm(const uint16_t* input, uint16_t* output, float* c_t
   return pega::wna16_gemm(input, output, c_tmp, c_tmp_len, b_qweight, b_scales, workspace,
                           workspace_len, sorted_token_ids, expert_ids, num_tokens_post_padded,
                           topk_weights, sorted_token_ids_len, moe_block_size, top_k,
-                          mul_topk_weights, size_m, size_n, size_k, local_experts, group_size,
+                          mul_topk_weights, size_m, size_n, size_k, local_experts, 1, group_size,
                           sm_count, stream);
 }
 
@@ -1912,8 +1925,27 @@ PEGA_API int pega_wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* 
   return pega::wna16_w13_swiglu(input, act, partials, partials_len, b_qweight, b_scales,
                                 sorted_token_ids, expert_ids, num_tokens_post_padded,
                                 sorted_token_ids_len, moe_block_size, top_k, size_m,
-                                intermediate_dim, size_k, local_experts, group_size, sm_count,
+                                intermediate_dim, size_k, local_experts, 1, group_size, sm_count,
                                 stream);
+}
+
+// The same where the experts are one GPU's of `ep_size` that the routes are spread over.
+PEGA_API int pega_wna16_w13_swiglu_ep(const uint16_t* input, uint16_t* act, float* partials,
+                                      long long partials_len, const uint8_t* b_qweight,
+                                      const uint16_t* b_scales, const int32_t* sorted_token_ids,
+                                      const int32_t* expert_ids,
+                                      const int32_t* num_tokens_post_padded,
+                                      int sorted_token_ids_len, int moe_block_size, int top_k,
+                                      int size_m, int intermediate_dim, int size_k,
+                                      int local_experts, int ep_size, int group_size,
+                                      int sm_count, hipStream_t stream) {
+  if (ep_size < 1)
+    return pega::fail(pega::kInvalidValue, "w13_swiglu: ep_size %d is below 1", ep_size);
+  return pega::wna16_w13_swiglu(input, act, partials, partials_len, b_qweight, b_scales,
+                                sorted_token_ids, expert_ids, num_tokens_post_padded,
+                                sorted_token_ids_len, moe_block_size, top_k, size_m,
+                                intermediate_dim, size_k, local_experts, ep_size, group_size,
+                                sm_count, stream);
 }
 
 // ---------------------------------------------------------------- no-allocation variant
@@ -1983,7 +2015,7 @@ PEGA_API int pega_wna16_w13_swiglu_noalloc(const uint16_t* input, uint16_t* act,
   return pega::wna16_w13_swiglu(input, act, partials, kScratchFloats, b_qweight, b_scales,
                                 sorted_token_ids, expert_ids, num_tokens_post_padded,
                                 sorted_token_ids_len, moe_block_size, top_k, size_m,
-                                intermediate_dim, size_k, local_experts, group_size, sm_count,
+                                intermediate_dim, size_k, local_experts, 1, group_size, sm_count,
                                 stream);
 }
 

@@ -47,8 +47,11 @@ class RoutedExperts:
 
     def __init__(self, w13: ops.MarlinInt4Weight, w2: ops.MarlinInt4Weight, *, max_tokens: int,
                  topk: int, block_size: int, global_start: int = 0, device="cuda",
-                 extra_splits: int = 1):
+                 extra_splits: int = 1, ep_size: int = None):
+        """ep_size: GPUs that the routes' experts are spread over, where that is not Kimi's
+        eight (48 experts, top-8) or this GPU alone (any other share)."""
         self.w13, self.w2 = w13, w2
+        self.ep_size = ep_size
         self.E = w13.local_experts
         self.H = w13.in_dim
         self.I = w13.out_dim // 2
@@ -83,8 +86,8 @@ class RoutedExperts:
         non-local routes) and fuses SwiGLU into W13.  The two give the same bits
         whenever the fused and the plain W13 add over the same K shares (prefill
         block sizes; decode grids that expect two or more W13 (block, tile) units
-        per CU, four on a 48-expert share, with K >= 512); a small decode grid splits K differently, and a W13 sum may then
-        differ in the last fp32 bit.
+        per CU, four on an expert-parallel share, with K >= 512); a small decode grid
+        splits K differently, and a W13 sum may then differ in the last fp32 bit.
         `w13_timer` (optional) exposes start()/stop(mark) and is called around the
         W13 GEMM launch so a caller can time that kernel with stream events.
         `companion` (optional, prefill block sizes only): a (W13, W2) pair of
@@ -116,12 +119,13 @@ class RoutedExperts:
             # SwiGLU in the W13 epilogue (gate and up tiles in one workgroup), routed rows
             # only
             ops.wna16_w13_swiglu(self.gemm_ws, routing, hidden, self.w13, act, top_k=self.topk,
-                                 size_m=T)
+                                 size_m=T, ep_size=self.ep_size)
             if w13_timer is not None:
                 w13_timer.stop(mark)
         else:
             ops.wna16_gemm(self.gemm_ws, routing, hidden, self.w13, topk_w, w13_out,
-                           top_k=self.topk, mul_topk_weights=False, size_m=T)
+                           top_k=self.topk, mul_topk_weights=False, size_m=T,
+                           ep_size=self.ep_size)
             if w13_timer is not None:
                 w13_timer.stop(mark)
             ops.kimi_marlin_w13_swiglu(w13_out, act, rows, self.I)
@@ -134,7 +138,7 @@ class RoutedExperts:
                 topk_weight=topk_w, mul_topk_weights=weighted_in_gemm))
         else:
             ops.wna16_gemm(self.gemm_ws, routing, act, self.w2, topk_w, route_out, top_k=1,
-                           mul_topk_weights=weighted_in_gemm, size_m=rows)
+                           mul_topk_weights=weighted_in_gemm, size_m=rows, ep_size=self.ep_size)
         if reference_flow:
             if weighted_in_gemm:
                 ops.kimi_marlin_sum_topk_rows_f32(route_out, T, out_f32, self.topk, self.H)

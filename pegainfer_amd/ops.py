@@ -383,11 +383,24 @@ class KimiMarlinWna16Workspace:
         self.c_tmp = torch.zeros(max(1, c_tmp), dtype=torch.float32, device=device)
 
 
+def _ep_size(routing: KimiMarlinRouting, weight: MarlinInt4Weight, ep_size) -> int:
+    """GPUs that the routes' experts are spread over: the launch rules expect one route in
+    ep_size to be local.  Kimi's share (48 experts, top-8) is one GPU's of eight; any other
+    routing is taken to be all local unless the caller says otherwise."""
+    if ep_size is not None:
+        _ensure(ep_size >= 1, f"ep_size must be >= 1, got {ep_size}")
+        return ep_size
+    kimi = weight.local_experts == KIMI_K2_LOCAL_EXPERTS and routing.topk == KIMI_K2_TOPK
+    return KIMI_K2_EP_WORLD if kimi else 1
+
+
 def wna16_gemm(workspace: KimiMarlinWna16Workspace, routing: KimiMarlinRouting,
                input: torch.Tensor, weight: MarlinInt4Weight, topk_weight: torch.Tensor,
-               output: torch.Tensor, *, top_k: int, mul_topk_weights: bool, size_m: int) -> None:
+               output: torch.Tensor, *, top_k: int, mul_topk_weights: bool, size_m: int,
+               ep_size: int = None) -> None:
     """C[sorted_id] = bf16(A[sorted_id / top_k] . dequant(W[expert]))  (optionally
-    times bf16(topk_weight[sorted_id])).  Rows not routed here are left as they are."""
+    times bf16(topk_weight[sorted_id])).  Rows not routed here are left as they are.
+    `ep_size`: see _ep_size (48 experts of eight GPUs go through the reference symbol)."""
     size_n, size_k = weight.out_dim, weight.in_dim
     _ensure(workspace.block_size == routing.block_size,
             f"Kimi Marlin WNA16 workspace block_size {workspace.block_size} must match routing "
@@ -400,7 +413,10 @@ def wna16_gemm(workspace: KimiMarlinWna16Workspace, routing: KimiMarlinRouting,
     _ensure(topk_weight.dtype == torch.float32, "topk_weight must be float32")
     _ensure(_is_bf16(input) and _is_bf16(output), "input/output must be bf16")
     weight.validate()
-    kimi = weight.local_experts == KIMI_K2_LOCAL_EXPERTS
+    # an expert-major routing (the reference's expanded path) holds local rows alone
+    kimi = weight.local_experts == KIMI_K2_LOCAL_EXPERTS and (
+        routing.max_padded_tokens <= size_m * top_k
+        or _ep_size(routing, weight, ep_size) == KIMI_K2_EP_WORLD)
     if kimi:
         _lib.call("kimi_marlin_wna16_gemm_cuda", _ptr(input), _ptr(output), _ptr(workspace.c_tmp),
                   _ptr(weight.weight_packed_uint4b8), _ptr(weight.weight_scale_permuted),
@@ -422,24 +438,27 @@ def wna16_gemm(workspace: KimiMarlinWna16Workspace, routing: KimiMarlinRouting,
 
 def wna16_w13_swiglu(workspace: KimiMarlinWna16Workspace, routing: KimiMarlinRouting,
                      input: torch.Tensor, weight: MarlinInt4Weight, act: torch.Tensor, *,
-                     top_k: int, size_m: int, split_k: bool = True) -> None:
+                     top_k: int, size_m: int, split_k: bool = True,
+                     ep_size: int = None) -> None:
     """act[sorted_id] = SwiGLU(bf16(A[sorted_id / top_k] . dequant(W13[expert]))) in one
     call, routed rows only.  Block sizes 8/16: when too few workgroups would fill the GPU,
     K is split across workgroups and the partials (the workspace's c_tmp) are summed by the
     SwiGLU kernel; otherwise (or with split_k=False) a gate tile and its up tile share a
-    workgroup with SwiGLU in the epilogue.  32/48/64: the tile GEMM with a SwiGLU epilogue."""
+    workgroup with SwiGLU in the epilogue.  32/48/64: the tile GEMM with a SwiGLU epilogue.
+    `ep_size`: see _ep_size."""
     inter = weight.out_dim // 2
     _ensure(workspace.block_size == routing.block_size, "workspace / routing block size differ")
     _ensure(2 * inter <= workspace.max_size_n, "W13 width exceeds the workspace")
     _ensure(act.dtype == torch.bfloat16 and act.numel() >= size_m * top_k * inter,
             "act must be bf16 [size_m * top_k, inter]")
-    _lib.call("pega_wna16_w13_swiglu", _ptr(input), _ptr(act),
+    _lib.call("pega_wna16_w13_swiglu_ep", _ptr(input), _ptr(act),
               _ptr(workspace.c_tmp) if split_k else None,
               workspace.c_tmp.numel() if split_k else 0, _ptr(weight.weight_packed_uint4b8),
               _ptr(weight.weight_scale_permuted), _ptr(routing.sorted_token_ids),
               _ptr(routing.expert_ids), _ptr(routing.num_tokens_post_padded),
               routing.sorted_token_ids.numel(), routing.block_size, top_k, size_m, inter,
-              weight.in_dim, weight.local_experts, 32, 0, _stream())
+              weight.in_dim, weight.local_experts, _ep_size(routing, weight, ep_size), 32, 0,
+              _stream())
 
 
 def wna16_problem(routing: KimiMarlinRouting, input: torch.Tensor, weight: MarlinInt4Weight, *,

@@ -644,3 +644,59 @@ def test_decode_merges_blocks_of_eight_rows(oracle):
                             moe_block_size=bs, top_k=1, mul_topk_weights=False, size_m=T, size_n=N,
                             size_k=K, output=np.full((T, N), 0x40E0, np.uint16), threads=8)
     assert np.array_equal(host(out), ref)
+
+
+def test_expert_parallel_share_is_said_not_inferred(oracle):
+    """Whether a launch's routes are an eighth local is the caller's to say.  W13 + SwiGLU of
+    three tokens over 48 experts: all local (the shape-general entry, an expert-major launch
+    and an ep_size of 1) there are workgroups enough without a K split, so the partials buffer
+    stays as it was; on Kimi's share (ep_size 8, and the Python op on Kimi's routing) K is
+    split through it.  Exact inputs: the same bits either way."""
+    from pegainfer_amd import _lib, ops
+    g = np.random.default_rng(48)
+    E, T, topk, bs, N, K = 48, 3, 8, 8, 4096, 1024
+    q = g.integers(-8, 8, size=(E, N, K))
+    scale_bits = oracle.f32_to_bf16(
+        (2.0 ** g.integers(-6, -2, size=(E, N, K // 32))).astype(np.float32))
+    a = dev(oracle.f32_to_bf16(g.integers(-2, 3, size=(T * topk, K)).astype(np.float32)))
+    w, _ = _setup(E, N, K, q, scale_bits)
+    ws = ops.KimiMarlinRouteWorkspace(T, bs, topk=topk, local_experts=E)
+    idx = np.stack([g.permutation(E)[:topk] for _ in range(T)]).astype(np.int32)
+    r = ops.moe_align_block_size(ws, dev(idx.reshape(-1)), T, T, 0)
+    gws = ops.KimiMarlinWna16Workspace(ws.max_m_blocks, N, bs)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def run(ep, sorted_ids, tokens, k):
+        gws.c_tmp.fill_(float("nan"))
+        act = torch.zeros(tokens * k, N // 2, dtype=torch.bfloat16, device="cuda")
+        args = [a.data_ptr(), act.data_ptr(), gws.c_tmp.data_ptr(), gws.c_tmp.numel(),
+                w.weight_packed_uint4b8.data_ptr(), w.weight_scale_permuted.data_ptr(),
+                sorted_ids.data_ptr(), r.expert_ids.data_ptr(),
+                r.num_tokens_post_padded.data_ptr(), sorted_ids.numel(), bs, k, tokens, N // 2, K,
+                E]
+        if ep is None:
+            _lib.call("pega_wna16_w13_swiglu", *args, 32, 0, stream)
+        else:
+            _lib.call("pega_wna16_w13_swiglu_ep", *args, ep, 32, 0, stream)
+        return host(act), not bool(torch.isnan(gws.c_tmp).all())
+
+    ref, split = run(None, r.sorted_token_ids, T, topk)
+    assert not split
+    got, split = run(1, r.sorted_token_ids, T, topk)
+    assert not split and np.array_equal(got, ref)
+    got, split = run(8, r.sorted_token_ids, T, topk)
+    assert split and np.array_equal(got, ref)
+    act = torch.zeros(T * topk, N // 2, dtype=torch.bfloat16, device="cuda")
+    for ep, want in ((None, True), (1, False)):
+        gws.c_tmp.fill_(float("nan"))
+        ops.wna16_w13_swiglu(gws, r, a, w, act, top_k=topk, size_m=T, ep_size=ep)
+        assert np.array_equal(host(act), ref)
+        assert bool(torch.isnan(gws.c_tmp).all()) != want
+    # expert-major: identity ids, no room beyond the rows
+    rows = 24
+    ids = torch.arange(rows, dtype=torch.int32, device="cuda")
+    r.expert_ids[:3] = 1
+    r.num_tokens_post_padded.fill_(rows)
+    ref, split = run(None, ids, rows, 1)
+    got, split8 = run(8, ids, rows, 1)
+    assert split8 == split and np.array_equal(got, ref)
