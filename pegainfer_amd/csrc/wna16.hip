@@ -466,7 +466,6 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 6) void wna16_decode16_k
   __shared__ float s_red[kWaves][16][64];
   __shared__ __align__(16) uint32_t s_w[kWaves][2][kSlotDwords];
 
-  __builtin_amdgcn_s_setprio(1);  // ahead of the few-rows kernel's waves (see there)
   const int n_tiles = p.size_n >> 6;
   const int n_units = kPair ? (p.inter >> 6) : n_tiles;
   const int split = blockIdx.x / n_units;
@@ -669,22 +668,19 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 6) void wna16_decode16_k
 // next group is dequantised between this group's MFMAs (one expert, 2048 x 7168 at 64 rows:
 // 56 us without, 72 with the tile kernel; two waves a tile 39).  Kimi's MoE block, 160 tokens
 // (35 experts touched): 245 us against 289 with the tile kernel.
-// The other kernels of this file run at a wave priority of 1: a shared expert in this form
-// beside the routed experts, on another stream, then takes what they leave (DeepSeek-V2-Lite
-// layer at 64 / 100 tokens 106 / 114 us; at equal priority 116 / 126).
 struct GroupRegs32 {
   u32x4_t raw;
   uint32_t sp;
   u32x4_t a0, a1;
 };
 
-// CS = 2: two waves per column tile, one of its n0 columns, one of its n1 columns.
+// CS = 2: two workgroups per column tile, one of its n0 columns, one of its n1 columns.
 template <int D, bool kPair, int CS>
-__global__ __launch_bounds__(64 * (kPair ? 2 : CS), CS == 1 ? 3 : 2)
+__global__ __launch_bounds__(kPair ? 128 : 64, CS == 1 ? 3 : 2)
 void wna16_decode32_kernel(GemmArgs p) {
   static_assert(D % 2 == 0, "the two transpose slots alternate with the ring position");
   static_assert(!(kPair && CS == 2), "a pair has its two waves already");
-  constexpr int kWaves = kPair ? 2 : CS;  // kPair: a gate tile's wave, then its up tile's
+  constexpr int kWaves = kPair ? 2 : 1;  // kPair: a gate tile's wave, then its up tile's
   constexpr int NB = 2 / CS;                    // 32-column MFMAs of a wave
   __shared__ int s_sid[32];
   // the transpose slots ([wave][2][kSlotDwords]), then the sums ([wave][16 NB][64])
@@ -705,8 +701,8 @@ void wna16_decode32_kernel(GemmArgs p) {
   if (ntp < (mb + 1) * p.bs || expert < 0 || expert >= p.num_experts || !routed) return;
 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nt = blockIdx.x + (kPair ? wave * (p.inter >> 6) : 0);
-  const int cs = CS == 2 ? wave : 0;
+  const int tile = blockIdx.x / CS, cs = CS == 2 ? blockIdx.x & 1 : 0;
+  const int nt = tile + (kPair ? wave * (p.inter >> 6) : 0);
   if (tid < 32) s_sid[tid] = sid;
   const int c = lane & 31, h = lane >> 5;
   const int my_sid = __builtin_amdgcn_ds_bpermute(c << 2, sid);
@@ -832,10 +828,10 @@ void wna16_decode32_kernel(GemmArgs p) {
   __syncthreads();
 
   const int col0 = (c >> 3) * 16 + (c & 7);
-  for (int j = wave; j < 32; j += kWaves) {
+  for (int j = wave; j < 16 * NB; j += kWaves) {
     const int rsid = s_sid[acc_row(j & 15, h)];
     if (static_cast<unsigned>(rsid) >= static_cast<unsigned>(valid_limit)) continue;
-    const int col = blockIdx.x * 64 + col0 + (j < 16 ? 0 : 8);
+    const int col = tile * 64 + col0 + (j < 16 && cs == 0 ? 0 : 8);
     const float sg = s_red[j * 64 + lane];
     if constexpr (kPair) {
       const float su = s_red[(32 + j) * 64 + lane];
@@ -884,25 +880,34 @@ void launch_decode_pair(const GemmArgs& args, int max_m_blocks, hipStream_t stre
   }
 }
 
-// W13 + SwiGLU with args.act, else the plain GEMM.  Two waves a column tile in a plain GEMM
-// where one expert's 32-row parts and tiles (units) are at most three quarters of the CUs, so
-// that each has a CU to itself (2048 x 7168, 64 rows, 64 units: 39 us against 56 with one wave; 9728 x
-// 2560, 17 rows, 152 units, 17.3 against 23.9; 64 rows, 304 units, 31.3 against 26.0).
-// W13 + SwiGLU has its two waves already (7168 x 2048 expert, 64 rows, both GEMMs, 74 us; with
-// four waves 88).
+// W13 + SwiGLU with args.act, else the plain GEMM.  Two workgroups a column tile in a plain
+// GEMM where one expert's 32-row parts and tiles (units) are at most three quarters of the CUs,
+// so that each half has a CU to itself (2048 x 7168, 64 rows, 64 units: 36.5 us against 52 with
+// one; 9728 x 2560, 17 rows, 152 units, 16.7 against 22.4; 64 rows, 304 units, 24 either way).
+// Six groups in flight (2048 x 7168 38 us, with four 45), but four where one expert has few
+// units and a short K (2048 x 2048, 17 rows, 15.4 us against 13.5 with six) and in its W13 (2048 x
+// 2816 expert, 17 rows, 42 against 36): such a launch is a layer's shared expert beside its
+// routed ones, which more loads in flight delay (DeepSeek-V2-Lite layer at 24 tokens, weights
+// not in cache, 97.6 us against 100.7).
 void launch_few_rows(const GemmArgs& args, int max_m_blocks, int cu_count, hipStream_t stream) {
-  constexpr int D = 6;
   const int z = ceil_div(args.bs, 32);
   const auto go = [&](auto kernel, int tiles, int waves) {
     hipLaunchKernelGGL(kernel, dim3(tiles, max_m_blocks, z), dim3(64 * waves), 0, stream, args);
   };
-  const long long rows = static_cast<long long>(args.size_m) * args.top_k;
-  if (args.act != nullptr)
-    go(wna16_decode32_kernel<D, true, 1>, args.inter / 64, 2);
-  else if (args.num_experts == 1 && (rows + 31) / 32 * (args.size_n / 64) * 4 <= 3LL * cu_count)
-    go(wna16_decode32_kernel<D, false, 2>, args.size_n / 64, 2);
-  else
-    go(wna16_decode32_kernel<D, false, 1>, args.size_n / 64, 1);
+  const int tiles = args.size_n / 64;
+  const bool one = args.num_experts == 1;
+  const long long units = (static_cast<long long>(args.size_m) * args.top_k + 31) / 32 * tiles;
+  if (args.act != nullptr) {
+    if (one) go(wna16_decode32_kernel<4, true, 1>, args.inter / 64, 2);
+    else go(wna16_decode32_kernel<6, true, 1>, args.inter / 64, 2);
+  } else if (one && units * 4 <= 3LL * cu_count) {
+    if (units <= cu_count / 4 && args.size_k <= 4096)
+      go(wna16_decode32_kernel<4, false, 2>, 2 * tiles, 1);
+    else
+      go(wna16_decode32_kernel<6, false, 2>, 2 * tiles, 1);
+  } else {
+    go(wna16_decode32_kernel<6, false, 1>, tiles, 1);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1255,7 +1260,6 @@ constexpr int kPfScanSlab = 1024;  // block experts staged in LDS per scan pass
 // blocks, block order.
 template <int R>
 __device__ __forceinline__ void prefill_block(const GemmArgs& p, int tx, int ty) {
-  __builtin_amdgcn_s_setprio(1);  // ahead of the few-rows kernel's waves (see there)
   __shared__ __align__(1024) uint8_t smem[pf_ring_bytes(R)];
   __shared__ int s_sid[R];
   __shared__ float s_tw[R];  // with mul: the row's top-k weight rounded to bf16
