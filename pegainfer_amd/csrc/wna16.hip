@@ -13,10 +13,11 @@
 //
 // Dequantisation is exact: the nibble v, masked out of its word, is the fp16
 // denormal v 2^-24 (or v 2^-20, four bits further up), v_fma_mix_f32 forms
-// v 2^-24 * 2^24 s - 8 s = (v - 8) s with no rounding (both terms and the result fit
-// fp32 for scales below 2^104), and v_cvt_pk_bf16_f32 rounds that product to bf16
-// with round-to-nearest-even -- the same value as the reference's bf16 multiply
-// q*s.  The mask is a two-operand v_and_b32; biasing the nibble to 1024 + v takes a
+// v 2^-24 * 2^24 s - 8 s = (v - 8) s with no rounding, and v_cvt_pk_bf16_f32 rounds
+// that product to bf16 with round-to-nearest-even -- the same value as the
+// reference's bf16 multiply q*s.  From scales of 2^104 on 2^24 s is infinite, and every sum of
+// the column is infinite or NaN: a wave that ends with such a sum forms its sums again with
+// (v - 8) * s multiplied out (the wide form, right for every scale).  The mask is a two-operand v_and_b32; biasing the nibble to 1024 + v takes a
 // three-operand v_and_or_b32, which issues at half the rate once two waves share a
 // SIMD (1.0 against 1.8 ns an instruction).
 //
@@ -131,6 +132,39 @@ __device__ __forceinline__ BFrags make_b(const uint32_t w[4], uint32_t scale_pai
   f.y1 = as_bf16x8(q0.n1_lo, q1.n1_lo, q2.n1_lo, q3.n1_lo);
   f.y2 = as_bf16x8(q0.n1_hi, q1.n1_hi, q2.n1_hi, q3.n1_hi);
   return f;
+}
+
+// The same without the 2^24 s of the form above, for the rare sums that it left infinite or
+// NaN: about three times the instructions.
+__device__ __forceinline__ uint32_t wide_pair(uint32_t x, int bit, float s) {
+  return pack_bf16x2((static_cast<float>((x >> bit) & 15u) - 8.0f) * s,
+                     (static_cast<float>((x >> (bit + 16)) & 15u) - 8.0f) * s);
+}
+__device__ __forceinline__ WordPairs dequant_word_wide(uint32_t x, float a, float b) {
+  return WordPairs{wide_pair(x, 0, a), wide_pair(x, 4, a), wide_pair(x, 8, b),
+                   wide_pair(x, 12, b)};
+}
+__device__ __forceinline__ BFrags make_b_wide(const uint32_t w[4], uint32_t scale_pair) {
+  const float a = bf_lo(scale_pair), b = bf_hi(scale_pair);
+  WordPairs q[4];
+#pragma unroll
+  for (int jj = 0; jj < 4; ++jj) q[jj] = dequant_word_wide(w[jj], a, b);
+  BFrags f;
+  f.x1 = as_bf16x8(q[0].n0_lo, q[1].n0_lo, q[2].n0_lo, q[3].n0_lo);
+  f.x2 = as_bf16x8(q[0].n0_hi, q[1].n0_hi, q[2].n0_hi, q[3].n0_hi);
+  f.y1 = as_bf16x8(q[0].n1_lo, q[1].n1_lo, q[2].n1_lo, q[3].n1_lo);
+  f.y2 = as_bf16x8(q[0].n1_hi, q[1].n1_hi, q[2].n1_hi, q[3].n1_hi);
+  return f;
+}
+
+// Whether any lane's sum is infinite or NaN (x * 0 is NaN for those alone).  An infinite or
+// NaN weight makes every row's sum of its column so, rows of zeros included, so one element of
+// a lane's accumulators tells for its column.
+template <typename... F>
+__device__ __forceinline__ bool wave_any_nan(F... sums) {
+  float t = 0.0f;
+  ((t = __builtin_fmaf(sums, 0.0f, t)), ...);
+  return __ballot(t != t) != 0;
 }
 
 // Row of the 32x32 MFMA output held in accumulator element i by k-half h.
@@ -369,6 +403,23 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 4) void wna16_decode_ker
     if (g + q < g1) {
       if (q + 1 < D - 1 && g + q + 1 < g1) write_tr(slot[q + 1], (q + 1) & 1);
       compute_group(slot[q], q & 1);
+    }
+  }
+
+  if (__builtin_expect(wave_any_nan(accx_lo[0], accx_hi[0], accy_lo[0], accy_hi[0]), 0)) {
+    accx_lo = accx_hi = accy_lo = accy_hi = floatx16_t{};
+#pragma unroll 1
+    for (int g1w = g0; g1w < g1; ++g1w) {
+      load_group(slot[0], g1w);
+      write_tr(slot[0], 0);
+      const u32x4_t fw = *reinterpret_cast<const u32x4_t*>(slot_r0);
+      const uint32_t w4[4] = {fw[0], fw[1], fw[2], fw[3]};
+      const BFrags b = make_b_wide(w4, slot[0].sp);
+      const bf16x8_t A = __builtin_bit_cast(bf16x8_t, slot[0].a);
+      accx_lo = mfma(A, b.x1, accx_lo);
+      accx_hi = mfma(A, b.x2, accx_hi);
+      accy_lo = mfma(A, b.y1, accy_lo);
+      accy_hi = mfma(A, b.y2, accy_hi);
     }
   }
 
@@ -611,6 +662,28 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 6) void wna16_decode16_k
     }
   }
 
+  if (__builtin_expect(wave_any_nan(acc[0][0], acc[1][0], acc[2][0], acc[3][0]), 0)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = floatx4_t{};
+#pragma unroll 1
+    for (int gw = g0; gw < g1; ++gw) {
+      GroupRegs16& r = slot[0];
+      load_group(r, gw);
+      write_tr(r, 0);
+      const WordPairs qa0 = dequant_word_wide(slot_r0[0], bf_lo(r.sp0), bf_hi(r.sp0));
+      const WordPairs qa1 = dequant_word_wide(slot_r0[1], bf_lo(r.sp0), bf_hi(r.sp0));
+      const WordPairs qb0 = dequant_word_wide(slot_r0[32], bf_lo(r.sp1), bf_hi(r.sp1));
+      const WordPairs qb1 = dequant_word_wide(slot_r0[33], bf_lo(r.sp1), bf_hi(r.sp1));
+      const auto s0 = __builtin_amdgcn_permlane16_swap(r.a[0], r.a[2], false, false);
+      const auto s1 = __builtin_amdgcn_permlane16_swap(r.a[1], r.a[3], false, false);
+      const bf16x8_t A = as_bf16x8(s0[0], s1[0], s0[1], s1[1]);
+      acc[0] = mfma16(A, as_bf16x8(qa0.n0_lo, qa1.n0_lo, qa0.n0_hi, qa1.n0_hi), acc[0]);
+      acc[1] = mfma16(A, as_bf16x8(qa0.n1_lo, qa1.n1_lo, qa0.n1_hi, qa1.n1_hi), acc[1]);
+      acc[2] = mfma16(A, as_bf16x8(qb0.n0_lo, qb1.n0_lo, qb0.n0_hi, qb1.n0_hi), acc[2]);
+      acc[3] = mfma16(A, as_bf16x8(qb0.n1_lo, qb1.n1_lo, qb0.n1_hi, qb1.n1_hi), acc[3]);
+    }
+  }
+
   // element e = 4j + i of a lane: row 4 kb + i, column 32 a2 + 8 j + cc
 #pragma unroll
   for (int j = 0; j < 4; ++j)
@@ -817,6 +890,30 @@ void wna16_decode32_kernel(GemmArgs p) {
     if (g + q < groups) step(slot[q], slot[q + 1], slot[(q + 2) % D], 0, g + q, cur, nxt);
     if (g + q + 1 < groups)
       step(slot[q + 1], slot[(q + 2) % D], slot[(q + 3) % D], 1, g + q + 1, nxt, cur);
+  }
+
+  if (__builtin_expect(wave_any_nan(acc[0][0], acc[NB - 1][0]), 0)) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) acc[b] = floatx16_t{};
+#pragma unroll 1
+    for (int gw = 0; gw < groups; ++gw) {
+      GroupRegs32& r = slot[0];
+      load_group(r, gw);
+      write_tr(r, 0);
+      const u32x4_t fw = *reinterpret_cast<const u32x4_t*>(slot_r0);
+      const uint32_t w4[4] = {fw[0], fw[1], fw[2], fw[3]};
+      const BFrags f = make_b_wide(w4, r.sp);
+      const bf16x8_t A1 = __builtin_bit_cast(bf16x8_t, r.a0);
+      const bf16x8_t A2 = __builtin_bit_cast(bf16x8_t, r.a1);
+      if (NB == 2 || cs == 0) {
+        acc[0] = mfma(A1, f.x1, acc[0]);
+        acc[0] = mfma(A2, f.x2, acc[0]);
+      }
+      if (NB == 2 || cs == 1) {
+        acc[NB - 1] = mfma(A1, f.y1, acc[NB - 1]);
+        acc[NB - 1] = mfma(A2, f.y2, acc[NB - 1]);
+      }
+    }
   }
 
   float* s_red = reinterpret_cast<float*>(s_mem);
@@ -1136,6 +1233,41 @@ __device__ __forceinline__ void prefill_tile(const GemmArgs& p, uint8_t* smem, c
   int ch = 0;
   for (; ch + NS - 1 < chunks; ++ch) chunk(ch, std::true_type{});
   for (; ch < chunks; ++ch) chunk(ch, std::false_type{});
+  if constexpr (!IDLE) {
+    if (__builtin_expect(wave_any_nan(accx[0][0], accy[0][0]), 0)) {
+      // straight from memory: this lane's words, scale pair and rows of each group
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) accx[rb] = accy[rb] = floatx16_t{};
+      const uint32_t* words = p.qweight + static_cast<long long>(expert) * (expert_bytes / 4u) +
+                              nt * 128 + 16 * (c & 7) + (c >> 3);
+      const uint16_t* scales = p.scales + static_cast<long long>(expert) * (K >> 5) * N + nt * 64 +
+                               8 * (c & 7) + 2 * (c >> 3);
+#pragma unroll 1
+      for (int g = 0; g < K >> 5; ++g) {
+        uint32_t w4[4];
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj)
+          w4[jj] = words[static_cast<long long>(2 * g + h) * n_tiles * 128 + 4 * jj];
+        const BFrags f = make_b_wide(
+            w4, *reinterpret_cast<const uint32_t*>(scales + static_cast<long long>(g) * N));
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+          const int sid = s_sid[32 * rb + c];
+          bf16x8_t A1 = {}, A2 = {};
+          if (static_cast<unsigned>(sid) < static_cast<unsigned>(valid_limit)) {
+            const uint16_t* row =
+                p.input + static_cast<long long>(sid / p.top_k) * K + 32 * g + 16 * h;
+            A1 = *reinterpret_cast<const bf16x8_t*>(row);
+            A2 = *reinterpret_cast<const bf16x8_t*>(row + 8);
+          }
+          accx[rb] = mfma(A1, f.x1, accx[rb]);
+          accy[rb] = mfma(A1, f.y1, accy[rb]);
+          accx[rb] = mfma(A2, f.x2, accx[rb]);
+          accy[rb] = mfma(A2, f.y2, accy[rb]);
+        }
+      }
+    }
+  }
   lds_barrier();  // the epilogue's staging overwrites the ring
   uint16_t* s_a = reinterpret_cast<uint16_t*>(smem);
 

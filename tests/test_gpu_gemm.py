@@ -700,3 +700,44 @@ def test_expert_parallel_share_is_said_not_inferred(oracle):
     ref, split = run(None, ids, rows, 1)
     got, split8 = run(8, ids, rows, 1)
     assert split8 == split and np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("E,T,topk,bs,N,K", [
+    (1, 3, 1, 8, 128, 1024),     # 32-row decode kernel, sixteen waves
+    (1, 9, 1, 16, 8192, 256),    # eight
+    (4, 2, 2, 8, 256, 160),      # an odd group count
+    (48, 64, 8, 16, 1024, 512),  # 16-row decode kernel
+    (48, 70, 8, 8, 1024, 96),    # and two blocks of an expert a workgroup
+    (1, 20, 1, 64, 256, 192), (1, 70, 1, 64, 12800, 128), (6, 30, 1, 32, 256, 128),  # few rows
+    (2, 400, 1, 64, 320, 192), (2, 300, 1, 48, 256, 64), (8, 200, 1, 32, 384, 448)])  # tiles
+def test_scales_up_to_the_end_of_the_biased_forms_range(oracle, E, T, topk, bs, N, K):
+    """Scales from 2^104 to 2^117 in half the columns, among ordinary ones: their weights are
+    finite and exact, as every product bf16(q * s) that fits is.  Activations of 2^-115 times
+    small whole numbers keep the sums exact, so the oracle's bits are the only right ones."""
+    from pegainfer_amd import ops
+    g = np.random.default_rng(E * 100 + T + K)
+    q = g.integers(-8, 8, size=(E, N, K))
+    e = np.where(g.random((E, N, 1)) < 0.5, g.integers(104, 118, size=(E, N, 1)),
+                 g.integers(-3, 4, size=(E, N, 1)))
+    scale_bits = oracle.f32_to_bf16(np.ldexp(np.ones((E, N, K // 32), np.float32), e))
+    a_bits = oracle.f32_to_bf16(np.ldexp(g.integers(-2, 3, size=(T, K)).astype(np.float32), -115))
+    idx = g.integers(0, 2 * E if E == 48 else E, size=(T, topk)).astype(np.int32)
+    got, ref = _run(oracle, E=E, N=N, K=K, T=T, topk=topk, bs=bs, mul=False, a_bits=a_bits, q=q,
+                    scale_bits=scale_bits, idx=idx, tw=np.ones((T, topk), np.float32))
+    assert np.isfinite(oracle.bf16_to_f32(ref)).all() and np.array_equal(got, ref)
+    if N % 128:
+        return
+    w, packed = _setup(E, N, K, q, scale_bits)
+    ws = ops.KimiMarlinRouteWorkspace(T, bs, topk=topk, local_experts=E)
+    r = ops.moe_align_block_size(ws, dev(idx.reshape(-1)), T, T, 0)
+    gws = ops.KimiMarlinWna16Workspace(ws.max_m_blocks, N, bs, extra_splits=4)
+    routing = {k: host(getattr(r, k)) for k in ("sorted_token_ids", "expert_ids",
+                                                "num_tokens_post_padded")}
+    ref13 = oracle.wna16_gemm(a_bits, packed, scale_bits, routing, np.ones((T, topk), np.float32),
+                              moe_block_size=bs, top_k=topk, mul_topk_weights=False, size_m=T,
+                              size_n=N, size_k=K, threads=16)
+    local = idx.reshape(-1) < E
+    for split_k in (True, False):
+        act = torch.zeros(T * topk, N // 2, dtype=torch.bfloat16, device="cuda")
+        ops.wna16_w13_swiglu(gws, r, dev(a_bits), w, act, top_k=topk, size_m=T, split_k=split_k)
+        assert np.array_equal(host(act)[local], oracle.swiglu(ref13, N // 2)[local])
