@@ -159,15 +159,18 @@ typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
 // Global memory straight to LDS: lane l's 16 (or 4) bytes at voff + soff go to
 // lds + 16 l (4 l).  In asm so that the compiler, which cannot tell a ring's
 // stages apart, does not drain every load in flight at each LDS read; the kernels
-// count them themselves (vm_wait) and no register is written.  The resource is four
-// words (rsrc_words); lanes out of its range bring zeros.
+// count them themselves (vm_wait) and no register is written.  m0, which holds the LDS
+// address, is an operand, so the compiler sets it and knows that it has (the s_nop is the
+// wait that a load to LDS needs after m0 is set).  The resource is four
+// words (rsrc_words); lanes out of its range bring zeros (dense.hip's chunks that end inside a
+// stage rely on it).
 __device__ __forceinline__ void dma_b128(u32x4_t rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :: "{m0}"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
 }
 __device__ __forceinline__ void dma_b32(u32x4_t rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-               :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+  asm volatile("s_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+               :: "{m0}"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
 }
 template <int N>
 __device__ __forceinline__ void vm_wait() {

@@ -1102,8 +1102,7 @@ __device__ __forceinline__ void prefill_tile(const GemmArgs& p, uint8_t* smem, c
   // Activation staging: a row is 8 pieces of 16 bytes per chunk, piece q of row r at
   // position q ^ (r % 8), so that the MFMA fragments' reads (32 rows, one piece) spread
   // over the banks.  Load i of wave w brings rows 32 i + 8 w .. + 7, one row per 8 lanes;
-  // rows not routed here are out of range (zeros, or stale bytes: their products are
-  // never stored).
+  // rows not routed here are out of range and bring zeros.
   uint32_t a_voff[RB];
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
