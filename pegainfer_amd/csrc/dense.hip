@@ -285,7 +285,7 @@ int dense_launch(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M,
   if ((reinterpret_cast<uintptr_t>(W) & 15u) != 0 || (reinterpret_cast<uintptr_t>(X) & 15u) != 0)
     return fail(kNotSupported, "%s: W and X must be 16-byte aligned", name);
   // X is addressed through one 32-bit buffer range that must stay below the
-  // out-of-range offset, and so is a streaming workgroup's W span: 32 rows (it reads 16), or
+  // out-of-range offset, and so is a streaming workgroup's W span: its 16 or 32 rows, or
   // with SwiGLU its gate rows through its up rows.  The size of W as a whole does not matter.
   const long long w_span = SWIGLU ? static_cast<long long>(M) + 16 : 32;
   if (static_cast<long long>(N) * K * 2 >= static_cast<long long>(kOutOfRange) ||
@@ -318,6 +318,8 @@ int dense_launch(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M,
   const int rb = N <= 16 || fits(1, 1) ? 1 : (shares == 16 && !fits(1, 2) && fits(1, 3) ? 3 : 2);
   const bool many = N > 16 || (N > 8 && w_bytes >= (64LL << 20)) ||
                     (N > 4 && w_bytes >= (128LL << 20));
+  // a tile workgroup reads up to 128 rows of W through one 32-bit range
+  const bool tile_fits = 128LL * K * 2 < static_cast<long long>(kOutOfRange);
   bool two = false;
   if (!fits(1, rb) && tiles % 2 == 0) {
     if (rb == 1)
@@ -326,7 +328,7 @@ int dense_launch(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M,
     else if (rb == 2)
       two = fits(2, 2) && (shares == 16 ? N > 32 : shares >= 2 && N > 128);
   }
-  if (!two && !fits(1, rb) && (N > 32 || (many && tiles >= cu * 5LL / 4)))
+  if (tile_fits && !two && !fits(1, rb) && (N > 32 || (many && tiles >= cu * 5LL / 4)))
     return dense_tile<SWIGLU, F32>(W, X, Y, rows, M, N, K, shares, cu, stream, name);
   const auto go = [&](auto wv, auto mr, auto rbc) {
     launch_dense<decltype(wv)::value, decltype(mr)::value, decltype(rbc)::value, SWIGLU, F32>(
