@@ -465,8 +465,9 @@ def test_gemm_decode_accepts_k_multiple_of_32(oracle, bs, K):
 
 @pytest.mark.parametrize("K", [64, 96, 1056, 2080])
 def test_decode16_uneven_and_empty_k_shares(oracle, K):
-    """The 16x16x32 decode kernel (4 K-share waves per tile, picked when the launch has at
-    least 4 workgroups per CU: here 77 m-blocks x 16 tiles = 1232 on 256 CUs) with group
+    """The 16x16x32 decode kernel (4 K-share waves per tile, picked when the launch expects at
+    least a workgroup per CU: here, on Kimi's eighth of 512 routes, 64 m-blocks x 16 tiles =
+    1024 on 256 CUs, and 64 x 8 gate/up pairs for W13, too many for a K split) with group
     counts that 4 does not divide (33, 65: shares of 8 and 9, 16 and 17 groups) and with
     fewer groups than waves (2, 3: some waves add nothing), through the plain GEMM with the
     top-k weight and through W13 + SwiGLU (616 gate/up pairs: the paired launch, 4 waves
@@ -487,7 +488,8 @@ def test_decode16_uneven_and_empty_k_shares(oracle, K):
     w, packed = _setup(E, N, K, q, scale_bits)
     ws = ops.KimiMarlinRouteWorkspace(T, bs, topk=topk, local_experts=E)
     routing = ops.moe_align_block_size(ws, dev(idx.reshape(-1)), T, T, 0)
-    assert ws.max_m_blocks * (N // 64) >= 4 * 256 and ws.max_m_blocks * (inter // 64) >= 2 * 256
+    live = min(T * topk // 8, ws.max_m_blocks)
+    assert live * (N // 64) >= 4 * 256 and live * (inter // 64) >= 256
     gws = ops.KimiMarlinWna16Workspace(ws.max_m_blocks, N, bs)
     act = torch.full((T * topk, inter), 3.0, dtype=torch.bfloat16, device="cuda")
     ops.wna16_w13_swiglu(gws, routing, dev(a_bits), w, act, top_k=topk, size_m=T)
@@ -607,6 +609,49 @@ def test_tile_kernel_rows_and_chunks_exact(oracle, R_rows, K):
         got, ref = _run(oracle, E=E, N=N, K=K, T=T, topk=1, bs=bs, mul=False, a_bits=a_bits, q=q,
                         scale_bits=scale_bits, idx=idx, tw=np.ones((T, 1), np.float32))
         assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("R_rows", [1, 32, 33, 64, 65])
+@pytest.mark.parametrize("K", [64, 128, 192, 320, 512])
+def test_tile_kernel_of_64_rows_and_chunks_exact(oracle, R_rows, K):
+    """The same of the 64-row tiles, whose ring has its own stages: a launch with more experts
+    than rows to fill them (no id reaches the others), five column tiles and three gate/up
+    pairs, so that waves are idle."""
+    from pegainfer_amd import _lib, ops
+    g = np.random.default_rng(R_rows * 11 + K)
+    E, T, experts = 2, 400, 16
+    idx = np.zeros((T, 1), np.int32)
+    idx[g.permutation(T)[:R_rows], 0] = 1
+    a_bits = oracle.f32_to_bf16(g.integers(-2, 3, size=(T, K)).astype(np.float32))
+    a, ones = dev(a_bits), np.ones((T, 1), np.float32)
+    stream = torch.cuda.current_stream().cuda_stream
+    for bs, N in ((32, 320), (64, 384)):
+        q = g.integers(-8, 8, size=(E, N, K))
+        scale_bits = oracle.f32_to_bf16(
+            (2.0 ** g.integers(-6, -2, size=(E, N, K // 32))).astype(np.float32))
+        w, packed = _setup(E, N, K, q, scale_bits)
+        ws = ops.KimiMarlinRouteWorkspace(T, bs, topk=1, local_experts=E)
+        r = ops.moe_align_block_size(ws, dev(idx.reshape(-1)), T, T, 0)
+        out = torch.full((T, N), 7.0, dtype=torch.bfloat16, device="cuda")
+        tw = dev(ones.reshape(-1))
+        ids = (r.sorted_token_ids.data_ptr(), r.expert_ids.data_ptr(),
+               r.num_tokens_post_padded.data_ptr())
+        _lib.call("pega_wna16_gemm", a.data_ptr(), out.data_ptr(), None, 0,
+                  w.weight_packed_uint4b8.data_ptr(), w.weight_scale_permuted.data_ptr(), None, 0,
+                  *ids, tw.data_ptr(), r.max_padded_tokens, bs, 1, False, T, N, K, experts, 32, 0,
+                  stream)
+        routing = {k: host(getattr(r, k)) for k in ("sorted_token_ids", "expert_ids",
+                                                    "num_tokens_post_padded")}
+        ref = oracle.wna16_gemm(a_bits, packed, scale_bits, routing, ones, moe_block_size=bs,
+                                top_k=1, mul_topk_weights=False, size_m=T, size_n=N, size_k=K,
+                                output=np.zeros((T, N), np.uint16), threads=8)
+        assert np.array_equal(host(out), ref)
+        if N == 384:
+            act = torch.full((T, N // 2), 7.0, dtype=torch.bfloat16, device="cuda")
+            _lib.call("pega_wna16_w13_swiglu", a.data_ptr(), act.data_ptr(), None, 0,
+                      w.weight_packed_uint4b8.data_ptr(), w.weight_scale_permuted.data_ptr(),
+                      *ids, r.max_padded_tokens, bs, 1, T, N // 2, K, experts, 32, 0, stream)
+            assert np.array_equal(host(act), oracle.swiglu(ref, N // 2))
 
 
 def test_decode_merges_blocks_of_eight_rows(oracle):
