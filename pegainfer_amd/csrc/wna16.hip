@@ -1682,7 +1682,7 @@ int wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long long 
                int size_m, int size_n, int size_k, int local_experts, int ep, int group_size,
                int cu_count, hipStream_t stream) {
   if (!input || !output || !b_qweight || !b_scales || !sorted_token_ids || !expert_ids ||
-      !num_tokens_post_padded || !topk_weights)
+      !num_tokens_post_padded || (mul_topk_weights && !topk_weights))
     return fail(kInvalidValue, "wna16_gemm: null pointer");
   if (group_size != 32 || top_k <= 0 || size_m <= 0 || size_n <= 0 || size_k <= 0 ||
       sorted_token_ids_len <= 0 || local_experts <= 0)
@@ -1695,7 +1695,7 @@ int wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long long 
     return fail(kInvalidValue, "wna16_gemm: size_k %% 32 and size_n %% 64 must be 0 (k=%d n=%d)",
                 size_k, size_n);
   if (moe_block_size > 16 && size_k % 64 != 0)
-    return fail(kNotSupported, "wna16_gemm: the prefill tile kernel needs size_k %% 64 == 0 "
+    return fail(kNotSupported, "wna16_gemm: block sizes above 16 need size_k %% 64 == 0 "
                 "(k=%d)", size_k);
   if ((reinterpret_cast<uintptr_t>(input) & 15u) != 0 ||
       (reinterpret_cast<uintptr_t>(output) & 15u) != 0)
@@ -1772,7 +1772,7 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
   if (size_k % 32 != 0 || inter % 64 != 0)
     return fail(kInvalidValue, "w13_swiglu: size_k %% 32 and inter %% 64 must be 0");
   if (moe_block_size > 16 && size_k % 64 != 0)
-    return fail(kNotSupported, "w13_swiglu: the prefill tile kernel needs size_k %% 64 == 0");
+    return fail(kNotSupported, "w13_swiglu: block sizes above 16 need size_k %% 64 == 0");
   if ((reinterpret_cast<uintptr_t>(input) & 15u) != 0 ||
       (reinterpret_cast<uintptr_t>(act) & 15u) != 0 ||
       (reinterpret_cast<uintptr_t>(partials) & 15u) != 0)
@@ -1916,8 +1916,7 @@ int prefill_problem(const pega_wna16_problem* q, const char* which, GemmArgs& ar
   return kSuccess;
 }
 
-// A checked problem as its own launch.  Weights that are not multiplied are not read, so a
-// NULL there is replaced by a pointer the single entry's null check accepts.
+// A checked problem as its own launch.
 int single_problem(const pega_wna16_problem* q, int cu_count, hipStream_t stream) {
   if (q->act != nullptr)
     return wna16_w13_swiglu(q->input, q->act, nullptr, 0, q->b_qweight, q->b_scales,
@@ -1925,9 +1924,8 @@ int single_problem(const pega_wna16_problem* q, int cu_count, hipStream_t stream
                             q->sorted_token_ids_len, q->moe_block_size, q->top_k, q->size_m,
                             q->size_n / 2, q->size_k, q->local_experts, 1, q->group_size,
                             cu_count, stream);
-  const float* tw = q->topk_weights ? q->topk_weights : reinterpret_cast<const float*>(q->input);
   return wna16_gemm(q->input, q->output, nullptr, 0, q->b_qweight, q->b_scales, nullptr, 0,
-                    q->sorted_token_ids, q->expert_ids, q->num_tokens_post_padded, tw,
+                    q->sorted_token_ids, q->expert_ids, q->num_tokens_post_padded, q->topk_weights,
                     q->sorted_token_ids_len, q->moe_block_size, q->top_k,
                     q->mul_topk_weights != 0, q->size_m, q->size_n, q->size_k, q->local_experts, 1,
                     q->group_size, cu_count, stream);
@@ -2040,6 +2038,7 @@ PEGA_API int pega_wna16_gemm(const uint16_t* input, uint16_t* output, float* c_t
                              bool mul_topk_weights, int size_m, int size_n, int size_k,
                              int local_experts, int group_size, int sm_count,
                              hipStream_t stream) {
+  if (!topk_weights) return pega::fail(pega::kInvalidValue, "wna16_gemm: null pointer");
   return pega::wna16_gemm(input, output, c_tmp, c_tmp_len, b_qweight, b_scales, workspace,
                           workspace_len, sorted_token_ids, expert_ids, num_tokens_post_padded,
                           topk_weights, sorted_token_ids_len, moe_block_size, top_k,
