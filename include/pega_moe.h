@@ -130,12 +130,10 @@ int pega_wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long 
  * rounded to bf16 as the W13 output is, for the routed rows only (other rows are left as they
  * are), and the W13 output never reaches HBM.  The bits are the pair's whenever both add the
  * fp32 products over the same K shares: always at block sizes 32-64 (both take the same form
- * and the same split of K), and at block sizes 8/16 when the launch expects at least two (block,
- * 64-column tile) units per CU, or four on an expert-parallel share, and K is at least 512 (the
- * Kimi decode layer from 16 tokens on, for one).  A launch expects one block per route (per
- * ep_size routes in the _ep form below).  Otherwise the shares differ (the K split below, or 8
- * waves where the GEMM runs 16), and the sums may differ from the pair's in the last fp32
- * bit, within the same summation error bound.
+ * and the same split of K), and at block sizes 8/16 when there are at least four (block, 64-column
+ * tile) units per CU, counting a block per route, K is at least 512 and K is not split (below).
+ * Otherwise the shares differ, and the sums may differ from the pair's in the last fp32 bit,
+ * within the same summation error bound.
  *  - Block size 8 or 16 (decode): when the (block, tile) units are too few to fill the GPU
  *    (one expert at batch 1-8), K is split across workgroups; the fp32 partials (partials:
  *    at least 2 * size_m * top_k * 2 * intermediate_dim floats for a split, more allows more
@@ -157,7 +155,8 @@ int pega_wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials,
 
 /* The same where the experts are one GPU's of ep_size (at least 1, which is the entry above)
  * that the routes are spread over: the launch rules then expect one route in ep_size to be
- * local.  The outputs are the entry's above within the bound stated there.
+ * local, and split K further where the blocks that hold local routes leave CUs idle (Kimi's up
+ * to 15 tokens).  The outputs are the entry's above within the bound stated there.
  * kimi_marlin_wna16_gemm_cuda, whose 48 experts are one GPU's of eight, expects that by
  * itself; pega_wna16_gemm takes every route to be local, and so do both for an expert-major
  * launch (sorted_token_ids_len <= size_m * top_k). */

@@ -227,9 +227,9 @@ __device__ __forceinline__ u32x4_t buf_load_b128(__amdgpu_buffer_rsrc_t r, uint3
 }
 
 // ---------------------------------------------------------------------------
-// Decode kernel: one workgroup per (m-block, 64-column tile); WK waves split
-// the K range and are reduced through LDS in a fixed wave order (bit-for-bit
-// reproducible).  The block's rows (<= 32, one MFMA row block) occupy NI
+// Decode kernel: one workgroup per (m-block, 64-column tile); WK waves take the
+// SPW * WK shares of the K range, SPW one after another, which are added through
+// LDS in share order (bit-for-bit reproducible).  The block's rows (<= 32, one MFMA row block) occupy NI
 // accumulator elements per lane (rows < bs).
 //
 // Weight traffic is shaped for the texture-address unit: per quant group a
@@ -257,12 +257,13 @@ struct GroupRegs {
 // over a gate tile, waves WK..2WK-1 over the matching up tile (inter/64 tiles
 // further), and the epilogue writes SwiGLU of the two bf16-rounded sums to
 // p.act (p.output and p.partial are not used).
-template <int WK, int NI, int D, bool kPair = false>
-__global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 4) void wna16_decode_kernel(GemmArgs p) {
+template <int WK, int NI, int D, bool kPair, int SPW>
+__global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), SPW * NI == 16 ? 2 : 4)
+void wna16_decode_kernel(GemmArgs p) {
   static_assert(D % 2 == 0, "the two transpose slots alternate with the ring position");
-  constexpr int kWaves = WK * (kPair ? 2 : 1);
+  constexpr int kWaves = WK * (kPair ? 2 : 1), kShares = SPW * WK;
   __shared__ int s_sid[32];
-  __shared__ float s_red[kWaves][2 * NI][64];
+  __shared__ float s_red[SPW * kWaves][2 * NI][64];
   __shared__ __align__(16) uint32_t s_w[kWaves][2][kSlotDwords];
 
   const int n_tiles = p.size_n >> 6;
@@ -298,7 +299,9 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 4) void wna16_decode_ker
   const int groups = K >> 5;
   // this workgroup's share of the K groups, then this wave's share of that
   const int gs0 = (groups * split) / p.splits, gs1 = (groups * (split + 1)) / p.splits;
-  const int g0 = gs0 + ((gs1 - gs0) * kw) / WK, g1 = gs0 + ((gs1 - gs0) * (kw + 1)) / WK;
+  const auto share_start = [&](int sh) { return gs0 + ((gs1 - gs0) * sh) / kShares; };
+  const int g0 = share_start(SPW * kw), g1 = share_start(SPW * (kw + 1));
+  const int g_mid = SPW == 2 ? share_start(2 * kw + 1) : g1;  // where its second share starts
 
   const uint32_t expert_bytes = static_cast<uint32_t>(N) * static_cast<uint32_t>(K) / 2u;
   const __amdgpu_buffer_rsrc_t wr = make_rsrc(
@@ -362,6 +365,23 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 4) void wna16_decode_ker
     sw[64] = r.raw[2];
     sw[96] = r.raw[3];
   };
+  // the sums of this wave's share number i of SPW: of a row's NI elements in use, the k-lo part
+  // (rows 0..15) and the k-hi part (folded to rows 16..31)
+  auto store_share = [&](int i) {
+    float(*red)[64] = s_red[SPW * wave + i];
+#pragma unroll
+    for (int e = 0; e < NI; ++e) {
+      red[e][lane] = accx_lo[e] + accx_hi[e + 8];
+      red[NI + e][lane] = accy_lo[e] + accy_hi[e + 8];
+    }
+  };
+  bool again = false;  // a first share's sums were infinite or NaN
+  auto end_group = [&](int g) {
+    if (SPW == 1 || g + 1 != g_mid) return;
+    again = wave_any_nan(accx_lo[0], accx_hi[0], accy_lo[0], accy_hi[0]);
+    store_share(0);
+    accx_lo = accx_hi = accy_lo = accy_hi = floatx16_t{};
+  };
   auto compute_group = [&](const GroupRegs& r, int par) {
     const u32x4_t fw = *reinterpret_cast<const u32x4_t*>(par ? slot_r1 : slot_r0);
     const uint32_t w4[4] = {fw[0], fw[1], fw[2], fw[3]};
@@ -394,6 +414,7 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 4) void wna16_decode_ker
     for (int q = 0; q < D; ++q) {
       write_tr(slot[(q + 1) % D], (q + 1) & 1);
       compute_group(slot[q], q & 1);
+      end_group(g + q);
       load_group(slot[q], min(g + q + D, g1 - 1));
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -403,14 +424,15 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 4) void wna16_decode_ker
     if (g + q < g1) {
       if (q + 1 < D - 1 && g + q + 1 < g1) write_tr(slot[q + 1], (q + 1) & 1);
       compute_group(slot[q], q & 1);
+      end_group(g + q);
     }
   }
 
-  if (__builtin_expect(wave_any_nan(accx_lo[0], accx_hi[0], accy_lo[0], accy_hi[0]), 0)) {
+  if (__builtin_expect(wave_any_nan(accx_lo[0], accx_hi[0], accy_lo[0], accy_hi[0]) || again, 0)) {
     accx_lo = accx_hi = accy_lo = accy_hi = floatx16_t{};
 #pragma unroll 1
-    for (int g1w = g0; g1w < g1; ++g1w) {
-      load_group(slot[0], g1w);
+    for (int gw = g0; gw < g1; ++gw) {
+      load_group(slot[0], gw);
       write_tr(slot[0], 0);
       const u32x4_t fw = *reinterpret_cast<const u32x4_t*>(slot_r0);
       const uint32_t w4[4] = {fw[0], fw[1], fw[2], fw[3]};
@@ -420,17 +442,13 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 4) void wna16_decode_ker
       accx_hi = mfma(A, b.x2, accx_hi);
       accy_lo = mfma(A, b.y1, accy_lo);
       accy_hi = mfma(A, b.y2, accy_hi);
+      end_group(gw);
     }
   }
 
-  // Deterministic reduction over the WK waves (fixed order 0..WK-1); only the
-  // NI accumulator elements that hold rows < bs are exchanged, each the sum
-  // of its k-lo part (rows 0..15) and k-hi part (folded to rows 16..31).
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    s_red[wave][i][lane] = accx_lo[i] + accx_hi[i + 8];
-    s_red[wave][NI + i][lane] = accy_lo[i] + accy_hi[i + 8];
-  }
+  // Deterministic reduction over the shares, in order; only the NI accumulator elements that
+  // hold rows < bs are exchanged.
+  store_share(SPW - 1);
   __syncthreads();
 
   if constexpr (kPair) {
@@ -439,9 +457,9 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 4) void wna16_decode_ker
     for (int j = wave; j < 2 * NI; j += kWaves) {
       float sg = 0.0f, su = 0.0f;
 #pragma unroll
-      for (int w = 0; w < WK; ++w) {
+      for (int w = 0; w < kShares; ++w) {
         sg += s_red[w][j][lane];
-        su += s_red[WK + w][j][lane];
+        su += s_red[kShares + w][j][lane];
       }
       const int row = acc_row(j < NI ? j : j - NI, h);
       const int col = (j < NI) ? col0 : col0 + 8;
@@ -458,7 +476,7 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 4) void wna16_decode_ker
   for (int j = wave; j < 2 * NI; j += WK) {
     float s = 0.0f;
 #pragma unroll
-    for (int w = 0; w < WK; ++w) s += s_red[w][j][lane];
+    for (int w = 0; w < kShares; ++w) s += s_red[w][j][lane];
     const int row = acc_row(j < NI ? j : j - NI, h);
     const int n = (j < NI) ? n0 : n0 + 8;
     if (row < p.bs) {
@@ -942,39 +960,41 @@ void wna16_decode32_kernel(GemmArgs p) {
 
 constexpr int kDecodeDepth = 4;
 
-// WK = 4 runs the 16x16x32 kernel, the other share counts the 32-row one
-// (at 8 and 16 waves per workgroup the 16x16x32 form gains no occupancy and
-// its extra scale work cost C1/C2 2-4%).
-template <int WK>
-void launch_decode(const GemmArgs& args, int max_m_blocks, hipStream_t stream) {
+// Four shares run the 16x16x32 kernel, eight and sixteen the 32-row one (at 8 and 16 waves
+// per workgroup the 16x16x32 form gains no occupancy and its extra scale work cost C1/C2
+// 2-4%), sixteen on eight waves where `few_waves`.
+void launch_decode(const GemmArgs& args, int shares, bool few_waves, int max_m_blocks,
+                   hipStream_t stream) {
+  constexpr int D = kDecodeDepth;
   const dim3 grid(args.size_n / 64 * args.splits, max_m_blocks);
-  if constexpr (WK == 4) {
-    hipLaunchKernelGGL((wna16_decode16_kernel<WK, kDecodeDepth>), grid, dim3(64 * WK), 0, stream,
-                       args);
-  } else {
-    if (args.bs <= 8)
-      hipLaunchKernelGGL((wna16_decode_kernel<WK, 4, kDecodeDepth>), grid, dim3(64 * WK), 0,
-                         stream, args);
-    else
-      hipLaunchKernelGGL((wna16_decode_kernel<WK, 8, kDecodeDepth>), grid, dim3(64 * WK), 0,
-                         stream, args);
-  }
+  const auto go = [&](auto kernel, int waves) {
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), 0, stream, args);
+  };
+  const bool bs8 = args.bs <= 8;
+  if (shares == 4) go(wna16_decode16_kernel<4, D>, 4);
+  else if (shares == 8 && bs8) go(wna16_decode_kernel<8, 4, D, false, 1>, 8);
+  else if (shares == 8) go(wna16_decode_kernel<8, 8, D, false, 1>, 8);
+  else if (few_waves && bs8) go(wna16_decode_kernel<8, 4, D, false, 2>, 8);
+  else if (few_waves) go(wna16_decode_kernel<8, 8, D, false, 2>, 8);
+  else if (bs8) go(wna16_decode_kernel<16, 4, D, false, 1>, 16);
+  else go(wna16_decode_kernel<16, 8, D, false, 1>, 16);
 }
 
-template <int WK>
-void launch_decode_pair(const GemmArgs& args, int max_m_blocks, hipStream_t stream) {
+// Gate and up tile in one workgroup: four or eight shares each, eight on four waves each where
+// `few_waves`.
+void launch_decode_pair(const GemmArgs& args, int shares, bool few_waves, int max_m_blocks,
+                        hipStream_t stream) {
+  constexpr int D = kDecodeDepth;
   const dim3 grid(args.inter / 64, max_m_blocks);
-  if constexpr (WK == 4) {
-    hipLaunchKernelGGL((wna16_decode16_kernel<WK, kDecodeDepth, true>), grid, dim3(128 * WK), 0,
-                       stream, args);
-  } else {
-    if (args.bs <= 8)
-      hipLaunchKernelGGL((wna16_decode_kernel<WK, 4, kDecodeDepth, true>), grid, dim3(128 * WK),
-                         0, stream, args);
-    else
-      hipLaunchKernelGGL((wna16_decode_kernel<WK, 8, kDecodeDepth, true>), grid, dim3(128 * WK),
-                         0, stream, args);
-  }
+  const auto go = [&](auto kernel, int waves) {
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), 0, stream, args);
+  };
+  const bool bs8 = args.bs <= 8;
+  if (shares == 4) go(wna16_decode16_kernel<4, D, true>, 8);
+  else if (few_waves && bs8) go(wna16_decode_kernel<4, 4, D, true, 2>, 8);
+  else if (few_waves) go(wna16_decode_kernel<4, 8, D, true, 2>, 8);
+  else if (bs8) go(wna16_decode_kernel<8, 4, D, true, 1>, 16);
+  else go(wna16_decode_kernel<8, 8, D, true, 1>, 16);
 }
 
 // W13 + SwiGLU with args.act, else the plain GEMM.  Two workgroups a column tile in a plain
@@ -1617,8 +1637,10 @@ bool mean_rows_at_most(long long routes, long long experts, int ep, long long ro
   return routes <= rows * experts * ep;
 }
 
-// Blocks that a decode launch is expected to find work for: at most one per local route.
-long long live_blocks(long long routes, int ep, long long max_m_blocks) {
+// Blocks that a decode launch is expected to find work for: at most one per local route, and
+// with one expert as many as its rows fill.
+long long live_blocks(long long routes, int experts, int ep, int bs, long long max_m_blocks) {
+  if (experts == 1) return std::min((routes + bs - 1) / bs, max_m_blocks);
   return std::min((routes + ep - 1) / ep, max_m_blocks);
 }
 
@@ -1627,14 +1649,25 @@ bool pair_blocks(int bs, long long routes, int experts, int ep) {
   return bs == 8 && routes >= 4LL * experts * ep;
 }
 
-// Waves that share a workgroup's K: four from a workgroup per CU on, more below that, where
-// the CUs have no other work to hide a wave's latency behind.  Kimi W2 with one live block
-// (112 workgroups) in a decode layer at one token: 16 / 8 / 4 waves 55 / 51.7 / 53 us, with
-// three (336) 75 / 69.4 / 69.5 at 3 tokens; 28672 x 4096, one row (448) 19.4 / 16.1 / 16.1
-// us; 2560 x 9728, one row (40) 16.0 / 16.8 / 20.8.
-int decode_waves(long long wgs, int cu_count) {
-  return wgs >= cu_count ? 4 : (wgs >= cu_count * 3LL / 8 ? 8 : 16);
+// K shares of a decode launch of `wgs` workgroups (blocks, one per route at most, times
+// tiles): four from four workgroups per CU on, eight from two, else sixteen.  The numbers were
+// chosen for a kernel whose waves took a share each; they are kept, whatever share of the
+// routes is local and however many waves run, because the order of the sums is part of the
+// results' bits.
+int decode_shares(long long wgs, int cu_count) {
+  return wgs >= 4LL * cu_count ? 4 : (wgs >= 2LL * cu_count ? 8 : 16);
 }
+
+// Sixteen shares on eight waves, two each, from three workgroups on eight CUs on, where the CUs
+// have other work to hide a wave's latency behind (7168 x 2048, 112 workgroups, 7.4 us with
+// sixteen waves, 7.1 with eight; 28672 x 4096, 448, 20.6 / 17.7; 4096 x 4096, 64, 9.6 / 10.0).
+bool few_decode_waves(long long live_wgs, int cu_count) { return live_wgs >= cu_count * 3LL / 8; }
+
+// A W13 pair's eight shares on four waves, two each, past one and a half workgroups a CU, which
+// the 16 waves of the other form fill (DeepSeek-V2-Lite block at 3 tokens, 396 workgroups, 56
+// us against 59; 24 experts of another share at one token, 256 counted, 32 live, 37.3 against
+// 34.5).
+bool few_pair_waves(long long live_wgs, int cu_count) { return live_wgs > cu_count * 3LL / 2; }
 
 // Prefill tile height: 64 rows (three workgroups a CU instead of two) when the
 // routes come to few rows per expert, else 128.  Few rows per expert leave the
@@ -1721,15 +1754,13 @@ int wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long long 
     // Decode: one workgroup per (m-block, tile).  Fewer expected workgroups ->
     // more waves per workgroup splitting K, so the chip stays busy.
     const int groups = size_k / 32;
-    const long long est_blocks = live_blocks(routes, ep, max_m_blocks);
     args.pair_blocks = pair_blocks(moe_block_size, routes, local_experts, ep);
-    const long long wgs = est_blocks * n_tiles;
-    int wk = decode_waves(wgs, cu_count);
-    while (wk > 4 && groups < wk) wk >>= 1;  // waves past the last group idle
+    int shares = decode_shares(std::min<long long>(routes, max_m_blocks) * n_tiles, cu_count);
+    while (shares > 4 && groups < shares) shares >>= 1;  // none without a group
     if (max_m_blocks > 65535) return fail(kNotSupported, "wna16_gemm: too many m-blocks");
-    if (wk == 4) launch_decode<4>(args, max_m_blocks, stream);
-    else if (wk == 8) launch_decode<8>(args, max_m_blocks, stream);
-    else launch_decode<16>(args, max_m_blocks, stream);
+    const long long live =
+        live_blocks(routes, local_experts, ep, moe_block_size, max_m_blocks);
+    launch_decode(args, shares, few_decode_waves(live * n_tiles, cu_count), max_m_blocks, stream);
     return launch_status("wna16_gemm (decode)");
   }
   if (max_m_blocks > 65535) return fail(kNotSupported, "wna16_gemm: too many m-blocks");
@@ -1809,49 +1840,45 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
   if (cu_count <= 0) return fail(kInvalidValue, "w13_swiglu: no device");
   const int n_tiles = size_n / 64;
   const int groups = size_k / 32;
-  const long long est_blocks = live_blocks(routes, ep, max_m_blocks);
+  const long long est_blocks = std::min<long long>(routes, max_m_blocks);
   const long long wgs = est_blocks * n_tiles;
-  // Shares: about two workgroups per CU, at least 8 groups (two per wave) each, as many as
-  // the partials buffer holds.  On an expert-parallel share four per CU, since the routes that
-  // fall on it vary, and at most four shares, since most workgroups of its grid find no block
-  // and each share dispatches them again (decode layer at 1 / 3 / 12 tokens: one share 62.5
-  // / 69.5 / 98 us, two 55.7 / 62.4 / 96, four 53 / 59.5 / 95, eight 57 / 65 / -).
-  const long long aim = (ep > 1 ? 4LL : 2LL) * cu_count;
-  long long sp = (aim + wgs - 1) / wgs;
-  if (sp > (ep > 1 ? 4 : 16)) sp = ep > 1 ? 4 : 16;
+  const long long live = live_blocks(routes, local_experts, ep, moe_block_size, max_m_blocks);
+  // K splits: about two workgroups per CU, at least 8 groups each, as many as the partials
+  // buffer holds.  On an expert-parallel share four per CU of the blocks expected to hold local
+  // routes, since their number varies, and at most four splits, since most workgroups of its
+  // grid find no block and each split dispatches them again (decode layer at 1 / 3 / 12 tokens:
+  // one split 62.5 / 69.5 / 98 us, two 55.7 / 62.4 / 96, four 53 / 59.5 / 95, eight 57 / 65 / -).
+  const bool share = ep > 1;
+  const long long split_wgs = share ? live * n_tiles : wgs;
+  long long sp = ((share ? 4LL : 2LL) * cu_count + split_wgs - 1) / split_wgs;
+  if (sp > (share ? 4 : 16)) sp = share ? 4 : 16;
   if (sp > groups / 8) sp = groups / 8;
   const long long cap = partials ? partials_len / (routes * size_n) : 0;
   if (sp > cap) sp = cap;
-  if (sp <= 1) {
-    // No K split: a gate tile and its up tile in one workgroup of 2 WK waves,
-    // SwiGLU in the epilogue (partials not used).
-    GemmArgs args{input, nullptr, nullptr, reinterpret_cast<const uint32_t*>(b_qweight),
-                  b_scales, nullptr, sorted_token_ids, expert_ids, num_tokens_post_padded,
-                  nullptr, sorted_token_ids_len, moe_block_size, top_k, 0, size_m, size_n,
-                  size_k, local_experts, 1, nullptr, act, inter};
-    args.pair_blocks = pair_blocks(moe_block_size, routes, local_experts, ep);
-    const long long pair_wgs = est_blocks * (inter / 64);
-    // As the plain GEMM's from two units per CU on, so that the two give the same bits there
-    // (DeepSeek-V2-Lite block at 3 / 8 tokens: 61.2 / 81.6 us with four waves, 63.9 / 81.9
-    // with eight).
-    int wk = pair_wgs >= cu_count ? 4 : 8;
-    while (wk > 4 && groups < 2 * wk) wk >>= 1;  // keep >= 2 groups per wave
-    if (wk == 4) launch_decode_pair<4>(args, max_m_blocks, stream);
-    else launch_decode_pair<8>(args, max_m_blocks, stream);
-    return launch_status("w13_swiglu (decode)");
-  }
-  const int splits = static_cast<int>(sp);
   GemmArgs args{input, nullptr, nullptr, reinterpret_cast<const uint32_t*>(b_qweight), b_scales,
                 nullptr, sorted_token_ids, expert_ids, num_tokens_post_padded, nullptr,
                 sorted_token_ids_len, moe_block_size, top_k, 0, size_m, size_n, size_k,
-                local_experts, splits, partials};
+                local_experts, 1, nullptr, act, inter};
   args.pair_blocks = pair_blocks(moe_block_size, routes, local_experts, ep);
-  const long long total_wgs = wgs * splits;
-  int wk = decode_waves(total_wgs, cu_count);
-  while (wk > 4 && groups / splits < 2 * wk) wk >>= 1;  // keep >= 2 groups per wave
-  if (wk == 4) launch_decode<4>(args, max_m_blocks, stream);
-  else if (wk == 8) launch_decode<8>(args, max_m_blocks, stream);
-  else launch_decode<16>(args, max_m_blocks, stream);
+  if (sp <= 1) {
+    // No K split: a gate tile and its up tile in one workgroup, SwiGLU in the epilogue
+    // (partials not used).
+    const long long pair_wgs = est_blocks * (inter / 64);
+    int shares = pair_wgs >= 2LL * cu_count ? 4 : 8;
+    while (shares > 4 && groups < 2 * shares) shares >>= 1;  // at least two groups each
+    launch_decode_pair(args, shares, few_pair_waves(live * (inter / 64), cu_count), max_m_blocks,
+                       stream);
+    return launch_status("w13_swiglu (decode)");
+  }
+  const int splits = static_cast<int>(sp);
+  args.splits = splits;
+  args.partial = partials;
+  // shares of a split: on a share as few as fill the CUs, since the splits are shares already
+  int shares = share && live * n_tiles * splits >= cu_count ? 4
+                                                            : decode_shares(split_wgs * splits, cu_count);
+  while (shares > 4 && groups / splits < 2 * shares) shares >>= 1;
+  launch_decode(args, shares, few_decode_waves(live * n_tiles * splits, cu_count), max_m_blocks,
+                stream);
   const int rc = launch_status("w13_swiglu (GEMM)");
   if (rc != kSuccess) return rc;
   const long long work = static_cast<long long>(sorted_token_ids_len) * (inter / 2);

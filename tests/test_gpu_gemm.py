@@ -786,3 +786,64 @@ def test_scales_up_to_the_end_of_the_biased_forms_range(oracle, E, T, topk, bs, 
         act = torch.zeros(T * topk, N // 2, dtype=torch.bfloat16, device="cuda")
         ops.wna16_w13_swiglu(gws, r, dev(a_bits), w, act, top_k=topk, size_m=T, split_k=split_k)
         assert np.array_equal(host(act)[local], oracle.swiglu(ref13, N // 2)[local])
+
+
+@pytest.mark.parametrize("E,T,topk,bs,N,K,shares,w13_shares", [
+    (1, 1, 1, 8, 128, 1024, 16, 0),     # sixteen shares on sixteen waves
+    (1, 1, 1, 8, 6400, 1056, 16, 0),    # on eight
+    (1, 9, 1, 16, 6400, 1056, 16, 0),
+    (1, 2, 1, 8, 19200, 512, 8, 8),     # eight, and eight of a gate tile and of its up tile
+    (1, 2, 1, 8, 38400, 544, 4, 4),     # four
+    (48, 1, 8, 8, 6144, 1024, 8, 0),    # Kimi's share
+    (48, 3, 8, 8, 4096, 1024, 4, 0)])
+def test_decode_sums_are_shares_of_k_in_order(oracle, E, T, topk, bs, N, K, shares, w13_shares):
+    """The order of a decode launch's fp32 sums: contiguous shares of K's 32-k groups, added in
+    order, however many waves or workgroups run them.  One nonzero k in each share makes a
+    share's sum one exact product, and a large term that a later share cancels makes the
+    order show in bf16."""
+    from pegainfer_amd import ops
+    g = np.random.default_rng(E * 7 + T + N)
+    groups = K // 32
+
+    def problem(n):
+        used = [32 * int(g.integers(groups * s // n, groups * (s + 1) // n)) + int(g.integers(0, 32))
+                for s in range(n)]
+        first, last = (int(v) for v in sorted(g.choice(used, 2, replace=False)))
+        q = g.integers(1, 8, size=(E, N, K))
+        q[:, :, last] = q[:, :, first]
+        a = np.zeros((T, K), np.float32)
+        a[:, used] = oracle.bf16_to_f32(oracle.f32_to_bf16(
+            g.uniform(0.5, 1, (T, n)).astype(np.float32)))
+        a[:, first], a[:, last] = 2.0 ** 20, -2.0 ** 20
+        sums = np.zeros((E, T, N), np.float32)
+        for k in used:
+            sums = sums + a[None, :, k, None] * q[:, None, :, k].astype(np.float32)
+        return q, oracle.f32_to_bf16(a), oracle.f32_to_bf16(sums)
+
+    idx = np.stack([g.permutation(8 * E if E > 1 else 1)[:topk] for _ in range(T)]).astype(np.int32)
+    if E > 1:
+        idx[:, 0] = np.arange(T) % 2  # a local route each
+    flat = idx.reshape(-1)
+    local = np.flatnonzero(flat < E)
+    one = oracle.f32_to_bf16(np.ones((E, N, K // 32), np.float32))
+    q, a_bits, sums = problem(shares)
+    w, _ = _setup(E, N, K, q, one)
+    ws = ops.KimiMarlinRouteWorkspace(T, bs, topk=topk, local_experts=E)
+    r = ops.moe_align_block_size(ws, dev(flat), T, T, 0)
+    gws = ops.KimiMarlinWna16Workspace(ws.max_m_blocks, N, bs, extra_splits=16)
+    out = torch.zeros(T * topk, N, dtype=torch.bfloat16, device="cuda")
+    ops.wna16_gemm(gws, r, dev(a_bits), w, dev(np.ones(T * topk, np.float32)), out, top_k=topk,
+                   mul_topk_weights=False, size_m=T)
+    got = host(out)
+    for s in local:
+        assert np.array_equal(got[s], sums[flat[s], s // topk]), s
+    if not w13_shares:
+        return
+    q, a_bits, sums = problem(w13_shares)
+    w, _ = _setup(E, N, K, q, one)
+    act = torch.zeros(T * topk, N // 2, dtype=torch.bfloat16, device="cuda")
+    ops.wna16_w13_swiglu(gws, r, dev(a_bits), w, act, top_k=topk, size_m=T)
+    got = host(act)
+    for s in local:
+        want = oracle.swiglu(sums[flat[s], s // topk][None], N // 2)[0]
+        assert np.array_equal(got[s], want), s
