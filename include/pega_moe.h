@@ -130,7 +130,7 @@ int pega_wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long 
  * rounded to bf16 as the W13 output is, for the routed rows only (other rows are left as they
  * are), and the W13 output never reaches HBM.  The bits are the pair's whenever both add the
  * fp32 products over the same K shares: always at block sizes 32-64 (both take the same form
- * and the same split of K), and at block sizes 8/16 when there are at least four (block, 64-column
+ * and the same split of K), and at block sizes 8/16 when there are at least two (block, 64-column
  * tile) units per CU, counting a block per route, K is at least 512 and K is not split (below).
  * Otherwise the shares differ, and the sums may differ from the pair's in the last fp32 bit,
  * within the same summation error bound.

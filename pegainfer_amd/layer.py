@@ -85,7 +85,7 @@ class RoutedExperts:
         GPUs are never read: W2 reads only local rows, and the combine skips
         non-local routes) and fuses SwiGLU into W13.  The two give the same bits
         whenever the fused and the plain W13 add over the same K shares (prefill
-        block sizes; decode grids of four or more W13 (block, tile) units per CU with
+        block sizes; decode grids of two or more W13 (block, tile) units per CU with
         K >= 512 and no K split, Kimi's from 16 tokens on); a small decode grid splits
         K differently, and a W13 sum may then differ in the last fp32 bit.
         `w13_timer` (optional) exposes start()/stop(mark) and is called around the
