@@ -514,7 +514,7 @@ void wna16_decode_kernel(GemmArgs p) {
 // Blocks of 8 rows run two to a workgroup where an expert has several, so that its
 // weights are dequantised once per 16 rows (512 rows in blocks of 8 over 48 experts, W13 /
 // W2: 267 / 165 -> 186 / 121 us); from four routes per expert on, since looking the run up
-// costs about half a microsecond (Kimi's decode layer at 3 tokens 80.4 -> 81.6 us).
+// costs about half a microsecond a launch.
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4_t;
 
 __device__ __forceinline__ floatx4_t mfma16(bf16x8_t a, bf16x8_t b, floatx4_t c) {
@@ -756,9 +756,9 @@ __global__ __launch_bounds__(64 * WK * (kPair ? 2 : 1), 6) void wna16_decode16_k
 // (part, column tile) runs all of K, in the tile kernel's order, so a launch's bits do not
 // depend on which of the two a dispatch rule picks.  Bound by the dequant's vector
 // instructions like the kernels above; where few waves run, by one wave's chain, so the
-// next group is dequantised between this group's MFMAs (one expert, 2048 x 7168 at 64 rows:
-// 56 us without, 72 with the tile kernel; two waves a tile 39).  Kimi's MoE block, 160 tokens
-// (35 experts touched): 245 us against 289 with the tile kernel.
+// next group is dequantised between this group's MFMAs (one expert, 2048 x 7168 at 64 rows,
+// one workgroup a tile: 52 us, 56 without; the tile kernel 69).  Kimi's decode layer at 160
+// tokens: 266 us against 287 with the tile kernel.
 struct GroupRegs32 {
   u32x4_t raw;
   uint32_t sp;
@@ -1682,18 +1682,20 @@ bool small_prefill_tiles(long long routes, long long experts, int ep) {
   return mean_rows_at_most(routes, experts, ep, ep > 1 ? 24 : 64);
 }
 
-// Launches at block sizes above 16 that take the decode kernel's 32-row form instead
-// of the tile kernel: its units are a column tile's K shares, an eighth of a tile
-// workgroup's work, so few rows or few tiles still balance over the CUs, but every
-// column tile reads the activations again, which rules out many rows.
-//   * Few rows per expert on average (a decode batch on an eighth share: Kimi's decode
-//     layer at 110 / 180 / 220 / 256 tokens 242 / 286 / 316 / 313 us against
-//     271 / 310 / 336 / 317 with tiles; at 400 tokens, 8 rows, 393 against 364).
+// Launches at block sizes above 16 that take the decode kernel's 32-row form instead of the
+// tile kernel, with the same bits: its units are a 32-row part's column tiles (an eighth or a
+// sixteenth of a tile workgroup's work), so few rows or few tiles still balance over the CUs,
+// but every column tile reads the activations again, which rules out many rows.
+//   * Few rows per expert on average (a decode batch on an eighth share: Kimi's decode layer
+//     at 110 / 160 / 180 / 220 / 280 tokens 243 / 266 / 256 / 266 / 287 us against 259 / 287 /
+//     278 / 278 / 302 with tiles, but 310 against 301 at 256, by its routing; at the line the
+//     two are level: 64 experts, 64 tokens of top-6, 87.3 us either way).
 //   * One expert whose 32-row parts and column tiles are at most three workgroups a CU:
-//     the tile kernel would leave CUs idle for its whole chain over K (9728 x 2560,
-//     40 / 90 rows 18 / 23 against 34 / 39 us; 2048 x 7168, 64 rows 27 against 82; 14336 x
-//     4096, 128 rows, 3.5 a CU, 62 against 60).  Up to 128 rows, so that the shared
-//     expert of a prefill chunk stays with the routed experts' launch.
+//     the tile kernel would leave CUs idle for its whole chain over K (9728 x 2560, 17 / 64 /
+//     128 rows 16.5 / 24.6 / 27.8 against 25.7 / 29.8 / 38.6 us; 2048 x 7168, 64 rows 35.9
+//     against 69.3; 14336 x 4096, 17 / 96 rows, 0.9 / 2.6 a CU, 32.3 / 38.7 against 37.9 / 50.2;
+//     7168 x 2048 expert, 17 / 128 rows 83 / 100 against 87 / 129).  Up to 128 rows, so that
+//     the shared expert of a prefill chunk stays with the routed experts' launch.
 bool few_rows(long long routes, long long experts, int ep, int n_tiles, int cu_count) {
   if (experts == 1) return routes <= 128 && (routes + 31) / 32 * n_tiles <= 3LL * cu_count;
   return mean_rows_at_most(routes, experts, ep, 6);

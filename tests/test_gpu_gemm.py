@@ -506,16 +506,16 @@ def test_decode16_uneven_and_empty_k_shares(oracle, K):
 
 
 @pytest.mark.parametrize("E,T,topk,bs,N,K,mul", [
-    (48, 20, 8, 32, 128, 64, False),     # two groups for eight K shares, one column tile pair
+    (48, 20, 8, 32, 128, 64, False),     # two groups in a ring of six, one column tile pair
     (48, 100, 8, 48, 192, 160 * 2, True),  # odd tile count, a 48-row block's second, half part
-    (48, 250, 8, 64, 4096, 512, True),   # four K shares
+    (48, 250, 8, 64, 4096, 512, True),   # many column tiles
     (1, 17, 1, 64, 640, 192, False), (1, 31, 1, 64, 640, 192, True), (1, 32, 1, 64, 640, 192, False),
     (1, 33, 1, 64, 640, 448, True),      # second 32-row part with one row
     (1, 65, 1, 64, 128, 1024, False),    # second block
     (1, 128, 1, 32, 128, 2048, True), (6, 30, 1, 32, 256, 256, True)])
 def test_few_rows_form_exact(oracle, E, T, topk, bs, N, K, mul):
     """Block sizes above 16 with few rows (the decode kernel's 32-row form): exact inputs, so
-    both the GEMM and W13 + SwiGLU equal the oracle bit for bit whatever the K shares; rows not
+    both the GEMM and W13 + SwiGLU equal the oracle bit for bit in any order of sums; rows not
     routed here keep their contents."""
     from pegainfer_amd import ops
     g = np.random.default_rng(E * 1000 + T + K)
