@@ -301,7 +301,7 @@ int dense_launch(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M,
   // blocks (2048 x 2816, 24 tokens, 256 workgroups of 16 or 128 of 32 tokens: 4.5 / 5.7 us;
   // 64 tokens, 512 or 256: 7.3 / 6.0).  Blocks of 48 tokens only where the sums are in 16
   // shares, whose short chunks cost the tile kernel most (router logits, 384 tokens, 23.8
-  // here / 29.9 there; with two shares, 4096 x 7168, 40 tokens, 23.7 / 21.1).
+  // here / 29.9 there; with two shares, 4096 x 7168, 40 tokens, 23.7 / 17.6).
   // With more workgroups, the LDS-tiled kernel below from 33 tokens on, and from 17 where its
   // own tiles give the CUs a workgroup each; its tiles read X for 32 features at a time, not
   // 16, which also counts for fewer tokens where the weights are many: from 64 MB at 9 to 16
@@ -360,14 +360,14 @@ int dense_launch(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M,
 // above: at a share's end a wave adds the share's sums to its totals.  One barrier per chunk.
 //
 // Kimi's shared expert (gate/up with SwiGLU 4096 x 7168, down 7168 x 2048) at 64 / 160 / 250
-// tokens: gate/up 22.5 / 32.5 / 35.0 us, down 9.6 / 20.1 / 20.3 us, against 26.4 / 47.0 / 59.8
+// tokens: gate/up 20.8 / 32.5 / 35.0 us, down 9.6 / 20.1 / 20.3 us, against 26.4 / 47.0 / 59.8
 // and 12.1 / 22.2 / 30.7 us with the streaming kernel, whose fragments cross lanes through
 // ds_bpermute; the router's logits (384 x 7168, fp32) at 1000 / 4096 tokens 27.9 / 67.8
 // against 41.0 / 90.6 us.
 //
-// A row's 16-byte pieces are stored at slot piece ^ (row % pieces), which spreads the
-// fragment reads (16 rows, one piece) over the banks.  Bound by what a CU can bring in
-// from L2 at few tokens, by LDS reads and the matrix pipe at many.
+// A row's 16-byte pieces are stored at slot piece ^ (row % 16) (% pieces where a row has
+// fewer), which spreads the fragment reads (16 rows, one piece) over the banks.  Bound by what
+// a CU can bring in from L2 at few tokens, by LDS reads and the matrix pipe at many.
 template <int WM_, int WN_, int TM_, int TN_, int KC_, int NS_>
 struct TileShape {
   static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, KC = KC_, NS = NS_;
@@ -375,6 +375,7 @@ struct TileShape {
   static constexpr int kRowBytes = 2 * KC, kPieces = kRowBytes / 16;
   static constexpr int BM = 16 * WM * TM, BN = 16 * WN * TN;
   static constexpr int kStage = (BM + BN) * kRowBytes;
+  static constexpr int kSwizzle = kPieces < 16 ? kPieces : 16;
   static constexpr int kRowsPerLoad = 1024 / kRowBytes;
   static constexpr int P = (BM + BN) / kRowsPerLoad / kWaves;  // loads per wave and chunk
   static constexpr int kPitch = BM + 8;                        // floats per row of the epilogue
@@ -424,7 +425,7 @@ __global__ __launch_bounds__(S::kThreads) void dense_tile_kernel(const uint16_t*
                          static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
                              rows * static_cast<int>(row_bytes))));
     const int r = r0 + lane / S::kPieces;
-    const int piece = (lane % S::kPieces) ^ (r % S::kPieces);
+    const int piece = (lane % S::kPieces) ^ (r % S::kSwizzle);
     dst[j] = lds0 + static_cast<uint32_t>(r0 * S::kRowBytes);
     voff[j] = static_cast<uint32_t>(r - part0) * row_bytes + 16u * piece;
     piece_k[j] = 8 * piece;
@@ -463,7 +464,7 @@ __global__ __launch_bounds__(S::kThreads) void dense_tile_kernel(const uint16_t*
   auto read = [&](Frags& f, int st) {
 #pragma unroll
     for (int i = 0; i < kSteps; ++i) {
-      const int slot = 16 * ((4 * i + q) ^ (c % S::kPieces)) + st;
+      const int slot = 16 * ((4 * i + q) ^ (c % S::kSwizzle)) + st;
 #pragma unroll
       for (int t = 0; t < TM; ++t)
         f.w[i][t] = *reinterpret_cast<const bf16x8_t*>(w_rd + slot + 16 * S::kRowBytes * t);
@@ -598,8 +599,10 @@ int launch_tile(const uint16_t* W, const uint16_t* X, void* Y, int M, int N, int
 
 // The tile shape whose slowest CU brings in the fewest bytes: a CU's workgroups times the
 // rows of a stage, since all of these shapes read their operands at about the same rate
-// (what bounds them).  On a tie the larger tile.  The 32 x 32 tile has eight stages: it brings
-// in the least per chunk (4096 x 7168, 40 tokens, four / eight stages 23.8 / 21.1 us).
+// (what bounds them).  On a tie the larger tile.  The 32 x 32 tile has chunks of 256 k: a wave
+// has one MFMA per 32-k step there, so that a chunk's barrier and LDS round trip count most
+// (4096 x 7168, 40 tokens, weights not in cache, 17.6 us, 20.9 with eight stages of 128 k and 23.8
+// with four; 64 tokens, weights in cache, 16.5 / 20.3 with the first two).
 template <bool SWIGLU, bool F32>
 int dense_tile(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M, int N, int K,
                int shares, int cu, hipStream_t stream, const char* name) {
@@ -625,7 +628,7 @@ int dense_tile(const uint16_t* W, const uint16_t* X, void* Y, int rows, int M, i
     case 2: return go(TileShape<4, 2, 1, 1, 128, 6>{});
     case 3: return go(TileShape<2, 4, 1, 1, 128, 6>{});
     case 4: return go(TileShape<2, 2, 1, 3, 128, 4>{});
-    default: return go(TileShape<2, 2, 1, 1, 128, 8>{});
+    default: return go(TileShape<2, 2, 1, 1, 256, 4>{});
   }
 }
 
@@ -745,8 +748,8 @@ using namespace pega;
 
 // Reference: pegainfer-kernels/src/ffi/shared.rs:220-228 (gemm_cuda) and
 // :230-238 (gemm_graphsafe_cuda); both compute the same GEMM.  Below 256
-// tokens this library's kernels run; from 256 up, hipBLASLt (no workspace).  Neither allocates device memory per call, so both are
-// graph-safe once a shape has been called outside the capture (its first call
+// tokens this library's kernels run; from 256 up, hipBLASLt (no workspace).
+// Neither allocates device memory per call, so both are graph-safe once a shape has been called outside the capture (its first call
 // on a device makes the hipBLASLt handle and plan).
 PEGA_API int gemm_cuda(const uint16_t* W, const uint16_t* X, uint16_t* Y, int M, int N, int K,
                        hipStream_t stream) {

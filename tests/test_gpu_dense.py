@@ -325,6 +325,15 @@ def test_dense_tile_swiglu_equals_gemm_then_swiglu(oracle, I, N, K):
     assert np.array_equal(host(fused), host(chain))
 
 
+@pytest.mark.parametrize("M,N,K", [(4096, 33, 32), (4096, 64, 288), (4096, 50, 800),
+                                   (4128, 64, 1056), (4096, 64, 2080), (8192, 17, 576)])
+def test_dense_tile_long_chunks_exact(oracle, M, N, K):
+    """The 32 x 32 tile's chunks of 256 k: fewer chunks than its ring has stages, the ring come
+    round, and a tail of every kind (a step, most of a chunk) at the ends of K's shares."""
+    test_dense_tile_shapes_exact(oracle, M, N, K)
+    test_dense_tile_swiglu_equals_gemm_then_swiglu(oracle, M // 2, N, K)
+
+
 @pytest.mark.parametrize("N,K", [(33, 96), (100, 2080), (700, 160), (1500, 64), (4100, 32)])
 def test_dense_tile_router_logits_exact(oracle, N, K):
     """The fp32 epilogue through the router entry point, on exact operands."""
