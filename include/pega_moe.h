@@ -131,7 +131,7 @@ int pega_wna16_gemm(const uint16_t* input, uint16_t* output, float* c_tmp, long 
  * are), and the W13 output never reaches HBM.  The bits are the pair's whenever both add the
  * fp32 products over the same K shares: always at block sizes 32-64 (both take the same form
  * and the same split of K), and at block sizes 8/16 when there are at least two (block, 64-column
- * tile) units per CU, counting a block per route, K is at least 512 and K is not split (below).
+ * tile) units per CU, counting a block per route, and K is at least 512.
  * Otherwise the shares differ, and the sums may differ from the pair's in the last fp32 bit,
  * within the same summation error bound.
  *  - Block size 8 or 16 (decode): when the (block, tile) units are too few to fill the GPU
@@ -155,8 +155,7 @@ int pega_wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials,
 
 /* The same where the experts are one GPU's of ep_size (at least 1, which is the entry above)
  * that the routes are spread over: the launch rules then expect one route in ep_size to be
- * local, and split K further where the blocks that hold local routes leave CUs idle (Kimi's up
- * to 15 tokens).  The outputs are the entry's above within the bound stated there.
+ * local.  The outputs are the entry's above, bit for bit.
  * kimi_marlin_wna16_gemm_cuda, whose 48 experts are one GPU's of eight, expects that by
  * itself; pega_wna16_gemm takes every route to be local, and so do both for an expert-major
  * launch (sorted_token_ids_len <= size_m * top_k). */

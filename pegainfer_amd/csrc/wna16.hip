@@ -1845,15 +1845,13 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
   const long long est_blocks = std::min<long long>(routes, max_m_blocks);
   const long long wgs = est_blocks * n_tiles;
   const long long live = live_blocks(routes, local_experts, ep, moe_block_size, max_m_blocks);
-  // K splits: about two workgroups per CU, at least 8 groups each, as many as the partials
-  // buffer holds.  On an expert-parallel share four per CU of the blocks expected to hold local
-  // routes, since their number varies, and at most four splits, since most workgroups of its
-  // grid find no block and each split dispatches them again (decode layer at 1 / 3 / 12 tokens:
-  // one split 62.5 / 69.5 / 98 us, two 55.7 / 62.4 / 96, four 53 / 59.5 / 95, eight 57 / 65 / -).
-  const bool share = ep > 1;
-  const long long split_wgs = share ? live * n_tiles : wgs;
-  long long sp = ((share ? 4LL : 2LL) * cu_count + split_wgs - 1) / split_wgs;
-  if (sp > (share ? 4 : 16)) sp = share ? 4 : 16;
+  // K splits: about two workgroups per CU, counting a block per route whatever share of them is
+  // local (the split is part of the results' bits), at least 8 groups each, as many as the
+  // partials buffer holds.  Splitting for the blocks expected on an expert-parallel share won
+  // where few of them hold routes (Kimi's routed experts at 3 tokens 39.5 -> 27.5 us) but lost
+  // where more do (4096 x 1024, 8 tokens, 35.6 -> 40.8; 2048 x 1408, 12 tokens, 26.4 -> 29.4).
+  long long sp = (2LL * cu_count + wgs - 1) / wgs;
+  if (sp > 16) sp = 16;
   if (sp > groups / 8) sp = groups / 8;
   const long long cap = partials ? partials_len / (routes * size_n) : 0;
   if (sp > cap) sp = cap;
@@ -1875,9 +1873,7 @@ int wna16_w13_swiglu(const uint16_t* input, uint16_t* act, float* partials, long
   const int splits = static_cast<int>(sp);
   args.splits = splits;
   args.partial = partials;
-  // shares of a split: on a share as few as fill the CUs, since the splits are shares already
-  int shares = share && live * n_tiles * splits >= cu_count ? 4
-                                                            : decode_shares(split_wgs * splits, cu_count);
+  int shares = decode_shares(wgs * splits, cu_count);
   while (shares > 4 && groups / splits < 2 * shares) shares >>= 1;
   launch_decode(args, shares, few_decode_waves(live * n_tiles * splits, cu_count), max_m_blocks,
                 stream);
